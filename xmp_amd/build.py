@@ -33,6 +33,7 @@ SOURCES = [
     "k_powm.hip",
     "k_powm_latency.hip",
     "k_powm_wide.hip",
+    "k_powm_mx.hip",
     "k_probe.hip",
     "k_noalloc.hip",
 ]

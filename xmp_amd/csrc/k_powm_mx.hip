@@ -1,0 +1,567 @@
+// k_powm_mx.hip -- modular exponentiation on the matrix cores.
+//
+// One wave holds one instance.  A Montgomery product is three N-byte products
+// (x y, then q = low(x y) m' mod R, then q m; R = 256^N), each a contraction
+// that v_mfma_i32_16x16x64_i8 sums exactly.
+//
+// Digits are balanced bytes (-128 .. 127).  With N = 16 S, digit 16 u + v of a
+// product is
+//   P[16u + v] = sum_{s,t} Y[16 s + v - t] X[16 (u - s) + t],   t = 0 .. 15,
+// a 16 x 16 tile (rows v, columns u) of a matrix product over k = (s, t): the
+// rows' operand is 16-byte windows of Y at byte offsets (T fragments), the
+// columns' operand whole 16-byte blocks of X (C fragments).  Lane (g, i) of
+// the wave, g = lane / 16, i = lane % 16, supplies row or column i at
+// s = 4 kb + g, so a C fragment depends on u0 - 4 kb alone and is shared by
+// the tiles; within a fragment both operands run t downwards, so windows of Y
+// are read as stored and X is stored with the bytes of each block reversed.
+// An accumulator tile leaves four consecutive digits in a lane, which are one
+// 32-bit limb: limb 4 (16 r + i) + g of tile r.
+//
+// Carries: a tile's accumulators start at 128 per digit, so a lane's
+// sum s = d0 + 2^8 d1 + 2^16 d2 + 2^24 d3 is the limb's balanced bytes plus
+// 0x80808080, its low word taken as is.  Its high word (a few bits, signed)
+// moves one limb up by one cross-lane move; what that addition carries is
+// almost always nothing (a chance of 2^-15 a limb), and then resolved by
+// rounds of the same move.  No digit is ever unpacked.
+//
+// Values stay balanced, |x| <= 0.502 R, for any m < R: q is balanced, so
+// (x y + q m) / R is at most 0.252 R + 0.502 m, and the top limb's high word
+// k, seen before any carry, says whether m is to be subtracted or added once.
+// The low half of x y + q m is zero mod R; what it carries into the high half
+// is the rounded top limb of the low tile (the limbs below it move it by less
+// than 2^-15).  m' = -1/m mod R comes from Newton's iteration on the same
+// products.
+#include "devmp.hpp"
+#include "powm.hpp"
+
+namespace xmp {
+
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+constexpr uint32_t kBias = 0x80808080u;
+
+__device__ __forceinline__ void mx_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// -m0^-1 mod 2^32 for odd m0
+__device__ __forceinline__ uint32_t neg_inverse32(uint32_t m0) {
+  uint32_t inv = m0;
+#pragma unroll
+  for (int it = 0; it < 4; it++) inv = inv * (2u - m0 * inv);
+  return 0u - inv;
+}
+
+template <int S>
+struct Mx {
+  static_assert(S % 4 == 0 && S >= 4, "whole k-blocks");
+  static constexpr int N = 16 * S;            // bytes of R
+  static constexpr int LIMBS = 4 * S;
+  static constexpr int T = (S + 15) / 16;     // tiles of a half product
+  static constexpr int KB = S / 4;            // k-blocks of s = 0 .. S-1; k-block KB holds s = S
+  static constexpr int NF = (S + 12) / 4 + 1; // C fragments, u0 - 4 kb = -12 .. S
+  static constexpr int NQ = 4 * (T - 1) + 4;  // those of a low half product, -12 .. 16 (T-1)
+  static constexpr int TOP = (S - 1) % 16;    // column of the top limb in the last tile
+  static constexpr bool PART = S % 16 != 0;   // the last tile's columns past TOP hold nothing
+  static constexpr int C_BYTES = 16 * (S + 31);   // blocks -15 .. S+15
+  static constexpr int T_BYTES = 16 * (S + 6);    // bytes -16 .. 16 (S+5) - 1
+
+  uint8_t *cb, *tb;     // LDS: X by reversed blocks, Y plain
+  const uint8_t *cread; // this lane's C fragments (offset 16 (u0 - 4 kb + 12))
+  const uint8_t *tread; // this lane's T fragments (offset 64 kb)
+  int lane, i, g, rot;
+  uint32_t tshift;
+  int32_t k8, k16, k24;      // 2^8, 2^16, 2^24 in registers, for v_mad_i64_i32
+  v4i bias4;
+  v4i mp[KB];                // T fragments of m' and m
+  v4i mt[KB + 1];
+  uint32_t mw[T];            // this lane's limbs of m
+
+  __device__ __forceinline__ Mx(uint8_t *lds) {
+    lane = threadIdx.x;
+    i = lane & 15;
+    g = lane >> 4;
+    cb = lds;
+    tb = lds + C_BYTES;
+    cread = cb + 16 * (3 + i - g);
+    tread = tb + 16 * g + ((1 + i) & ~3);
+    tshift = (uint32_t)(1 + i) & 3u;
+    rot = 4 * (g ? lane - 16 : (i ? 47 + i : 63));
+    asm volatile("s_mov_b32 %0, 0x100" : "=s"(k8));
+    asm volatile("s_mov_b32 %0, 0x10000" : "=s"(k16));
+    asm volatile("s_mov_b32 %0, 0x1000000" : "=s"(k24));
+    asm volatile("v_mov_b32 %0, 0x80" : "=v"(bias4.x));
+    bias4 = v4i{bias4.x, bias4.x, bias4.x, bias4.x};
+    for (int b = lane; b < (C_BYTES + T_BYTES) / 16; b += 64) *reinterpret_cast<v4i *>(lds + 16 * b) = v4i{0, 0, 0, 0};
+    mx_fence();
+  }
+
+  __device__ __forceinline__ bool live(int r) const { return !PART || r < T - 1 || i <= TOP; }
+  __device__ __forceinline__ uint32_t limb(int r) const { return (uint32_t)(4 * (16 * r + i) + g); }
+  __device__ __forceinline__ static int top_lane(int r) { return r < T - 1 ? 63 : 48 + TOP; }
+
+  // the digits of e, as bytes: plain for T fragments, reversed blocks for C
+  __device__ __forceinline__ void put_c(const uint32_t (&e)[T]) const {
+#pragma unroll
+    for (int r = 0; r < T; r++)
+      *reinterpret_cast<uint32_t *>(cb + 16 * (15 + 16 * r + i) + 4 * (3 - g)) = __builtin_bswap32(e[r] ^ kBias);
+  }
+  __device__ __forceinline__ void put_t(const uint32_t (&e)[T]) const {
+#pragma unroll
+    for (int r = 0; r < T; r++)
+      if (live(r)) *reinterpret_cast<uint32_t *>(tb + 16 + 16 * (16 * r + i) + 4 * g) = e[r] ^ kBias;
+  }
+  __device__ __forceinline__ v4i cfrag(int f) const { return *reinterpret_cast<const v4i *>(cread + 64 * f); }
+  // 16 bytes at this lane's byte offset, from the five words that hold them
+  // (a byte-aligned 16-byte LDS read takes seven times an aligned one)
+  __device__ __forceinline__ v4i tfrag(int kb) const {
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(tread + 64 * kb);
+    v4i x;
+    x.x = (int)__builtin_amdgcn_alignbyte(w[1], w[0], tshift);
+    x.y = (int)__builtin_amdgcn_alignbyte(w[2], w[1], tshift);
+    x.z = (int)__builtin_amdgcn_alignbyte(w[3], w[2], tshift);
+    x.w = (int)__builtin_amdgcn_alignbyte(w[4], w[3], tshift);
+    return x;
+  }
+
+  // 128 a digit: with one tile its two chains start at 64 each (an inline
+  // constant of the instruction), with more the tiles share a register
+  __device__ __forceinline__ v4i bias() const { return T == 1 ? v4i{64, 64, 64, 64} : bias4; }
+  __device__ __forceinline__ static v4i bias2() { return v4i{64, 64, 64, 64}; }
+  static __device__ __forceinline__ v4i mfma(v4i t, v4i c, v4i acc) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(t, c, acc, 0, 0, 0);
+  }
+
+  __device__ __forceinline__ int64_t sum(v4i a) const {
+    return (int64_t)a.w * k24 + ((int64_t)a.z * k16 + ((int64_t)a.y * k8 + a.x));
+  }
+
+  // the limb above takes c[r]; tile 0's first limb takes cin.  Returns what
+  // leaves the top limb.
+  __device__ __forceinline__ int32_t move_up(int32_t (&c)[T], int32_t cin) const {
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      const int32_t top = __builtin_amdgcn_readlane(c[r], top_lane(r));
+      const int32_t up = __builtin_amdgcn_ds_bpermute(rot, c[r]);
+      c[r] = lane == 0 ? cin : (live(r) ? up : 0);
+      cin = top;
+    }
+    return cin;
+  }
+
+  // e = lo + c moved up, resolved; returns the carry out of the top limb
+  __device__ __forceinline__ int32_t resolve(uint32_t (&e)[T], const uint32_t (&lo)[T], int32_t (&c)[T],
+                                             int32_t cin) const {
+    int32_t out = move_up(c, cin);
+    bool any = false;
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      const int64_t x = (int64_t)(uint64_t)lo[r] + c[r];
+      e[r] = (uint32_t)x;
+      c[r] = (int32_t)(x >> 32);
+      any |= c[r] != 0;
+    }
+    while (__builtin_amdgcn_ballot_w64(any) != 0) {
+      out += move_up(c, 0);
+      any = false;
+#pragma unroll
+      for (int r = 0; r < T; r++) {
+        const int64_t x = (int64_t)(uint64_t)e[r] + c[r];
+        e[r] = (uint32_t)x;
+        c[r] = (int32_t)(x >> 32);
+        any |= c[r] != 0;
+      }
+    }
+    return out;
+  }
+
+  // biased digits of a half product's tiles; returns the carry out
+  __device__ __forceinline__ int32_t digits(uint32_t (&e)[T], const v4i (&a)[T], int32_t cin) const {
+    uint32_t lo[T];
+    int32_t c[T];
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      const int64_t s = sum(a[r]);
+      lo[r] = live(r) ? (uint32_t)s : kBias;
+      c[r] = live(r) ? (int32_t)(s >> 32) : 0;
+    }
+    return resolve(e, lo, c, cin);
+  }
+
+  // the same for limb sums s of a value to be kept within 0.502 R by adding
+  // or subtracting m
+  __device__ __forceinline__ void digits_mod(uint32_t (&e)[T], int64_t (&s)[T], int32_t cin) const {
+    for (int it = 0; it < 4; it++) {
+      const int32_t k = __builtin_amdgcn_readlane((int32_t)(s[T - 1] >> 32), top_lane(T - 1));
+      if (k != 0) {
+#pragma unroll
+        for (int r = 0; r < T; r++) s[r] -= (int64_t)k * (int64_t)(uint64_t)mw[r];
+      }
+      uint32_t lo[T];
+      int32_t c[T];
+#pragma unroll
+      for (int r = 0; r < T; r++) {
+        lo[r] = live(r) ? (uint32_t)s[r] : kBias;
+        c[r] = live(r) ? (int32_t)(s[r] >> 32) : 0;
+      }
+      const int32_t out = resolve(e, lo, c, cin);
+      if (out == 0) break;
+      // the top limb's own carry was not seen above (rare): once more
+      cin = 0;
+#pragma unroll
+      for (int r = 0; r < T; r++)
+        s[r] = (int64_t)(uint64_t)e[r] + (r == T - 1 && lane == top_lane(r) ? (int64_t)out << 32 : 0);
+    }
+  }
+
+  // low half of (T fragments from tf) * (X in LDS), and its carry out
+  template <class F>
+  __device__ __forceinline__ int32_t low_product(uint32_t (&e)[T], const F &tf, int32_t cin) const {
+    v4i cf[NQ], a[T], b = bias2();
+#pragma unroll
+    for (int f = 0; f < NQ; f++) cf[f] = cfrag(f);
+    if (T == 1) __builtin_amdgcn_sched_barrier(0);   // all reads in flight before the first use
+#pragma unroll
+    for (int r = 0; r < T; r++) a[r] = bias();
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) {
+      const v4i t = tf(kb);
+#pragma unroll
+      for (int r = 0; r < T; r++)
+        if (kb < 4 * r + 4) {
+          if (T == 1 && kb % 2 == 1) b = mfma(t, cf[4 * r - kb + 3], b);
+          else a[r] = mfma(t, cf[4 * r - kb + 3], a[r]);
+        }
+    }
+    if (T == 1) a[0] += b;
+    return digits(e, a, cin);
+  }
+
+  // e = x y / R mod m for X in LDS (which this overwrites) and Y's T
+  // fragments.  XTOP: X has a digit of its own in block S, cleared once read.
+  template <bool XTOP = false, class F>
+  __device__ __forceinline__ void mont(uint32_t (&e)[T], const F &tf) const {
+    v4i hi[T], h2 = bias2();
+    uint32_t q[T];
+    int32_t carry;
+    {
+      v4i cf[NF], lo[T], l2 = bias2();
+#pragma unroll
+      for (int f = 0; f < NF; f++) cf[f] = cfrag(f);
+      if (T == 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int r = 0; r < T; r++) lo[r] = hi[r] = bias();
+#pragma unroll
+      for (int kb = 0; kb <= KB; kb++) {
+        const v4i t = tf(kb);
+#pragma unroll
+        for (int r = 0; r < T; r++) {
+          if (kb < KB && kb < 4 * r + 4) {
+            if (T == 1 && kb % 2 == 1) l2 = mfma(t, cf[4 * r - kb + 3], l2);
+            else lo[r] = mfma(t, cf[4 * r - kb + 3], lo[r]);
+          }
+          if (kb >= 4 * r) {
+            if (T == 1 && kb % 2 == 1) h2 = mfma(t, cf[KB + 4 * r - kb + 3], h2);
+            else hi[r] = mfma(t, cf[KB + 4 * r - kb + 3], hi[r]);
+          }
+        }
+      }
+      if (T == 1) lo[0] += l2;
+      carry = digits(q, lo, 0);
+    }
+    const uint32_t low_top = q[T - 1];
+    mx_fence();
+    if (XTOP && lane == 0) cb[16 * (15 + S) + 15] = 0;
+    put_c(q);
+    mx_fence();
+    (void)low_product(q, [&](int kb) { return mp[kb]; }, 0);
+    mx_fence();
+    put_c(q);
+    mx_fence();
+    v4i cf[NF], lt = v4i{0, 0, 0, 0}, lt2 = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int f = 0; f < NF; f++) cf[f] = cfrag(f);
+    if (T == 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int kb = 0; kb <= KB; kb++) {
+      if (kb < KB) {
+        if (kb % 2 == 1) lt2 = mfma(mt[kb], cf[4 * (T - 1) - kb + 3], lt2);
+        else lt = mfma(mt[kb], cf[4 * (T - 1) - kb + 3], lt);
+      }
+#pragma unroll
+      for (int r = 0; r < T; r++)
+        if (kb >= 4 * r) {
+          if (T == 1 && kb % 2 == 1) h2 = mfma(mt[kb], cf[KB + 4 * r - kb + 3], h2);
+          else hi[r] = mfma(mt[kb], cf[KB + 4 * r - kb + 3], hi[r]);
+        }
+    }
+    lt += lt2;
+    if (T == 1) hi[0] += h2;
+    const int64_t lsum = sum(lt) + (int64_t)(uint64_t)low_top + (0x80000000ll - (int64_t)kBias);
+    carry += __builtin_amdgcn_readlane((int32_t)(lsum >> 32), top_lane(T - 1));
+    int64_t s[T];
+#pragma unroll
+    for (int r = 0; r < T; r++) s[r] = sum(hi[r]);
+    digits_mod(e, s, carry);
+  }
+
+  // m and m' into their fragments; returns whether m is odd and not 1
+  __device__ __forceinline__ bool load_modulus(const Operand &mod, uint32_t mi) {
+    uint32_t lo[T], e[T], z[T];
+    int32_t c[T];
+    bool other = false;
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      mw[r] = live(r) ? ld_limb(mod, mi, limb(r)) : 0u;
+      other |= mw[r] != (limb(r) == 0 ? 1u : 0u);
+      const uint64_t x = (uint64_t)mw[r] + kBias;
+      lo[r] = (uint32_t)x;
+      c[r] = (int32_t)(x >> 32);
+    }
+    const bool not_one = __builtin_amdgcn_ballot_w64(other) != 0;
+    const uint32_t m0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)mw[0]);
+    // the digits past the top limb's: 0 or 1
+    const int32_t top = resolve(e, lo, c, 0);
+    put_t(e);
+    if (lane == 0) tb[16 + N] = (uint8_t)top;
+    mx_fence();
+#pragma unroll
+    for (int kb = 0; kb <= KB; kb++) mt[kb] = tfrag(kb);
+    mx_fence();
+    if (lane == 0) tb[16 + N] = 0;
+    // z = -1/m mod 2^32, then z (2 + m z) doubles the correct bits
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      const uint64_t x = (uint64_t)(limb(r) == 0 ? neg_inverse32(m0) : 0u) + kBias;
+      lo[r] = (uint32_t)x;
+      c[r] = (int32_t)(x >> 32);
+    }
+    (void)resolve(z, lo, c, 0);
+#pragma unroll 1
+    for (int bits = 32; bits < 8 * N; bits *= 2) {
+      put_c(z);
+      put_t(z);
+      mx_fence();
+      (void)low_product(e, [&](int kb) { return mt[kb]; }, 2);
+      mx_fence();
+      put_c(e);
+      mx_fence();
+      (void)low_product(z, [&](int kb) { return tfrag(kb); }, 0);
+      mx_fence();
+    }
+    put_t(z);
+    mx_fence();
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) mp[kb] = tfrag(kb);
+    mx_fence();
+    return not_one && (m0 & 1u) != 0;
+  }
+};
+
+// One wave an instance.  r2 holds 2^(8N + t) mod m, squared `squarings` times
+// into R^2 mod m (t 2^squarings = 8N).
+template <int S, int WAVES>
+__global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args, uint32_t squarings) {
+  using M = Mx<S>;
+  constexpr int T = M::T;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[M::C_BYTES + M::T_BYTES];
+  const uint32_t local = blockIdx.x;
+  const uint32_t gi = args.start + local;
+  const uint32_t bi = in_index(args.base, gi), ei = in_index(args.exp, gi), mi = in_index(args.mod, gi);
+  M mx(lds);
+  const bool valid = mx.load_modulus(args.mod, mi);
+  const uint32_t wbits = args.window_bits;
+  uint32_t *table = args.table + ((size_t)local << wbits) * M::LIMBS;
+  auto store_entry = [&](uint32_t x, const uint32_t (&e)[T]) {
+#pragma unroll
+    for (int r = 0; r < T; r++)
+      if (mx.live(r)) table[(size_t)x * M::LIMBS + mx.limb(r)] = e[r];
+  };
+  auto load_entry = [&](uint32_t (&e)[T], uint32_t x) {
+#pragma unroll
+    for (int r = 0; r < T; r++) e[r] = mx.live(r) ? table[(size_t)x * M::LIMBS + mx.limb(r)] : kBias;
+  };
+  auto from_lds = [&](int kb) { return mx.tfrag(kb); };
+
+  uint32_t e[T];
+  int64_t s[T];
+  // R^2 mod m
+#pragma unroll
+  for (int r = 0; r < T; r++) {
+    const uint32_t w = mx.limb(r);
+    s[r] = (int64_t)kBias + (mx.live(r) && w < args.mod.len ? args.r2[(size_t)w * args.r2_stride + mi] : 0u);
+  }
+  mx.digits_mod(e, s, 0);
+  for (uint32_t j = 0; j < squarings; j++) {
+    mx.put_c(e);
+    mx.put_t(e);
+    mx_fence();
+    mx.mont(e, from_lds);
+    mx_fence();
+  }
+  mx.put_t(e);
+  // slot 0 = R mod m = 1 * R^2 / R
+#pragma unroll
+  for (int r = 0; r < T; r++) e[r] = mx.limb(r) == 0 ? kBias + 1u : kBias;
+  mx.put_c(e);
+  mx_fence();
+  mx.mont(e, from_lds);
+  mx_fence();
+  store_entry(0, e);
+  // slot 1 = base R mod m; a base at or above R/2 has one more digit, 1
+  {
+    uint32_t lo[T];
+    int32_t c[T];
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      const uint64_t x = (uint64_t)(mx.live(r) ? ld_limb(args.base, bi, mx.limb(r)) : 0u) + kBias;
+      lo[r] = (uint32_t)x;
+      c[r] = (int32_t)(x >> 32);
+    }
+    const int32_t top = mx.resolve(e, lo, c, 0);
+    mx.put_c(e);
+    mx_fence();
+    if (mx.lane == 0) mx.cb[16 * (15 + S) + 15] = (uint8_t)top;
+    mx_fence();
+    mx.template mont<true>(e, from_lds);
+    mx_fence();
+  }
+  store_entry(1, e);
+  mx.put_c(e);
+  mx.put_t(e);
+  mx_fence();
+  for (uint32_t x = 2; x < (1u << wbits); x++) {
+    mx.mont(e, from_lds);
+    mx_fence();
+    store_entry(x, e);
+    mx.put_c(e);
+    mx_fence();
+  }
+  // every lane's table stores before any lane's loads
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+
+  // exponent scan, top window first
+  auto window = [&](uint32_t pos, uint32_t len) {
+    const uint32_t w = pos >> 5;
+    return funnel(ld_limb(args.exp, ei, w + 1), ld_limb(args.exp, ei, w), pos & 31) & ((1u << len) - 1);
+  };
+  const uint32_t bits = args.exp.len * 32;
+  uint32_t pos = bits - ((bits % wbits) ? (bits % wbits) : wbits);
+  load_entry(e, window(pos, bits - pos));
+  while (pos > 0) {
+    pos -= wbits;
+    uint32_t f[T];   // the window's entry, on its way during the squarings
+    load_entry(f, window(pos, wbits));
+    for (uint32_t k = 0; k <= wbits; k++) {
+      mx.put_c(e);
+      if (k < wbits)
+        mx.put_t(e);
+      else
+        mx.put_t(f);
+      mx_fence();
+      mx.mont(e, from_lds);
+      mx_fence();
+    }
+  }
+  // out of Montgomery form: x * 1 / R, at most 0.502 (m + 1) either way
+  mx.put_c(e);
+#pragma unroll
+  for (int r = 0; r < T; r++) e[r] = mx.limb(r) == 0 ? kBias + 1u : kBias;
+  mx.put_t(e);
+  mx_fence();
+  mx.mont(e, from_lds);
+  uint32_t lo[T];
+  int32_t c[T];
+#pragma unroll
+  for (int r = 0; r < T; r++) {
+    const int64_t x = mx.live(r) ? (int64_t)(uint64_t)e[r] - (int64_t)kBias : 0;
+    lo[r] = (uint32_t)x;
+    c[r] = (int32_t)(x >> 32);
+  }
+  if (mx.resolve(e, lo, c, 0) < 0) {
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      const uint64_t x = (uint64_t)e[r] + mx.mw[r];
+      lo[r] = (uint32_t)x;
+      c[r] = (int32_t)(x >> 32);
+    }
+    (void)mx.resolve(e, lo, c, 0);
+  }
+  uint32_t *out = args.out.data + out_index(args.out, gi);
+#pragma unroll
+  for (int r = 0; r < T; r++) {
+    const uint32_t w = mx.limb(r);
+    // an even modulus is outside Montgomery's domain: defined result 0
+    if (mx.live(r) && w < args.out.len) out[(size_t)w * args.out.stride] = valid ? e[r] : 0u;
+  }
+}
+
+struct MxEntry {
+  uint32_t blocks;
+  void (*kernel)(PowmArgs, uint32_t);
+};
+const MxEntry kMx[] = {
+    {4, powm_mx_kernel<4, 4>},   {8, powm_mx_kernel<8, 4>},   {12, powm_mx_kernel<12, 4>}, {16, powm_mx_kernel<16, 4>},
+    {20, powm_mx_kernel<20, 3>}, {24, powm_mx_kernel<24, 3>}, {28, powm_mx_kernel<28, 2>}, {32, powm_mx_kernel<32, 2>},
+    {40, powm_mx_kernel<40, 2>}, {48, powm_mx_kernel<48, 1>}, {56, powm_mx_kernel<56, 1>}, {64, powm_mx_kernel<64, 1>},
+};
+
+}  // namespace
+
+uint32_t powm_mx_blocks(uint32_t precision) {
+  for (const MxEntry &e : kMx)
+    if (128u * e.blocks >= precision) return e.blocks;
+  return 0;
+}
+
+// Where the matrix cores are faster than the lane layouts: up to a batch size
+// that depends on the modulus.  A wave finishes one instance in a quarter to
+// a tenth of a lane group's time, but a full GPU multiplies 64-bit digits of
+// short moduli faster.  Measured on one MI355X, this kernel against the lane
+// layouts, exponents as long as the moduli: 512 bits x 2,048 0.44 against
+// 0.59 ms (4,096: 0.60, 0.59); 544 x 2,048 0.55, 1.12 (4,096: 0.79, 0.63);
+// 1024 x 4,096 1.42, 1.84 (8,192: 2.73, 2.13); 1056 x 4,096 1.85, 1.95
+// (6,144: 2.93, 2.68); 1536 x 12,288 7.8, 8.4 (16,384: 10.1, 8.5); 2048 x
+// 1,024 1.96, 6.69, x 12,288 12.1, 14.1 (16,384: 15.8, 14.3); 2080 x 6,144
+// 9.5, 11.9 (8,192: 12.1, 11.9); 3072 x 1,024 4.2, 32.4, x 16,384 40.8, 43.4;
+// 4096 x 16,384 71, 98; 8192 x 8,192 227, 388.  With 32-bit exponents the
+// lines are the same but for 3072 bits, where R^2 mod m and the set-up weigh
+// more: x 16,384 0.82, 0.87, x 65,536 3.03, 2.76.
+bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
+#ifdef XMP_MX_ALWAYS
+  return true;
+#endif
+  if (precision <= 256) return false;
+  if (precision <= 640) return count <= 2048;
+  if (precision <= 1024) return count <= 5120;
+  if (precision <= 1152) return count <= 4096;
+  if (precision <= 2048) return count <= 12288;
+  if (precision <= 2176) return count <= 6144;
+  if (precision <= 3072 && exp_bits <= 64) return count <= 24576;
+  return true;
+}
+
+size_t powm_mx_table_words(uint32_t blocks, uint32_t count, uint32_t window_bits) {
+  return ((size_t)count << window_bits) * 4 * blocks;
+}
+
+hipError_t launch_mx_r2(uint32_t blocks, uint32_t *r2, uint32_t r2_stride, const uint32_t *m, uint32_t m_len,
+                        uint32_t m_stride, uint32_t count, hipStream_t stream) {
+  const uint32_t rbits = 128u * blocks, j = (uint32_t)__builtin_ctz(rbits);
+  return launch_pow2_mod(r2, m_len, r2_stride, m, m_len, m_stride, count, rbits + (rbits >> j), nullptr, stream);
+}
+
+hipError_t launch_powm_mx(uint32_t blocks, const PowmArgs &args, hipStream_t stream) {
+  const uint32_t squarings = (uint32_t)__builtin_ctz(128u * blocks);
+  for (const MxEntry &e : kMx)
+    if (e.blocks == blocks && args.count != 0) {
+      hipLaunchKernelGGL(e.kernel, dim3(args.count), dim3(64), 0, stream, args, squarings);
+      return hipGetLastError();
+    }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace xmp

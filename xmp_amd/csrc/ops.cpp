@@ -269,7 +269,10 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   }
   if (e != xmpErrorSuccess) return e;
   const PowmVariant v = wide ? PowmVariant{0, 0, 0} : powm_variant(c.variant);
+  // the matrix cores, where they are faster and their whole plan fits (below)
+  uint32_t mx = 0;
   auto table_words = [&](uint32_t n, uint32_t w) {
+    if (mx) return powm_mx_table_words(mx, n, w);
     return wide ? powm_wide_table_words(wide, n, w) : powm_table_words(v, round_up(n, kStrideAlign), w);
   };
 
@@ -288,6 +291,14 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   const size_t fixed = (r2_words + div_words + r2blk_words + obuf_words) * sizeof(uint32_t);
   uint32_t wbits = c.window_bits;
   uint32_t chunk = count;
+  if (!wide && p->algorithm == xmpAlgorithmDefault && powm_mx_pays(out->precision, exp->precision, count)) {
+    mx = powm_mx_blocks(out->precision);
+    const uint32_t mx_bits = best_window_bits(exp->precision);
+    if (mx && fixed + table_words(count, mx_bits) * sizeof(uint32_t) <= limit)
+      wbits = mx_bits;
+    else
+      mx = 0;
+  }
   while (fixed + table_words(chunk, wbits) * sizeof(uint32_t) > limit) {
     // (a workgroup-layout instance can need megabytes: its chunks may shrink further)
     if (!ws && chunk > (wide ? kStrideAlign : 65536u)) {
@@ -328,6 +339,7 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   uint32_t *table = r2blk + r2blk_words + obuf_words;
   if ((wide ? launch_wide_r2(wide, r2, mstride, mod->limbs, mod->nlimbs, mod->stride, nmod,
                              div_words ? divws : nullptr, r2blk_words ? r2blk : nullptr, handle->stream)
+       : mx ? launch_mx_r2(mx, r2, mstride, mod->limbs, mod->nlimbs, mod->stride, nmod, handle->stream)
             : launch_montgomery_r2(c.variant, r2, mstride, mod->limbs, mod->nlimbs, mod->stride, nmod,
                                    div_words ? divws : nullptr, handle->stream)) != hipSuccess)
     return xmpErrorCuda;
@@ -343,8 +355,9 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   for (uint32_t start = 0; start < count; start += chunk) {
     args.start = start;
     args.count = std::min(chunk, count - start);
-    if ((wide ? launch_powm_wide(wide, args, handle->stream) : launch_powm_variant(c.variant, args, handle->stream)) !=
-        hipSuccess)
+    if ((wide ? launch_powm_wide(wide, args, handle->stream)
+         : mx ? launch_powm_mx(mx, args, handle->stream)
+              : launch_powm_variant(c.variant, args, handle->stream)) != hipSuccess)
       return xmpErrorCuda;
   }
   if (inplace && hipMemcpyAsync(out->limbs, obuf, obytes, hipMemcpyDeviceToDevice, handle->stream) != hipSuccess)

@@ -102,6 +102,17 @@ hipError_t launch_powm_wide(uint32_t tier, const PowmArgs &args, hipStream_t str
 // words, and for the memory tier `tier_ws` of powm_wide_r2_scratch_words words)
 hipError_t launch_wide_r2(uint32_t tier, uint32_t *r2, uint32_t r2_stride, const uint32_t *m, uint32_t m_len,
                           uint32_t m_stride, uint32_t count, uint32_t *ws, uint32_t *tier_ws, hipStream_t stream);
+// Exponentiation on the matrix cores (k_powm_mx.hip), one wave an instance, R = 2^(128 blocks):
+// the 16-byte blocks for a precision, 0 where it does not reach
+uint32_t powm_mx_blocks(uint32_t precision);
+size_t powm_mx_table_words(uint32_t blocks, uint32_t count, uint32_t window_bits);
+// r2 = 2^(128 blocks + t) mod m, which launch_powm_mx squares into R^2 mod m (t the odd part of 128 blocks)
+hipError_t launch_mx_r2(uint32_t blocks, uint32_t *r2, uint32_t r2_stride, const uint32_t *m, uint32_t m_len,
+                        uint32_t m_stride, uint32_t count, hipStream_t stream);
+hipError_t launch_powm_mx(uint32_t blocks, const PowmArgs &args, hipStream_t stream);
+// whether a call takes it rather than a lane layout
+bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count);
+
 // variants usable for a modulus precision (in bits): those with R >= 2^(precision+2)
 bool variant_fits(const PowmVariant &v, uint32_t precision);
 // whether the persistent mixed-size kernel runs this variant
