@@ -99,3 +99,35 @@ def test_matrix_core_powm_gathered_and_shared(handle):
         E1.close()
     for x in (M, B, E, out):
         x.close()
+
+
+@pytest.mark.parametrize("counts", [(30, 20, 10, 5), (9000, 4000, 300, 3), (12500, 0, 0, 2)])
+def test_batch_of_matrix_core_and_queued_classes(handle, counts):
+    """A mixed batch whose classes all run on the matrix cores, one whose short
+    moduli go to the queue (the classes share the GPU, so the rule sees the
+    whole batch), and one with a single class of each; replayed on new inputs."""
+    from xmp_amd import ext
+
+    sizes = [bits for bits, c in zip((512, 1024, 3072, 4096), counts) if c]
+    counts = [c for c in counts if c]
+    arrays = [[handle.integers(b, c) for _ in range(2)] + [handle.integers(96, c), handle.integers(b, c)]
+              for b, c in zip(sizes, counts)]
+    batch = None
+    for seed in (1, 2, 3):
+        wants = []
+        for (out, B, E, M), bits, c in zip(arrays, sizes, counts):
+            m, b, e = inputs.powm_class(5000 + 10 * seed + bits, c, bits, exp_bits=96)
+            for x, v in ((M, m), (B, b), (E, e)):
+                x.load(v)
+            wants.append(gmp(O.GO_POWM, c, bits // 32, b, e, m))
+        if batch is None:
+            batch = ext.Batch(handle, *[[a[k] for a in arrays] for k in range(4)], counts)
+        else:
+            batch.prepare()
+        batch.launch_async()
+        for (out, _, _, _), want, bits in zip(arrays, wants, sizes):
+            assert_rows_equal(out.get(), want, "launch %d, %d bits" % (seed, bits))
+    batch.close()
+    for a in arrays:
+        for x in a:
+            x.close()

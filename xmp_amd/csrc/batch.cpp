@@ -8,8 +8,12 @@
 // one device queue ordered by decreasing modelled cost (longest tiles first),
 // so short tiles fill the SIMDs that long ones leave idle.  The queue reset
 // and the persistent kernel are captured in a HIP graph on the first launch
-// and replayed afterwards.  A one-class batch captures that class's own
-// kernel instead: with nothing to interleave, the queue only costs time.
+// and replayed afterwards.  Classes that the matrix cores take (powm_mx_pays
+// for the whole batch's instances, which share the GPU) are kernels of their
+// own, each on a branch of the graph beside the persistent kernel, so that the
+// longest chains start at once and the others fill the SIMDs around them.  A
+// one-class batch captures that class's own kernel alone: with nothing to
+// interleave, the queue only costs time.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -37,12 +41,15 @@ struct _xmpBatch_t {
   std::vector<uint32_t *> r2, table;
   std::vector<uint32_t> r2_stride;
   PowmArgs *d_classes = nullptr;
-  PowmArgs single;   // a one-class batch's arguments (that class's kernel runs directly)
+  std::vector<PowmArgs> args;      // per class, as launched
+  std::vector<uint32_t> mx;        // per class: the matrix-core kernel's blocks, or 0 for the queue
   int32_t *d_variant = nullptr;
   uint32_t *d_tile_class = nullptr, *d_tile_index = nullptr, *d_counter = nullptr;
   uint32_t ntiles = 0, grid = 0;
   size_t lds_bytes = 0;
   hipStream_t capture_stream = nullptr;
+  std::vector<hipStream_t> branches;        // while a capture lasts
+  std::vector<hipEvent_t> branch_events;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
 };
@@ -69,6 +76,55 @@ double tile_cost(const PowmVariant &v, uint32_t exp_bits, uint32_t wbits) {
   const double nd = (double)(v.lanes * v.digits);
   const double products = (double)(1u << wbits) + exp_bits + std::ceil((double)exp_bits / wbits) + 2;
   return products * nd * (2.0 * v.digits + (v.lanes > 1 ? 14.0 : 5.0));
+}
+
+// The launches of one replay, on the capturing stream: the matrix-core
+// classes on branches of their own, largest moduli first, and the queue on
+// the stream itself.  The branches' streams and events are only needed while
+// the capture lasts (drop_branches, after it has ended).
+hipError_t capture_launches(xmpBatch_t b) {
+  const hipStream_t main = b->capture_stream;
+  // one class has no tiles of other classes to interleave: its own kernel
+  // runs without the queue (and without the persistent kernel's calls)
+  if (b->classes == 1)
+    return b->mx[0] ? launch_powm_mx(b->mx[0], b->args[0], main) : launch_powm_variant(b->variant[0], b->args[0], main);
+  std::vector<uint32_t> order;
+  for (uint32_t c = 0; c < b->classes; c++)
+    if (b->mx[c]) order.push_back(c);
+  std::stable_sort(order.begin(), order.end(), [b](uint32_t x, uint32_t y) { return b->mx[x] > b->mx[y]; });
+  hipError_t e = hipSuccess;
+  auto event = [&](hipStream_t on) {
+    hipEvent_t ev = nullptr;
+    if (e == hipSuccess && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) == hipSuccess) {
+      b->branch_events.push_back(ev);
+      e = hipEventRecord(ev, on);
+    }
+    return ev;
+  };
+  const hipEvent_t fork = order.empty() ? nullptr : event(main);
+  std::vector<hipEvent_t> joins;
+  for (uint32_t c : order) {
+    hipStream_t st = nullptr;
+    if (e != hipSuccess || (e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking)) != hipSuccess) return e;
+    b->branches.push_back(st);
+    if ((e = hipStreamWaitEvent(st, fork, 0)) != hipSuccess) return e;
+    if ((e = launch_powm_mx(b->mx[c], b->args[c], st)) != hipSuccess) return e;
+    joins.push_back(event(st));
+  }
+  if (e == hipSuccess && b->ntiles) {
+    const BatchArgs ba{b->d_classes, b->d_variant, b->d_tile_class, b->d_tile_index, b->ntiles, b->d_counter};
+    e = launch_powm_batch(ba, b->grid, b->lds_bytes, main);
+  }
+  for (hipEvent_t ev : joins)
+    if (e == hipSuccess) e = hipStreamWaitEvent(main, ev, 0);
+  return e;
+}
+
+void drop_branches(xmpBatch_t b) {
+  for (hipEvent_t ev : b->branch_events) (void)hipEventDestroy(ev);
+  for (hipStream_t st : b->branches) (void)hipStreamDestroy(st);
+  b->branch_events.clear();
+  b->branches.clear();
 }
 
 }  // namespace
@@ -104,7 +160,10 @@ xmpError_t XMPAPI xmpBatchCreate(xmpHandle_t handle, xmpBatch_t *batch, uint32_t
   b->table.assign(classes, nullptr);
   b->r2_stride.assign(classes, 0);
   xmpError_t e = xmpErrorSuccess;
-  std::vector<PowmArgs> args(classes);
+  std::vector<PowmArgs> &args = b->args;
+  args.resize(classes);
+  uint64_t instances = 0;
+  for (uint32_t c = 0; c < classes; c++) instances += counts[c];
   struct Tile {
     uint32_t cls, idx;
     double cost;
@@ -114,17 +173,34 @@ xmpError_t XMPAPI xmpBatchCreate(xmpHandle_t handle, xmpBatch_t *batch, uint32_t
     PowmChoice ch;
     e = choose_powm(handle, out[c]->precision, exp[c]->precision, counts[c], xmpAlgorithmDefault, &ch, true);
     if (e != xmpErrorSuccess) break;
+    const uint32_t mx = powm_mx_pays(out[c]->precision, exp[c]->precision,
+                                     (uint32_t)std::min<uint64_t>(instances, 0xFFFFFFFFu))
+                            ? powm_mx_blocks(out[c]->precision)
+                            : 0u;
+    if (mx) ch.window_bits = best_window_bits(exp[c]->precision);
     PowmVariant v = powm_variant(ch.variant);
     b->variant.push_back(ch.variant);
+    b->mx.push_back(mx);
     b->wbits.push_back(ch.window_bits);
-    b->lds_bytes = std::max(b->lds_bytes, powm_variant_lds_bytes(ch.variant));
-    size_t tw = powm_table_words(v, round_up(counts[c], kStrideAlign), ch.window_bits);
+    if (!mx) b->lds_bytes = std::max(b->lds_bytes, powm_variant_lds_bytes(ch.variant));
+    size_t tw = mx ? powm_mx_table_words(mx, counts[c], ch.window_bits)
+                   : powm_table_words(v, round_up(counts[c], kStrideAlign), ch.window_bits);
     b->table[c] = (uint32_t *)handle->da(tw * sizeof(uint32_t));
     if (!b->table[c]) {
       e = xmpErrorInvalidCudaMalloc;
       break;
     }
-    e = montgomery_prepare(handle, mod[c], ch.variant, &b->r2[c], &b->r2_stride[c]);
+    if (mx) {
+      b->r2_stride[c] = round_up(mod[c]->count, kStrideAlign);
+      b->r2[c] = (uint32_t *)handle->da(sizeof(uint32_t) * (size_t)mod[c]->nlimbs * b->r2_stride[c]);
+      if (!b->r2[c])
+        e = xmpErrorInvalidCudaMalloc;
+      else if (launch_mx_r2(mx, b->r2[c], b->r2_stride[c], mod[c]->limbs, mod[c]->nlimbs, mod[c]->stride,
+                            mod[c]->count, handle->stream) != hipSuccess)
+        e = xmpErrorCuda;
+    } else {
+      e = montgomery_prepare(handle, mod[c], ch.variant, &b->r2[c], &b->r2_stride[c]);
+    }
     if (e != xmpErrorSuccess) break;
     PowmArgs &a = args[c];
     a.out = OutOperand{out[c]->limbs, out[c]->nlimbs, out[c]->stride, nullptr};
@@ -137,13 +213,13 @@ xmpError_t XMPAPI xmpBatchCreate(xmpHandle_t handle, xmpBatch_t *batch, uint32_t
     a.start = 0;
     a.count = counts[c];
     a.window_bits = ch.window_bits;
+    if (mx) continue;
     const uint32_t per_tile = 64u / (uint32_t)v.lanes;
     const uint32_t nt = div_round_up(counts[c], per_tile);
     const double cost = tile_cost(v, exp[c]->precision, ch.window_bits);
     for (uint32_t t = 0; t < nt; t++) tiles.push_back({c, t, cost});
   }
-  if (e == xmpErrorSuccess && classes == 1) b->single = args[0];
-  if (e == xmpErrorSuccess) {
+  if (e == xmpErrorSuccess && !tiles.empty()) {
     // longest tiles first (LPT order); stable so each class's tiles stay in order
     std::stable_sort(tiles.begin(), tiles.end(), [](const Tile &x, const Tile &y) { return x.cost > y.cost; });
     b->ntiles = (uint32_t)tiles.size();
@@ -198,6 +274,12 @@ xmpError_t XMPAPI xmpBatchPrepare(xmpHandle_t handle, xmpBatch_t batch) {
   XMP_SET_DEVICE(handle);
   for (uint32_t c = 0; c < batch->classes; c++) {
     xmpIntegers_t m = batch->mod[c];
+    if (batch->mx[c]) {
+      if (launch_mx_r2(batch->mx[c], batch->r2[c], batch->r2_stride[c], m->limbs, m->nlimbs, m->stride, m->count,
+                       handle->stream) != hipSuccess)
+        return xmpErrorCuda;
+      continue;
+    }
     uint32_t *ws = nullptr;
     if (m->nlimbs > kMaxRegDivisorLimbs) {
       xmpError_t e = set_necessary_scratch(handle, (size_t)(2 * m->nlimbs + 1) * round_up(m->count, 256) * 4);
@@ -216,20 +298,15 @@ xmpError_t XMPAPI xmpBatchLaunchAsync(xmpHandle_t handle, xmpBatch_t batch) {
   XMP_TRACE("xmpBatchLaunchAsync");
   XMP_CHECK_NE(batch, nullptr);
   XMP_SET_DEVICE(handle);
-  BatchArgs ba{batch->d_classes, batch->d_variant, batch->d_tile_class, batch->d_tile_index, batch->ntiles,
-               batch->d_counter};
   if (!batch->exec) {
     // capture on a private stream (the legacy default stream cannot be captured)
     if (!batch->capture_stream && hipStreamCreate(&batch->capture_stream) != hipSuccess) return xmpErrorCuda;
     if (hipStreamBeginCapture(batch->capture_stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
       return xmpErrorCuda;
-    // one class has no tiles of other classes to interleave: its own kernel
-    // runs without the queue (and without the persistent kernel's calls)
-    hipError_t st = batch->classes == 1
-                        ? launch_powm_variant(batch->variant[0], batch->single, batch->capture_stream)
-                        : launch_powm_batch(ba, batch->grid, batch->lds_bytes, batch->capture_stream);
+    const hipError_t st = capture_launches(batch);
     hipGraph_t g = nullptr;
-    hipError_t st2 = hipStreamEndCapture(batch->capture_stream, &g);
+    const hipError_t st2 = hipStreamEndCapture(batch->capture_stream, &g);
+    drop_branches(batch);
     if (st != hipSuccess || st2 != hipSuccess || !g) return xmpErrorCuda;
     batch->graph = g;
     if (hipGraphInstantiate(&batch->exec, g, nullptr, nullptr, 0) != hipSuccess) return xmpErrorCuda;
