@@ -28,6 +28,7 @@ SOURCES = [
     "logic.cpp",
     "k_xfer.hip",
     "k_arith.hip",
+    "k_mul_mx.hip",
     "k_div.hip",
     "k_logic.hip",
     "k_powm.hip",

@@ -634,13 +634,10 @@ namespace {
 // register-resident row kernels, the longer operand (a) as the multiplicand:
 // one lane per instance up to 1024 bits, then lane groups; b.len <= a.len
 // keeps the multiplier within the accumulator bound.  SQR: b is a, and on
-// the one-lane and 32-lane layouts each row takes the symmetric half of its
-// products.  Measured A/B on one MI355X: 2^20 512-bit squares 0.035 against
-// 0.038 ms, 1,024 16384-bit ones (32 x 19) 0.076 against 0.081, and the
-// 65536-bit Karatsuba squares whose half products they are 0.87 against
-// 0.91; the 2-, 4-, 8- and 16-lane groups keep full rows (4 x 37: 0.093
-// against 0.087 ms for 65,536 4096-bit squares; 8 x 38 and 16 x 38 even).
-// False when a is longer than every group holds.
+// the one-lane layouts each row takes the symmetric half of its products
+// (measured A/B on one MI355X: 2^20 512-bit squares 0.035 against 0.038 ms);
+// the 2- and 4-lane groups keep full rows (4 x 37: 0.093 against 0.087 ms for
+// 65,536 4096-bit squares).  False when a is longer than every group holds.
 template <bool SQR>
 bool launch_rows(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t stream, hipError_t *e) {
   if (a.len <= 4) *e = launch_mul_lanes<1, 5, 28, SQR>(p, a, b, count, stream);          // 140 bits
@@ -650,7 +647,8 @@ bool launch_rows(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t
   else if (a.len <= 48) *e = launch_mul_lanes<2, 28, 28>(p, a, b, count, stream);        // 56 digits >= 1536 bits
   else if (a.len <= 64) *e = launch_mul_lanes<2, 37, 28>(p, a, b, count, stream);        // 74 digits >= 2048 bits
   else if (a.len <= 128) *e = launch_mul_lanes<4, 37, 28>(p, a, b, count, stream);       // 148 digits >= 4096 bits
-  // Above 4096 bits a batch of fewer than 4,096 products takes 32-lane groups
+  // Above 4096 bits (here only by multipliers shorter than half, the others
+  // are on the matrix cores) a batch of fewer than 4,096 products takes 32-lane groups
   // (count / 2 waves where 8 or 16 lanes leave SIMDs without a wave).
   // Measured on one MI355X: 1,024 x 16384-bit products 0.082 against 0.100
   // ms, 2,048 0.091 against 0.110, 1,024 x 8192-bit 0.038 against 0.048; at
@@ -658,10 +656,10 @@ bool launch_rows(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t
   // gain (16384 bits x 8,191: 0.23 against 0.20 ms; 16 x 19 digits at 8192
   // bits was slower than 8 x 38 at every batch from 8,191 to 16,383).
   else if (a.len <= 256)   // 304 digits >= 8192 bits
-    *e = count < 4096 ? launch_mul_lanes<32, 10, 27, SQR>(p, a, b, count, stream)
+    *e = count < 4096 ? launch_mul_lanes<32, 10, 27>(p, a, b, count, stream)
                       : launch_mul_lanes<8, 38, 27>(p, a, b, count, stream);
   else if (a.len <= 512)   // 608 digits >= 16384 bits
-    *e = count < 4096 ? launch_mul_lanes<32, 19, 27, SQR>(p, a, b, count, stream)
+    *e = count < 4096 ? launch_mul_lanes<32, 19, 27>(p, a, b, count, stream)
                       : launch_mul_lanes<16, 38, 27>(p, a, b, count, stream);
   else
     return false;
@@ -671,6 +669,7 @@ bool launch_rows(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t
 }  // namespace
 
 hipError_t launch_mul(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t stream) {
+  if (mul_mx_pays(a.len, b.len, count)) return launch_mul_mx(p, a, b, count, false, stream);
   // one lane per product with both operands in registers (product scanning)
   // for 513-1024-bit by 513-1024-bit and 1537-2048-bit by 513-2048-bit
   if (a.len > 16 && a.len <= 32 && b.len > 16) return launch_mul_cols<37, 37, false>(p, a, b, count, stream);
@@ -685,10 +684,11 @@ hipError_t launch_mul(OutOperand p, Operand a, Operand b, uint32_t count, hipStr
 }
 
 hipError_t launch_sqr(OutOperand p, Operand a, uint32_t count, hipStream_t stream) {
+  if (mul_mx_pays(a.len, a.len, count)) return launch_mul_mx(p, a, a, count, true, stream);
   // symmetric product scanning: each product of two different digits once
   if (a.len > 16 && a.len <= 32) return launch_mul_cols<37, 37, true>(p, a, a, count, stream);
   if (a.len > 48 && a.len <= 64) return launch_mul_cols<74, 74, true>(p, a, a, count, stream);
-  // symmetric rows on the one-lane and 32-lane layouts, full rows elsewhere
+  // symmetric rows on the one-lane layouts, full rows elsewhere
   hipError_t e;
   if (launch_rows<true>(p, a, a, count, stream, &e)) return e;
   return launch_mul(p, a, a, count, stream);
@@ -850,7 +850,7 @@ __global__ void __launch_bounds__(64) kar_carry_kernel(OutOperand p, uint32_t co
 // workspace limbs per instance column for a product of a_len x b_len limbs
 // (a_len >= b_len): this level's terms, then the largest child's
 size_t kar_limbs(uint32_t a_len, uint32_t b_len) {
-  if (a_len < kKaratsubaMinLimbs) return 0;
+  if (a_len < kKaratsubaMinLimbs || mul_mx_holds(a_len, b_len)) return 0;
   const uint32_t h = (a_len + 1) / 2;
   const size_t rows = (a_len + b_len + kKarChunk - 1) / kKarChunk;   // chunk carries
   if (b_len <= h) {
@@ -871,7 +871,7 @@ hipError_t launch_mul_ws(OutOperand p, Operand a, Operand b, uint32_t count, boo
                          hipStream_t stream) {
   if (count == 0) return hipSuccess;
   if (a.len < b.len) std::swap(a, b);
-  if (a.len < kKaratsubaMinLimbs) return square ? launch_sqr(p, a, count, stream) : launch_mul(p, a, b, count, stream);
+  if (a.len < kKaratsubaMinLimbs || mul_mx_holds(a.len, b.len)) return square ? launch_sqr(p, a, count, stream) : launch_mul(p, a, b, count, stream);
   const uint32_t st = round_up(count, kStrideAlign);
   const uint32_t h = (a.len + 1) / 2;
   auto take = [&](uint32_t limbs) {
