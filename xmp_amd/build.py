@@ -30,6 +30,7 @@ SOURCES = [
     "k_arith.hip",
     "k_mul_mx.hip",
     "k_div.hip",
+    "k_div_lazy.hip",
     "k_logic.hip",
     "k_powm.hip",
     "k_powm_latency.hip",

@@ -871,9 +871,13 @@ hipError_t launch_divmod_pair(OutOperand q, OutOperand r, Operand a, Operand b, 
 hipError_t launch_divmod_ws(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, uint32_t *scratch,
                             hipStream_t stream) {
   if (count == 0) return hipSuccess;
+  hipError_t st;
+  if (launch_divmod_lazy(q, r, a, b, count, stream, &st)) return st;
   const uint32_t nb = b.len;
-  // Below 131,072 divisions one lane each gives fewer than two waves per
-  // SIMD (1,024 SIMDs x 2 x 64 lanes): two lanes per division instead
+  // What is left: divisors up to 512 bits, and dividends too long for the
+  // signed-digit kernels' rows in LDS.  Below 131,072 divisions one lane each
+  // gives fewer than two waves per SIMD (1,024 SIMDs x 2 x 64 lanes): two
+  // lanes per division instead
   if (count < 131072 && nb > 16 && nb <= 128) {
     if (nb <= 32) return launch_divmod_pair<16>(q, r, a, b, count, stream);
     if (nb <= 64) return launch_divmod_pair<32>(q, r, a, b, count, stream);
@@ -904,6 +908,8 @@ hipError_t launch_divmod_ws(OutOperand q, OutOperand r, Operand a, Operand b, ui
 hipError_t launch_pow2_mod(uint32_t *out, uint32_t out_len, uint32_t out_stride, const uint32_t *m, uint32_t m_len,
                            uint32_t m_stride, uint32_t count, uint32_t e, uint32_t *scratch, hipStream_t stream) {
   if (count == 0) return hipSuccess;
+  hipError_t st;
+  if (launch_pow2_mod_lazy(out, out_len, out_stride, m, m_len, m_stride, count, e, stream, &st)) return st;
   if (m_len <= 8) return launch_pow2_reg<8>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
   if (m_len <= 16) return launch_pow2_reg<16>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
   if (m_len <= 32) return launch_pow2_reg<32>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);

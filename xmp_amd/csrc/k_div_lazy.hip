@@ -1,0 +1,462 @@
+// k_div_lazy.hip -- long division without carry chains.
+//
+// Reference: src/div.cu:35-517, digitmp/div.h:108-423 (schoolbook digits with
+// estimate, multiply-subtract and add-back).  Here the quotient digits are
+// signed and the remainder is never carried:
+//
+//  * operands are radix-2^28 digits, the divisor V shifted up to ND = L*K
+//    digits with its top bit set, the remainder ND signed 64-bit lazy sums.
+//    A step takes the next dividend digit in, R' = 2^28 R + u, and subtracts
+//    q V with q the nearest integer to R' / V: one v_mad_i64_i32 per digit,
+//    where 32-bit limbs with borrows cost a multiply-add and two
+//    subtractions, in one serial chain from digit to digit;
+//  * q comes from the top three sums in double precision: what they leave
+//    out, and the rounding, move R'/V by less than 2^-18, so |R| stays below
+//    (1/2 + 2^-18) V, no digit is ever corrected, and adding 1.5 * 2^52 in
+//    the last multiply-add leaves -q in the low word;
+//  * a sum gains at most 2^55 + 2^38 a step and leaves the window after ND
+//    steps: below 2^63 up to 160 digits.  The top sum, folded into the one
+//    below it, is small because R is;
+//  * a division spans L lanes of K digits, the top digits on the group's
+//    first lane, whose q the others take by the same DPP moves as the
+//    Montgomery quotient; one 64-bit sum moves a lane up a step;
+//  * the dividend's digits wait in LDS, each replaced by its quotient digit;
+//    at the end R is carried once (V added and the quotient lowered by one
+//    if it is negative) and the signed quotient digits once.
+//
+// Division by zero writes q = 0 and r = a.
+#include <algorithm>
+
+#include "devmp.hpp"
+#include "kernels.hpp"
+#include "lanes.hpp"
+#include "powm.hpp"
+
+namespace xmp {
+
+namespace {
+
+constexpr int D = 28;
+constexpr uint32_t MASK = (1u << D) - 1;
+constexpr int kRun = 16;   // digits that a lane fetches at a time
+
+// Dividends and divisors.  load<N>: limbs k0 .. k0 + N - 1, 0 outside
+// [0, len), all loads unconditional, at limbs that exist, and masked (a select
+// lets the compiler put a load under a branch, and then every load waits for
+// the one before).  Where every lane's limbs exist the row's address is
+// scalar and a lane's offset one register for all of them.
+struct ArrayDividend {
+  const uint32_t *data;
+  uint32_t stride, len, inst;
+  template <int N>
+  __device__ __forceinline__ void load(uint32_t (&x)[N], int32_t k0) const {
+    const bool inside = k0 >= 0 && k0 + N <= (int32_t)len && (uint64_t)len * stride < (1ull << 30);
+    if (__builtin_amdgcn_ballot_w64(!inside) == 0) {
+      const uint32_t off = ((uint32_t)k0 * stride + inst) * 4u;
+#pragma unroll
+      for (int k = 0; k < N; k++)
+        x[k] = *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(data + (size_t)k * stride) + off);
+    } else {
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const int32_t kc = min(max(k0 + k, 0), (int32_t)len - 1);
+        const uint32_t v = data[(size_t)(uint32_t)kc * stride + inst], m = kc == k0 + k ? ~0u : 0u;
+        x[k] = v & m;
+      }
+    }
+  }
+  __device__ __forceinline__ uint32_t limb(int32_t k) const {
+    uint32_t x[1];
+    load<1>(x, k);
+    return x[0];
+  }
+};
+struct PowerDividend {   // 2^e
+  uint32_t e, len;
+  __device__ __forceinline__ uint32_t limb(int32_t k) const {
+    return k >= 0 && (uint32_t)k == (e >> 5) ? 1u << (e & 31) : 0u;
+  }
+  template <int N>
+  __device__ __forceinline__ void load(uint32_t (&x)[N], int32_t k0) const {
+#pragma unroll
+    for (int k = 0; k < N; k++) x[k] = limb(k0 + k);
+  }
+};
+
+// N digits from bit `off` (0 .. 31) of limb w up (they may lie below 0 or past the top)
+template <int N, class Dividend>
+__device__ __forceinline__ void digits_at(uint32_t (&d)[N], const Dividend &a, int32_t w, uint32_t off) {
+  constexpr int NW = (D * N + 31) / 32;
+  uint32_t x[NW + 1];
+  a.template load<NW + 1>(x, w);
+#pragma unroll
+  for (int j = 0; j < NW; j++) x[j] = funnel(x[j + 1], x[j], off);
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int j = (D * k) >> 5, s = (D * k) & 31;
+    d[k] = (s + D <= 32 ? x[j] >> s : funnel(x[j + 1 < NW ? j + 1 : j], x[j], s)) & MASK;
+  }
+}
+
+// limbs 7 m .. 7 m + 6 of an integer whose radix-2^28 digits 0 .. n-1 are at
+// d, from digit `skip` and bit s (0 .. 27) of it up: digits 8 m .. 8 m + 7
+__device__ __forceinline__ void limbs7(uint32_t (&w)[7], const uint32_t *d, int32_t n, int32_t m, int32_t skip,
+                                       uint32_t s) {
+  uint32_t x[9];
+#pragma unroll
+  for (int k = 0; k < 9; k++) {
+    const int32_t at = 8 * m + skip + k;
+    const uint32_t v = d[min(at, n - 1)], keep = at < n ? ~0u : 0u;
+    x[k] = v & keep;
+  }
+#pragma unroll
+  for (int k = 0; k < 8; k++) x[k] = (x[k] >> s) | ((x[k + 1] << (D - s)) & MASK);
+#pragma unroll
+  for (int j = 0; j < 7; j++) w[j] = (x[j] >> (4 * j)) | (x[j + 1] << (D - 4 * j));
+}
+
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <int L, int K>
+struct Lazy {
+  static constexpr int ND = L * K;
+  static_assert(K >= 3 && ND <= 160, "the estimate's digits on one lane; sums below 2^63");
+  const Group<L> g;
+  __device__ __forceinline__ explicit Lazy(int lane) : g(lane) {}
+
+  // the next lane's (lower digits') value, 0 on the group's last lane
+  __device__ __forceinline__ int64_t from_below(int64_t x) const {
+    if constexpr (L == 1) return 0;
+    const uint32_t lo = g.from_next((uint32_t)x), hi = g.from_next((uint32_t)(x >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+  }
+  // every lane's copy of the group's first lane's value
+  __device__ __forceinline__ uint32_t top(uint32_t x) const { return g.bcast0(x); }
+
+  // r = the sums' digits; returns the signed carry out of the top digit (0 or -1 for |R| < V)
+  __device__ __forceinline__ int32_t carry(uint32_t (&r)[K], const int64_t (&t)[K]) const {
+    int64_t c = 0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      const int64_t x = t[k] + c;
+      r[k] = (uint32_t)x & MASK;
+      c = x >> D;
+    }
+    int32_t out = (int32_t)c;
+    if constexpr (L > 1) {
+      for (int round = 1; round < L; round++) {
+        c = from_below(c);
+        if (__builtin_amdgcn_ballot_w64(c != 0) == 0) break;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+          const int64_t x = (int64_t)r[k] + c;
+          r[k] = (uint32_t)x & MASK;
+          c = x >> D;
+        }
+        out += (int32_t)c;
+      }
+    }
+    return (int32_t)top((uint32_t)out);
+  }
+};
+
+struct LazyOut {
+  uint32_t *q, *r;   // nullable, at the instance's column
+  uint32_t q_len, q_stride, r_len, r_stride;
+};
+
+// digits an instance's LDS row holds: the dividend's below the first window
+// (at most all of them, and one), or the remainder's
+__host__ __device__ inline uint32_t lazy_row(uint32_t a_len, uint32_t nd) {
+  const uint32_t n = (32u * a_len + D - 1) / D + 2;
+  return (n > nd ? n : nd) | 1u;   // odd: the groups' rows start in different banks
+}
+
+template <int L, int K, class Dividend>
+__device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDividend &B, const LazyOut &o, uint32_t *row,
+                                            bool active) {
+  using Z = Lazy<L, K>;
+  constexpr int ND = Z::ND;
+  const Z z(threadIdx.x & 63);
+  const int l = z.g.l;
+  const int32_t base = (L - 1 - l) * K;   // this lane's lowest digit
+
+  // the divisor's length in bits, from the top
+  int32_t bits = 0;
+  for (int32_t k = (int32_t)B.len - 1;; k -= L) {
+    const uint32_t x = B.limb(k - l);
+    if (x) bits = max(bits, 32 * (k - l) + 32 - __builtin_clz(x));
+    if constexpr (L > 1) {
+#pragma unroll
+      for (int d = 1; d < L; d <<= 1) bits = max(bits, __shfl_xor(bits, d, L));
+    }
+    if (k < L || __builtin_amdgcn_ballot_w64(bits == 0) == 0) break;
+  }
+  const bool zero = bits == 0;
+  const int32_t sh = D * ND - bits;
+  int32_t v[K];
+  {
+    uint32_t x[K];
+    const int32_t at = D * base - sh;
+    digits_at<K>(x, B, at >> 5, (uint32_t)at & 31u);
+#pragma unroll
+    for (int k = 0; k < K; k++) v[k] = (int32_t)x[k];
+  }
+  // -1 / (the top digits), on the group's first lane
+  const double vt = (double)v[K - 1] + (double)v[K - 2] * 0x1p-28;
+  const double ninv = zero ? 0.0 : -1.0 / vt;
+
+  // quotient digits: those of the wave's shortest divisor, the same count for all
+  int32_t nq = (int32_t)(32 * A.len) - bits;
+  nq = nq < 0 ? 1 : (nq + D - 1) / D + 1;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) nq = max(nq, __shfl_xor(nq, d, 64));
+  nq = __builtin_amdgcn_readfirstlane(nq);
+  const int32_t most = (int32_t)((32 * A.len + D - 1) / D) + 1;
+  nq = nq < most ? nq : most;
+
+  // the dividend's digits below the window, a run of them a lane at a time
+  // (16 digits are 14 limbs: every run starts at the same bit of a limb)
+  for (int32_t j = l; kRun * j < nq; j += L) {
+    uint32_t x[kRun];
+    digits_at<kRun>(x, A, D * kRun / 32 * j + (-sh >> 5), (uint32_t)-sh & 31u);
+#pragma unroll
+    for (int k = 0; k < kRun; k++)
+      if (kRun * j + k < nq) row[kRun * j + k] = x[k];
+  }
+  // the window starts as the ND - 1 digits above digit nq - 1 of a 2^sh
+  int64_t t[K];
+  {
+    uint32_t x[K];
+    const int32_t at = D * (nq + base) - sh;
+    digits_at<K>(x, A, at >> 5, (uint32_t)at & 31u);
+#pragma unroll
+    for (int k = 0; k < K; k++) t[k] = base + k < ND - 1 ? (int64_t)(uint64_t)x[k] : 0;
+  }
+  wave_sync();
+
+  uint32_t u = row[nq - 1];
+  for (int32_t j = nq - 1; j >= 0; j--) {
+    const uint32_t un = row[j > 0 ? j - 1 : 0];
+    // R' at the top digit's weight; the top two sums exactly, the third's high word
+    const int64_t y = (int64_t)((uint64_t)t[K - 1] << D) + t[K - 2];
+    const double f = __builtin_fma((double)(int32_t)(y >> 32), 0x1p32, (double)(uint32_t)y);
+    const double e = __builtin_fma((double)(int32_t)(t[K - 3] >> 32), 0x1p4, f);
+    const double m = __builtin_fma(e, ninv, 0x1.8p52);
+    const int32_t q = (int32_t)z.top((uint32_t)__builtin_bit_cast(uint64_t, m));   // -q
+    const int64_t below = z.from_below(t[K - 1]);
+    const bool first = L == 1 || l == 0, last = L == 1 || l == L - 1;
+    t[K - 1] = (first ? y : t[K - 2]) + (int64_t)q * v[K - 1];
+#pragma unroll
+    for (int k = K - 2; k > 0; k--) t[k] = t[k - 1] + (int64_t)q * v[k];
+    t[0] = (last ? (int64_t)(uint64_t)u : below) + (int64_t)q * v[0];
+    row[j] = (uint32_t)-q;
+    u = un;
+  }
+  // carry R; negative: one V more and one less in the quotient
+  uint32_t r[K];
+  const int32_t sign = z.carry(r, t);
+  if (__builtin_amdgcn_ballot_w64(sign < 0) != 0) {
+#pragma unroll
+    for (int k = 0; k < K; k++) t[k] = (int64_t)r[k] + (sign < 0 ? v[k] : 0);
+    (void)z.carry(r, t);
+  }
+  wave_sync();
+  if (o.q) {
+    // carry the quotient's digits: each lane a run of them, then its borrow
+    // up the runs while there is one
+    const int32_t run = (nq + L - 1) / L;
+    const int32_t lo = min(l * run, nq), hi = min(lo + run, nq);
+    int32_t c = l == 0 && sign < 0 ? -1 : 0;
+    for (int32_t k = lo; k < hi; k += 8) {
+      int32_t x[8];
+#pragma unroll
+      for (int i = 0; i < 8; i++) x[i] = (int32_t)row[min(k + i, hi - 1)];
+#pragma unroll
+      for (int i = 0; i < 8; i++) {
+        const int32_t y = x[i] + c;
+        if (k + i < hi) {
+          row[k + i] = (uint32_t)y & MASK;
+          c = y >> D;
+        }
+      }
+    }
+    if constexpr (L > 1) {
+      for (int round = 1; round < L; round++) {
+        c = (int32_t)__shfl_up(c, 1, L);
+        if (l == 0) c = 0;
+        if (__builtin_amdgcn_ballot_w64(c != 0) == 0) break;
+        for (int32_t k = lo; k < hi && c != 0; k++) {
+          const int32_t x = (int32_t)row[k] + c;
+          row[k] = (uint32_t)x & MASK;
+          c = x >> D;
+        }
+      }
+    }
+    wave_sync();
+    for (uint32_t m = (uint32_t)l; 7 * m < o.q_len; m += L) {
+      uint32_t w[7];
+      limbs7(w, row, nq, (int32_t)m, 0, 0);
+      if (active) {
+#pragma unroll
+        for (uint32_t j = 0; j < 7; j++)
+          if (7 * m + j < o.q_len) o.q[(size_t)(7 * m + j) * o.q_stride] = zero ? 0u : w[j];
+      }
+    }
+  }
+  if (o.r) {
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < K; k++) row[base + k] = r[k];
+    wave_sync();
+    const int32_t skip = sh / D;
+    for (uint32_t m = (uint32_t)l; 7 * m < o.r_len; m += L) {
+      uint32_t w[7];
+      limbs7(w, row, ND, (int32_t)m, skip, (uint32_t)(sh - D * skip));
+      if (zero) {
+#pragma unroll
+        for (int j = 0; j < 7; j++) w[j] = A.limb((int32_t)(7 * m) + j);
+      }
+      if (active) {
+#pragma unroll
+        for (uint32_t j = 0; j < 7; j++)
+          if (7 * m + j < o.r_len) o.r[(size_t)(7 * m + j) * o.r_stride] = w[j];
+      }
+    }
+  }
+}
+
+// one wave a workgroup, 64 / L divisions
+template <int L, int K>
+__global__ void __launch_bounds__(64) divmod_lazy_kernel(OutOperand q, OutOperand r, Operand a, Operand b,
+                                                         uint32_t count) {
+  extern __shared__ uint32_t div_rows[];
+  const uint32_t grp = threadIdx.x / L;
+  const uint32_t t = blockIdx.x * (64 / L) + grp;
+  const bool active = t < count;
+  const uint32_t i = active ? t : count - 1;   // groups past the end divide the last pair and store nothing
+  LazyOut o{};
+  if (q.data) {
+    o.q = q.data + out_index(q, i);
+    o.q_len = q.len;
+    o.q_stride = q.stride;
+  }
+  if (r.data) {
+    o.r = r.data + out_index(r, i);
+    o.r_len = r.len;
+    o.r_stride = r.stride;
+  }
+  const ArrayDividend A{a.data, a.stride, a.len, in_index(a, i)}, B{b.data, b.stride, b.len, in_index(b, i)};
+  divide_lazy<L, K>(A, B, o, div_rows + grp * lazy_row(a.len, L * K), active);
+}
+
+// 2^e mod m
+template <int L, int K>
+__global__ void __launch_bounds__(64) pow2_mod_lazy_kernel(uint32_t *out, uint32_t out_len, uint32_t out_stride,
+                                                           const uint32_t *m, uint32_t m_len, uint32_t m_stride,
+                                                           uint32_t count, uint32_t e) {
+  extern __shared__ uint32_t div_rows[];
+  const uint32_t grp = threadIdx.x / L;
+  const uint32_t t = blockIdx.x * (64 / L) + grp;
+  const bool active = t < count;
+  const uint32_t i = active ? t : count - 1;
+  LazyOut o{};
+  o.r = out + i;
+  o.r_len = out_len;
+  o.r_stride = out_stride;
+  const PowerDividend A{e, (e >> 5) + 1};
+  const ArrayDividend B{m, m_stride, m_len, i};
+  divide_lazy<L, K>(A, B, o, div_rows + grp * lazy_row(A.len, L * K), active);
+}
+
+struct LazyEntry {
+  uint32_t lanes, digits;
+  void (*div)(OutOperand, OutOperand, Operand, Operand, uint32_t);
+  void (*pow2)(uint32_t *, uint32_t, uint32_t, const uint32_t *, uint32_t, uint32_t, uint32_t, uint32_t);
+};
+#define XMP_LAZY(L, K) {L, K, divmod_lazy_kernel<L, K>, pow2_mod_lazy_kernel<L, K>}
+const LazyEntry kLazy[] = {
+    XMP_LAZY(4, 5),  XMP_LAZY(8, 5),  XMP_LAZY(16, 5), XMP_LAZY(4, 10), XMP_LAZY(8, 10), XMP_LAZY(16, 10), XMP_LAZY(1, 28),
+    XMP_LAZY(2, 28), XMP_LAZY(4, 28), XMP_LAZY(1, 37), XMP_LAZY(2, 37), XMP_LAZY(4, 37), XMP_LAZY(2, 19),  XMP_LAZY(4, 19),
+    XMP_LAZY(8, 19),
+};
+#undef XMP_LAZY
+
+// The lanes a division takes: few for a full batch, whose steps are bound by
+// issue (K multiply-adds and about 20 other instructions a lane), many for a
+// small one, whose steps are bound by the estimate's latency.  For a divisor
+// that `digits` hold, batches up to `count` take the entry.  Measured on one
+// MI355X, us: 2048/1024 bits x 300 (8,5) 10.6, (4,10) 12.0, (1,37) 18.8; x
+// 16,384 18.4, 13.9, 19.6; x 65,536 41, 29, 24; 4096/2048 x 300 (16,5) 14.1,
+// (8,10) 16.4, (4,19) 20, (2,37) 26; x 16,384 38, 30, 27, 29; x 65,536 121,
+// 78, 56, 48; 8192/4096 x 300 (16,10) 23, (8,19) 29, (4,37) 39; x 16,384 75,
+// 55, 49.  Against the 32-bit kernels, one and two lanes a division with
+// borrow chains: 4096/2048 x 300 51 us, x 65,536 71, x 131,072 109 (here 86);
+// 8192/4096 x 32,768 144 (here 72); 1024/512 x 300 12.2 (here (4,5) 9.0), x
+// 65,536 14.0 (here 14.1 and more: up to 512-bit divisors only small batches
+// come here, and none up to 256 bits).
+struct LazyRule {
+  uint32_t digits, count, lanes, per_lane;
+};
+constexpr uint32_t kAny = 0xFFFFFFFFu;
+const LazyRule kRules[] = {
+    {19, 16384, 4, 5},                                                            // 9 .. 16 limbs
+    {28, 4096, 8, 5},    {28, 32768, 4, 10},  {28, kAny, 1, 28},                  // .. 24
+    {37, 4096, 8, 5},    {37, 32768, 4, 10},  {37, kAny, 1, 37},                  // .. 32
+    {38, 4096, 8, 5},    {38, 32768, 4, 10},  {38, kAny, 2, 19},                  // 33
+    {40, 4096, 8, 5},    {40, 32768, 4, 10},  {40, kAny, 2, 28},                  // .. 35
+    {56, 2048, 16, 5},   {56, 8192, 8, 10},   {56, 16384, 4, 19},  {56, kAny, 2, 28},   // .. 49
+    {74, 2048, 16, 5},   {74, 8192, 8, 10},   {74, 24576, 4, 19},  {74, kAny, 2, 37},   // .. 64
+    {76, 2048, 16, 5},   {76, 8192, 8, 10},   {76, kAny, 4, 19},                  // .. 66
+    {112, 2048, 16, 10}, {112, 8192, 8, 19},  {112, kAny, 4, 28},                 // .. 98
+    {148, 2048, 16, 10}, {148, 8192, 8, 19},  {148, kAny, 4, 37},                 // .. 129
+};
+constexpr size_t kLazyLds = 64 * 1024;
+
+const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count) {
+  if (b_len <= 8) return nullptr;
+  const uint32_t nd = (32u * b_len + D - 1) / D;
+  uint32_t digits = 0;   // the smallest that hold the divisor
+  for (const LazyRule &r : kRules)
+    if (nd <= r.digits && !digits) digits = r.digits;
+  if (digits == 19 && count > 16384) return nullptr;
+  // the batch's rule; a dividend too long for its rows in LDS takes the first
+  // of the divisor's rules whose lanes are more and rows fewer
+  for (int any = 0; any < 2; any++)
+    for (const LazyRule &r : kRules)
+      if (r.digits == digits && (any || count <= r.count) &&
+          4 * (size_t)(64 / r.lanes) * lazy_row(a_len, r.lanes * r.per_lane) <= kLazyLds)
+        for (const LazyEntry &e : kLazy)
+          if (e.lanes == r.lanes && e.digits == r.per_lane) return &e;
+  return nullptr;
+}
+
+}  // namespace
+
+bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
+                        hipError_t *st) {
+  const LazyEntry *e = lazy_entry(a.len, b.len, count);
+  if (!e) return false;
+  const uint32_t per = 64 / e->lanes;
+  hipLaunchKernelGGL(e->div, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a.len, e->lanes * e->digits),
+                     stream, q, r, a, b, count);
+  *st = hipGetLastError();
+  return true;
+}
+
+bool launch_pow2_mod_lazy(uint32_t *out, uint32_t out_len, uint32_t out_stride, const uint32_t *m, uint32_t m_len,
+                          uint32_t m_stride, uint32_t count, uint32_t exponent, hipStream_t stream, hipError_t *st) {
+  const uint32_t a_len = (exponent >> 5) + 1;
+  const LazyEntry *e = lazy_entry(a_len, m_len, count);
+  if (!e) return false;
+  const uint32_t per = 64 / e->lanes;
+  hipLaunchKernelGGL(e->pow2, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a_len, e->lanes * e->digits),
+                     stream, out, out_len, out_stride, m, m_len, m_stride, count, exponent);
+  *st = hipGetLastError();
+  return true;
+}
+
+}  // namespace xmp

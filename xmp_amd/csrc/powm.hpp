@@ -16,6 +16,12 @@ constexpr uint32_t kMaxRegDivisorLimbs = 128;
 size_t divmod_scratch_words(uint32_t b_len, uint32_t count);
 hipError_t launch_divmod_ws(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, uint32_t *scratch,
                             hipStream_t stream);
+// the same two by signed radix-2^28 digits (k_div_lazy.hip), for the sizes and
+// batches where that is faster; false, and nothing launched, for the others
+bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
+                        hipError_t *st);
+bool launch_pow2_mod_lazy(uint32_t *out, uint32_t out_len, uint32_t out_stride, const uint32_t *m, uint32_t m_len,
+                          uint32_t m_stride, uint32_t count, uint32_t exponent, hipStream_t stream, hipError_t *st);
 // out[:, t] = 2^e mod m[:, t] for t < count (interleaved, m_stride/out_stride)
 hipError_t launch_pow2_mod(uint32_t *out, uint32_t out_len, uint32_t out_stride, const uint32_t *m, uint32_t m_len,
                            uint32_t m_stride, uint32_t count, uint32_t e, uint32_t *scratch, hipStream_t stream);
