@@ -66,6 +66,10 @@ def _check(handle, a, b, what):
     (66, 14), (65, 8193),                             # 16x5, 4x19
     (67, 15), (98, 2049), (98, 8193),                 # 16x10, 8x19, 4x28
     (99, 14), (128, 2049), (129, 8193), (128, 8194),  # 16x10, 8x19, 4x37
+    (130, 20), (195, 1100), (195, 8193),              # radix 2^27: 16x15, 8x29
+    (196, 15), (256, 513), (256, 8193),               # 32x10, 16x19, 8x38
+    (257, 14), (512, 100), (520, 2049),               # radix 2^26: 64x10, 16x40
+    (521, 14), (1040, 17),                            # 64x20
 ])
 def test_signed_digit_division(handle, lb, n):
     for la in ((2 * lb, lb + 3, lb, max(1, lb // 2), 3 * lb + 1) if n <= 300 else (2 * lb,)):
@@ -76,7 +80,7 @@ def test_signed_digit_division(handle, lb, n):
 def test_signed_digit_division_long_dividends(handle):
     """Rows in LDS up to their limit, more lanes than the batch's rule gives
     where its rows would not fit, and dividends that fit none."""
-    for la, lb, n in ((1024, 64, 30), (1100, 33, 4100), (3500, 20, 14), (4200, 50, 14)):
+    for la, lb, n in ((1024, 64, 30), (1100, 33, 4100), (3500, 20, 14), (4200, 50, 14), (9000, 300, 14)):
         a, b = _operands(7700 + la, n, la, lb)
         _check(handle, a, b, "%d / %d limbs x %d" % (la, lb, n))
 

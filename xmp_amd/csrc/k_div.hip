@@ -874,8 +874,8 @@ hipError_t launch_divmod_ws(OutOperand q, OutOperand r, Operand a, Operand b, ui
   hipError_t st;
   if (launch_divmod_lazy(q, r, a, b, count, stream, &st)) return st;
   const uint32_t nb = b.len;
-  // What is left: divisors up to 512 bits, and dividends too long for the
-  // signed-digit kernels' rows in LDS.  Below 131,072 divisions one lane each
+  // What is left: divisors up to 512 bits or above 33,280, and dividends too
+  // long for the signed-digit kernels' rows in LDS.  Below 131,072 divisions one lane each
   // gives fewer than two waves per SIMD (1,024 SIMDs x 2 x 64 lanes): two
   // lanes per division instead
   if (count < 131072 && nb > 16 && nb <= 128) {

@@ -4,19 +4,20 @@
 // estimate, multiply-subtract and add-back).  Here the quotient digits are
 // signed and the remainder is never carried:
 //
-//  * operands are radix-2^28 digits, the divisor V shifted up to ND = L*K
-//    digits with its top bit set, the remainder ND signed 64-bit lazy sums.
-//    A step takes the next dividend digit in, R' = 2^28 R + u, and subtracts
+//  * operands are radix-2^D digits (D = 28, or 27 and 26 for longer divisors),
+//    the divisor V shifted up to ND = L*K digits with its top bit set, the
+//    remainder ND signed 64-bit lazy sums.
+//    A step takes the next dividend digit in, R' = 2^D R + u, and subtracts
 //    q V with q the nearest integer to R' / V: one v_mad_i64_i32 per digit,
 //    where 32-bit limbs with borrows cost a multiply-add and two
 //    subtractions, in one serial chain from digit to digit;
 //  * q comes from the top three sums in double precision: what they leave
-//    out, and the rounding, move R'/V by less than 2^-18, so |R| stays below
-//    (1/2 + 2^-18) V, no digit is ever corrected, and adding 1.5 * 2^52 in
+//    out, and the rounding, move R'/V by less than 2^-14, so |R| stays below
+//    (1/2 + 2^-14) V, no digit is ever corrected, and adding 1.5 * 2^52 in
 //    the last multiply-add leaves -q in the low word;
-//  * a sum gains at most 2^55 + 2^38 a step and leaves the window after ND
-//    steps: below 2^63 up to 160 digits.  The top sum, folded into the one
-//    below it, is small because R is;
+//  * a sum gains little more than 2^(2D-1) a step and leaves the window after
+//    ND steps: below 2^63 for 160 digits at D = 28, 304 at 27 and 1,280 at 26.
+//    The top sum, folded into the one below it, is small because R is;
 //  * a division spans L lanes of K digits, the top digits on the group's
 //    first lane, whose q the others take by the same DPP moves as the
 //    Montgomery quotient; one 64-bit sum moves a lane up a step;
@@ -36,9 +37,14 @@ namespace xmp {
 
 namespace {
 
-constexpr int D = 28;
-constexpr uint32_t MASK = (1u << D) - 1;
-constexpr int kRun = 16;   // digits that a lane fetches at a time
+// digits whose bits are whole limbs (a lane fetches 14, 13 or 27 limbs at a time)
+template <int D>
+constexpr int kRun = D == 27 ? 32 : 16;
+// digits and limbs of an aligned piece of a result
+template <int D>
+constexpr int kPieceDigits = D == 28 ? 8 : D == 27 ? 32 : 16;
+template <int D>
+constexpr int kPieceLimbs = kPieceDigits<D> * D / 32;
 
 // Dividends and divisors.  load<N>: limbs k0 .. k0 + N - 1, 0 outside
 // [0, len), all loads unconditional, at limbs that exist, and masked (a select
@@ -84,7 +90,7 @@ struct PowerDividend {   // 2^e
 };
 
 // N digits from bit `off` (0 .. 31) of limb w up (they may lie below 0 or past the top)
-template <int N, class Dividend>
+template <int D, int N, class Dividend>
 __device__ __forceinline__ void digits_at(uint32_t (&d)[N], const Dividend &a, int32_t w, uint32_t off) {
   constexpr int NW = (D * N + 31) / 32;
   uint32_t x[NW + 1];
@@ -94,25 +100,31 @@ __device__ __forceinline__ void digits_at(uint32_t (&d)[N], const Dividend &a, i
 #pragma unroll
   for (int k = 0; k < N; k++) {
     const int j = (D * k) >> 5, s = (D * k) & 31;
-    d[k] = (s + D <= 32 ? x[j] >> s : funnel(x[j + 1 < NW ? j + 1 : j], x[j], s)) & MASK;
+    d[k] = (s + D <= 32 ? x[j] >> s : funnel(x[j + 1 < NW ? j + 1 : j], x[j], s)) & ((1u << D) - 1);
   }
 }
 
-// limbs 7 m .. 7 m + 6 of an integer whose radix-2^28 digits 0 .. n-1 are at
-// d, from digit `skip` and bit s (0 .. 27) of it up: digits 8 m .. 8 m + 7
-__device__ __forceinline__ void limbs7(uint32_t (&w)[7], const uint32_t *d, int32_t n, int32_t m, int32_t skip,
-                                       uint32_t s) {
-  uint32_t x[9];
+// piece m's limbs of an integer whose radix-2^D digits 0 .. n-1 are at d, taken
+// from digit `skip` and bit s (0 .. D-1) of it up
+template <int D>
+__device__ __forceinline__ void piece_limbs(uint32_t (&w)[kPieceLimbs<D>], const uint32_t *d, int32_t n, int32_t m,
+                                            int32_t skip, uint32_t s) {
+  constexpr int P = kPieceDigits<D>;
+  uint32_t x[P + 1];
 #pragma unroll
-  for (int k = 0; k < 9; k++) {
-    const int32_t at = 8 * m + skip + k;
+  for (int k = 0; k <= P; k++) {
+    const int32_t at = P * m + skip + k;
     const uint32_t v = d[min(at, n - 1)], keep = at < n ? ~0u : 0u;
     x[k] = v & keep;
   }
 #pragma unroll
-  for (int k = 0; k < 8; k++) x[k] = (x[k] >> s) | ((x[k + 1] << (D - s)) & MASK);
+  for (int k = 0; k < P; k++) x[k] = (x[k] >> s) | ((x[k + 1] << (D - s)) & ((1u << D) - 1));
 #pragma unroll
-  for (int j = 0; j < 7; j++) w[j] = (x[j] >> (4 * j)) | (x[j + 1] << (D - 4 * j));
+  for (int j = 0; j < kPieceLimbs<D>; j++) {
+    const int k = 32 * j / D, b = 32 * j - D * k;
+    w[j] = (x[k] >> b) | (x[k + 1] << (D - b));
+    if (2 * D - b < 32) w[j] |= x[k + 2 < P ? k + 2 : k] << (2 * D - b);
+  }
 }
 
 __device__ __forceinline__ void wave_sync() {
@@ -120,10 +132,12 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
-template <int L, int K>
+template <int L, int K, int D>
 struct Lazy {
   static constexpr int ND = L * K;
-  static_assert(K >= 3 && ND <= 160, "the estimate's digits on one lane; sums below 2^63");
+  static constexpr uint32_t MASK = (1u << D) - 1;
+  static_assert(K >= 3 && (double)(ND + 1) * (double)(1ull << (2 * D - 1)) < 9.2e18,
+                "the estimate's digits on one lane; sums below 2^63");
   const Group<L> g;
   __device__ __forceinline__ explicit Lazy(int lane) : g(lane) {}
 
@@ -170,16 +184,17 @@ struct LazyOut {
 
 // digits an instance's LDS row holds: the dividend's below the first window
 // (at most all of them, and one), or the remainder's
-__host__ __device__ inline uint32_t lazy_row(uint32_t a_len, uint32_t nd) {
-  const uint32_t n = (32u * a_len + D - 1) / D + 2;
+__host__ __device__ inline uint32_t lazy_row(uint32_t a_len, uint32_t nd, uint32_t d) {
+  const uint32_t n = (32u * a_len + d - 1) / d + 2;
   return (n > nd ? n : nd) | 1u;   // odd: the groups' rows start in different banks
 }
 
-template <int L, int K, class Dividend>
+template <int L, int K, int D, class Dividend>
 __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDividend &B, const LazyOut &o, uint32_t *row,
                                             bool active) {
-  using Z = Lazy<L, K>;
+  using Z = Lazy<L, K, D>;
   constexpr int ND = Z::ND;
+  constexpr uint32_t MASK = Z::MASK;
   const Z z(threadIdx.x & 63);
   const int l = z.g.l;
   const int32_t base = (L - 1 - l) * K;   // this lane's lowest digit
@@ -201,12 +216,12 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
   {
     uint32_t x[K];
     const int32_t at = D * base - sh;
-    digits_at<K>(x, B, at >> 5, (uint32_t)at & 31u);
+    digits_at<D, K>(x, B, at >> 5, (uint32_t)at & 31u);
 #pragma unroll
     for (int k = 0; k < K; k++) v[k] = (int32_t)x[k];
   }
   // -1 / (the top digits), on the group's first lane
-  const double vt = (double)v[K - 1] + (double)v[K - 2] * 0x1p-28;
+  const double vt = (double)v[K - 1] + (double)v[K - 2] * (1.0 / (double)(1u << D));
   const double ninv = zero ? 0.0 : -1.0 / vt;
 
   // quotient digits: those of the wave's shortest divisor, the same count for all
@@ -219,20 +234,21 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
   nq = nq < most ? nq : most;
 
   // the dividend's digits below the window, a run of them a lane at a time
-  // (16 digits are 14 limbs: every run starts at the same bit of a limb)
-  for (int32_t j = l; kRun * j < nq; j += L) {
-    uint32_t x[kRun];
-    digits_at<kRun>(x, A, D * kRun / 32 * j + (-sh >> 5), (uint32_t)-sh & 31u);
+  // (whole limbs, so every run starts at the same bit of one)
+  constexpr int RUN = kRun<D>;
+  for (int32_t j = l; RUN * j < nq; j += L) {
+    uint32_t x[RUN];
+    digits_at<D, RUN>(x, A, D * RUN / 32 * j + (-sh >> 5), (uint32_t)-sh & 31u);
 #pragma unroll
-    for (int k = 0; k < kRun; k++)
-      if (kRun * j + k < nq) row[kRun * j + k] = x[k];
+    for (int k = 0; k < RUN; k++)
+      if (RUN * j + k < nq) row[RUN * j + k] = x[k];
   }
   // the window starts as the ND - 1 digits above digit nq - 1 of a 2^sh
   int64_t t[K];
   {
     uint32_t x[K];
     const int32_t at = D * (nq + base) - sh;
-    digits_at<K>(x, A, at >> 5, (uint32_t)at & 31u);
+    digits_at<D, K>(x, A, at >> 5, (uint32_t)at & 31u);
 #pragma unroll
     for (int k = 0; k < K; k++) t[k] = base + k < ND - 1 ? (int64_t)(uint64_t)x[k] : 0;
   }
@@ -244,7 +260,7 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
     // R' at the top digit's weight; the top two sums exactly, the third's high word
     const int64_t y = (int64_t)((uint64_t)t[K - 1] << D) + t[K - 2];
     const double f = __builtin_fma((double)(int32_t)(y >> 32), 0x1p32, (double)(uint32_t)y);
-    const double e = __builtin_fma((double)(int32_t)(t[K - 3] >> 32), 0x1p4, f);
+    const double e = __builtin_fma((double)(int32_t)(t[K - 3] >> 32), (double)(1u << (32 - D)), f);
     const double m = __builtin_fma(e, ninv, 0x1.8p52);
     const int32_t q = (int32_t)z.top((uint32_t)__builtin_bit_cast(uint64_t, m));   // -q
     const int64_t below = z.from_below(t[K - 1]);
@@ -265,6 +281,7 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
     (void)z.carry(r, t);
   }
   wave_sync();
+  constexpr uint32_t W = kPieceLimbs<D>;
   if (o.q) {
     // carry the quotient's digits: each lane a run of them, then its borrow
     // up the runs while there is one
@@ -297,13 +314,13 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
       }
     }
     wave_sync();
-    for (uint32_t m = (uint32_t)l; 7 * m < o.q_len; m += L) {
-      uint32_t w[7];
-      limbs7(w, row, nq, (int32_t)m, 0, 0);
+    for (uint32_t m = (uint32_t)l; W * m < o.q_len; m += L) {
+      uint32_t w[W];
+      piece_limbs<D>(w, row, nq, (int32_t)m, 0, 0);
       if (active) {
 #pragma unroll
-        for (uint32_t j = 0; j < 7; j++)
-          if (7 * m + j < o.q_len) o.q[(size_t)(7 * m + j) * o.q_stride] = zero ? 0u : w[j];
+        for (uint32_t j = 0; j < W; j++)
+          if (W * m + j < o.q_len) o.q[(size_t)(W * m + j) * o.q_stride] = zero ? 0u : w[j];
       }
     }
   }
@@ -313,24 +330,22 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
     for (int k = 0; k < K; k++) row[base + k] = r[k];
     wave_sync();
     const int32_t skip = sh / D;
-    for (uint32_t m = (uint32_t)l; 7 * m < o.r_len; m += L) {
-      uint32_t w[7];
-      limbs7(w, row, ND, (int32_t)m, skip, (uint32_t)(sh - D * skip));
-      if (zero) {
-#pragma unroll
-        for (int j = 0; j < 7; j++) w[j] = A.limb((int32_t)(7 * m) + j);
-      }
+    for (uint32_t m = (uint32_t)l; W * m < o.r_len; m += L) {
+      uint32_t w[W];
+      piece_limbs<D>(w, row, ND, (int32_t)m, skip, (uint32_t)(sh - D * skip));
       if (active) {
 #pragma unroll
-        for (uint32_t j = 0; j < 7; j++)
-          if (7 * m + j < o.r_len) o.r[(size_t)(7 * m + j) * o.r_stride] = w[j];
+        for (uint32_t j = 0; j < W; j++) {
+          const uint32_t k = W * m + j;
+          if (k < o.r_len) o.r[(size_t)k * o.r_stride] = zero ? A.limb((int32_t)k) : w[j];
+        }
       }
     }
   }
 }
 
 // one wave a workgroup, 64 / L divisions
-template <int L, int K>
+template <int L, int K, int D>
 __global__ void __launch_bounds__(64) divmod_lazy_kernel(OutOperand q, OutOperand r, Operand a, Operand b,
                                                          uint32_t count) {
   extern __shared__ uint32_t div_rows[];
@@ -350,11 +365,11 @@ __global__ void __launch_bounds__(64) divmod_lazy_kernel(OutOperand q, OutOperan
     o.r_stride = r.stride;
   }
   const ArrayDividend A{a.data, a.stride, a.len, in_index(a, i)}, B{b.data, b.stride, b.len, in_index(b, i)};
-  divide_lazy<L, K>(A, B, o, div_rows + grp * lazy_row(a.len, L * K), active);
+  divide_lazy<L, K, D>(A, B, o, div_rows + grp * lazy_row(a.len, L * K, D), active);
 }
 
 // 2^e mod m
-template <int L, int K>
+template <int L, int K, int D>
 __global__ void __launch_bounds__(64) pow2_mod_lazy_kernel(uint32_t *out, uint32_t out_len, uint32_t out_stride,
                                                            const uint32_t *m, uint32_t m_len, uint32_t m_stride,
                                                            uint32_t count, uint32_t e) {
@@ -369,19 +384,21 @@ __global__ void __launch_bounds__(64) pow2_mod_lazy_kernel(uint32_t *out, uint32
   o.r_stride = out_stride;
   const PowerDividend A{e, (e >> 5) + 1};
   const ArrayDividend B{m, m_stride, m_len, i};
-  divide_lazy<L, K>(A, B, o, div_rows + grp * lazy_row(A.len, L * K), active);
+  divide_lazy<L, K, D>(A, B, o, div_rows + grp * lazy_row(A.len, L * K, D), active);
 }
 
 struct LazyEntry {
-  uint32_t lanes, digits;
+  uint32_t lanes, digits, radix;
   void (*div)(OutOperand, OutOperand, Operand, Operand, uint32_t);
   void (*pow2)(uint32_t *, uint32_t, uint32_t, const uint32_t *, uint32_t, uint32_t, uint32_t, uint32_t);
 };
-#define XMP_LAZY(L, K) {L, K, divmod_lazy_kernel<L, K>, pow2_mod_lazy_kernel<L, K>}
+#define XMP_LAZY(L, K, D) {L, K, D, divmod_lazy_kernel<L, K, D>, pow2_mod_lazy_kernel<L, K, D>}
 const LazyEntry kLazy[] = {
-    XMP_LAZY(4, 5),  XMP_LAZY(8, 5),  XMP_LAZY(16, 5), XMP_LAZY(4, 10), XMP_LAZY(8, 10), XMP_LAZY(16, 10), XMP_LAZY(1, 28),
-    XMP_LAZY(2, 28), XMP_LAZY(4, 28), XMP_LAZY(1, 37), XMP_LAZY(2, 37), XMP_LAZY(4, 37), XMP_LAZY(2, 19),  XMP_LAZY(4, 19),
-    XMP_LAZY(8, 19),
+    XMP_LAZY(4, 5, 28),   XMP_LAZY(8, 5, 28),   XMP_LAZY(16, 5, 28),  XMP_LAZY(4, 10, 28), XMP_LAZY(8, 10, 28),
+    XMP_LAZY(16, 10, 28), XMP_LAZY(1, 28, 28),  XMP_LAZY(2, 28, 28),  XMP_LAZY(4, 28, 28), XMP_LAZY(1, 37, 28),
+    XMP_LAZY(2, 37, 28),  XMP_LAZY(4, 37, 28),  XMP_LAZY(2, 19, 28),  XMP_LAZY(4, 19, 28), XMP_LAZY(8, 19, 28),
+    XMP_LAZY(16, 15, 27), XMP_LAZY(8, 29, 27),  XMP_LAZY(32, 10, 27), XMP_LAZY(16, 19, 27), XMP_LAZY(8, 38, 27),
+    XMP_LAZY(64, 10, 26), XMP_LAZY(16, 40, 26), XMP_LAZY(64, 20, 26),
 };
 #undef XMP_LAZY
 
@@ -398,39 +415,47 @@ const LazyEntry kLazy[] = {
 // 8192/4096 x 32,768 144 (here 72); 1024/512 x 300 12.2 (here (4,5) 9.0), x
 // 65,536 14.0 (here 14.1 and more: up to 512-bit divisors only small batches
 // come here, and none up to 256 bits).
+//   Longer divisors, against one wave a division with 32-bit limbs in LDS:
+// 12288/6144 x 100 (16,15) 37, 199, x 16,384 (8,29) 98, 752; 16384/8192 x 100
+// (32,10) 43, 291, x 4,096 (16,19) 68, 402, x 16,384 (8,38) 146, 1084;
+// 24576/16384 x 100 (64,10) 43, 415, x 4,096 (16,40) 102, 578; 49152/32000 x
+// 1,024 (64,20) 129, 1822.
 struct LazyRule {
-  uint32_t digits, count, lanes, per_lane;
+  uint32_t limbs, count, lanes, digits, radix;
 };
 constexpr uint32_t kAny = 0xFFFFFFFFu;
 const LazyRule kRules[] = {
-    {19, 16384, 4, 5},                                                            // 9 .. 16 limbs
-    {28, 4096, 8, 5},    {28, 32768, 4, 10},  {28, kAny, 1, 28},                  // .. 24
-    {37, 4096, 8, 5},    {37, 32768, 4, 10},  {37, kAny, 1, 37},                  // .. 32
-    {38, 4096, 8, 5},    {38, 32768, 4, 10},  {38, kAny, 2, 19},                  // 33
-    {40, 4096, 8, 5},    {40, 32768, 4, 10},  {40, kAny, 2, 28},                  // .. 35
-    {56, 2048, 16, 5},   {56, 8192, 8, 10},   {56, 16384, 4, 19},  {56, kAny, 2, 28},   // .. 49
-    {74, 2048, 16, 5},   {74, 8192, 8, 10},   {74, 24576, 4, 19},  {74, kAny, 2, 37},   // .. 64
-    {76, 2048, 16, 5},   {76, 8192, 8, 10},   {76, kAny, 4, 19},                  // .. 66
-    {112, 2048, 16, 10}, {112, 8192, 8, 19},  {112, kAny, 4, 28},                 // .. 98
-    {148, 2048, 16, 10}, {148, 8192, 8, 19},  {148, kAny, 4, 37},                 // .. 129
+    {16, 16384, 4, 5, 28},
+    {24, 4096, 8, 5, 28},    {24, 32768, 4, 10, 28},  {24, kAny, 1, 28, 28},
+    {32, 4096, 8, 5, 28},    {32, 32768, 4, 10, 28},  {32, kAny, 1, 37, 28},
+    {33, 4096, 8, 5, 28},    {33, 32768, 4, 10, 28},  {33, kAny, 2, 19, 28},
+    {35, 4096, 8, 5, 28},    {35, 32768, 4, 10, 28},  {35, kAny, 2, 28, 28},
+    {49, 2048, 16, 5, 28},   {49, 8192, 8, 10, 28},   {49, 16384, 4, 19, 28},  {49, kAny, 2, 28, 28},
+    {64, 2048, 16, 5, 28},   {64, 8192, 8, 10, 28},   {64, 24576, 4, 19, 28},  {64, kAny, 2, 37, 28},
+    {66, 2048, 16, 5, 28},   {66, 8192, 8, 10, 28},   {66, kAny, 4, 19, 28},
+    {98, 2048, 16, 10, 28},  {98, 8192, 8, 19, 28},   {98, kAny, 4, 28, 28},
+    {129, 2048, 16, 10, 28}, {129, 8192, 8, 19, 28},  {129, kAny, 4, 37, 28},
+    {195, 8192, 16, 15, 27}, {195, kAny, 8, 29, 27},
+    {256, 512, 32, 10, 27},  {256, 8192, 16, 19, 27}, {256, kAny, 8, 38, 27},
+    {520, 2048, 64, 10, 26}, {520, kAny, 16, 40, 26},
+    {1040, kAny, 64, 20, 26},
 };
 constexpr size_t kLazyLds = 64 * 1024;
 
 const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count) {
   if (b_len <= 8) return nullptr;
-  const uint32_t nd = (32u * b_len + D - 1) / D;
-  uint32_t digits = 0;   // the smallest that hold the divisor
+  uint32_t limbs = 0;   // the smallest that holds the divisor
   for (const LazyRule &r : kRules)
-    if (nd <= r.digits && !digits) digits = r.digits;
-  if (digits == 19 && count > 16384) return nullptr;
+    if (b_len <= r.limbs && !limbs) limbs = r.limbs;
+  if (limbs == 0 || (limbs == 16 && count > 16384)) return nullptr;
   // the batch's rule; a dividend too long for its rows in LDS takes the first
   // of the divisor's rules whose lanes are more and rows fewer
   for (int any = 0; any < 2; any++)
     for (const LazyRule &r : kRules)
-      if (r.digits == digits && (any || count <= r.count) &&
-          4 * (size_t)(64 / r.lanes) * lazy_row(a_len, r.lanes * r.per_lane) <= kLazyLds)
+      if (r.limbs == limbs && (any || count <= r.count) &&
+          4 * (size_t)(64 / r.lanes) * lazy_row(a_len, r.lanes * r.digits, r.radix) <= kLazyLds)
         for (const LazyEntry &e : kLazy)
-          if (e.lanes == r.lanes && e.digits == r.per_lane) return &e;
+          if (e.lanes == r.lanes && e.digits == r.digits && e.radix == r.radix) return &e;
   return nullptr;
 }
 
@@ -441,7 +466,7 @@ bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32
   const LazyEntry *e = lazy_entry(a.len, b.len, count);
   if (!e) return false;
   const uint32_t per = 64 / e->lanes;
-  hipLaunchKernelGGL(e->div, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a.len, e->lanes * e->digits),
+  hipLaunchKernelGGL(e->div, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a.len, e->lanes * e->digits, e->radix),
                      stream, q, r, a, b, count);
   *st = hipGetLastError();
   return true;
@@ -453,7 +478,7 @@ bool launch_pow2_mod_lazy(uint32_t *out, uint32_t out_len, uint32_t out_stride, 
   const LazyEntry *e = lazy_entry(a_len, m_len, count);
   if (!e) return false;
   const uint32_t per = 64 / e->lanes;
-  hipLaunchKernelGGL(e->pow2, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a_len, e->lanes * e->digits),
+  hipLaunchKernelGGL(e->pow2, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a_len, e->lanes * e->digits, e->radix),
                      stream, out, out_len, out_stride, m, m_len, m_stride, count, exponent);
   *st = hipGetLastError();
   return true;
