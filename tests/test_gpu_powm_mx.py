@@ -57,7 +57,7 @@ def test_matrix_core_powm_edges(handle, bits):
         x.close()
 
 
-@pytest.mark.parametrize("bits,count", [(512, 2048), (1024, 4096), (2048, 4096), (4096, 512)])
+@pytest.mark.parametrize("bits,count", [(480, 2048), (512, 2048), (640, 3072), (1024, 4096), (2048, 4096), (4096, 512)])
 def test_matrix_core_powm_long_runs(handle, bits, count):
     """Batches of full-length exponents: millions of limb sums, some of whose
     moved high words carry (about one limb in 2^15) and some of whose top

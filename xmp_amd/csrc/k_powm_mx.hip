@@ -31,6 +31,8 @@
 // is the rounded top limb of the low tile (the limbs below it move it by less
 // than 2^-15).  m' = -1/m mod R comes from Newton's iteration on the same
 // products.
+#include <type_traits>
+
 #include "devmp.hpp"
 #include "powm.hpp"
 
@@ -361,11 +363,218 @@ struct Mx {
   }
 };
 
+// Moduli of up to eight blocks: the whole product is one tile of 2 S columns,
+// its low half in columns 0 .. S-1 and its high half, where the values live,
+// in S .. 2S-1.  The tile of x y is the accumulator of q m, so the top low
+// limb's total already holds everything that the low half carries: its
+// rounded high word moves to the first high limb with the other high words,
+// and what x y's low digits carry out is not needed for anything else.  Eight
+// matrix instructions and three limb sums a product at S = 8, where the two
+// tiles of the longer moduli would take twelve and four: a wave's serial chain
+// and the matrix cores both shorten.  Measured at 1024 bits x 4,096 1.27 ms
+// (two tiles: 1.42), x 64 0.71 (0.82); 512 bits x 2,048 0.38 (0.44).
+template <int S>
+struct MxHalf {
+  static_assert(S == 4 || S == 8, "one tile");
+  static constexpr int N = 16 * S, LIMBS = 4 * S, T = 1, KB = S / 4;
+  static constexpr int C_BYTES = 16 * 31, T_BYTES = 16 * (S + 6);
+  static constexpr int TOP_LOW = 47 + S, TOP = 47 + 2 * S;   // lanes of the halves' top limbs
+
+  uint8_t *cb, *tb;
+  const uint8_t *cread, *tread;
+  int lane, i, g, rot;
+  uint32_t tshift;
+  bool low, high;
+  uint8_t *clow, *chigh, *twrite;
+  int32_t k8, k16, k24;
+  v4i mp[KB], mt[KB + 1];
+  uint32_t mw[1];   // the high lane's limb of m
+
+  __device__ __forceinline__ MxHalf(uint8_t *lds) {
+    lane = threadIdx.x;
+    i = lane & 15;
+    g = lane >> 4;
+    low = i < S;
+    high = i >= S && i < 2 * S;
+    cb = lds;
+    tb = lds + C_BYTES;
+    cread = cb + 16 * (15 + i - g);
+    tread = tb + 16 * g + ((1 + i) & ~3);
+    tshift = (uint32_t)(1 + i) & 3u;
+    rot = 4 * (g ? lane - 16 : (i ? 47 + i : 63));
+    clow = cb + 16 * (15 + i) + 4 * (3 - g);
+    chigh = cb + 16 * (15 + ((i - S) & 15)) + 4 * (3 - g);
+    twrite = tb + 16 + 16 * (i - S) + 4 * g;
+    asm volatile("s_mov_b32 %0, 0x100" : "=s"(k8));
+    asm volatile("s_mov_b32 %0, 0x10000" : "=s"(k16));
+    asm volatile("s_mov_b32 %0, 0x1000000" : "=s"(k24));
+    for (int b = lane; b < (C_BYTES + T_BYTES) / 16; b += 64) *reinterpret_cast<v4i *>(lds + 16 * b) = v4i{0, 0, 0, 0};
+    mx_fence();
+  }
+
+  __device__ __forceinline__ bool live(int) const { return high; }
+  __device__ __forceinline__ uint32_t limb(int) const { return (uint32_t)(4 * (i - S) + g); }
+
+  // (lanes outside a value's half hold zero digits)
+  __device__ __forceinline__ void put_c(const uint32_t (&e)[1]) const {
+    *reinterpret_cast<uint32_t *>(chigh) = __builtin_bswap32(e[0] ^ kBias);
+  }
+  __device__ __forceinline__ void put_c_low(uint32_t e) const {
+    *reinterpret_cast<uint32_t *>(clow) = __builtin_bswap32(e ^ kBias);
+  }
+  __device__ __forceinline__ void put_t(const uint32_t (&e)[1]) const {
+    if (high) *reinterpret_cast<uint32_t *>(twrite) = e[0] ^ kBias;
+  }
+  __device__ __forceinline__ v4i cfrag(int kb) const { return *reinterpret_cast<const v4i *>(cread - 64 * kb); }
+  __device__ __forceinline__ v4i tfrag(int kb) const {
+    const uint32_t *w = reinterpret_cast<const uint32_t *>(tread + 64 * kb);
+    v4i x;
+    x.x = (int)__builtin_amdgcn_alignbyte(w[1], w[0], tshift);
+    x.y = (int)__builtin_amdgcn_alignbyte(w[2], w[1], tshift);
+    x.z = (int)__builtin_amdgcn_alignbyte(w[3], w[2], tshift);
+    x.w = (int)__builtin_amdgcn_alignbyte(w[4], w[3], tshift);
+    return x;
+  }
+  static __device__ __forceinline__ v4i mfma(v4i t, v4i c, v4i acc) {
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(t, c, acc, 0, 0, 0);
+  }
+  __device__ __forceinline__ int64_t sum(v4i a) const {
+    return (int64_t)a.w * k24 + ((int64_t)a.z * k16 + ((int64_t)a.y * k8 + a.x));
+  }
+
+  // e = lo + the high words c, moved up a limb within one half (`mine`), until
+  // nothing carries.  Lanes outside it give only what a caller leaves in the
+  // lane below its first limb.  Returns what leaves the half's top limb
+  // (lane `top`).
+  template <bool OUT>
+  __device__ __forceinline__ int32_t resolve(uint32_t &e, uint32_t lo, int32_t c, bool mine, int top) const {
+    int32_t out = 0;
+    e = lo;
+    do {
+      if (OUT) out += __builtin_amdgcn_readlane(c, top);
+      const int32_t up = __builtin_amdgcn_ds_bpermute(rot, c);
+      const int64_t x = (int64_t)(uint64_t)e + (mine ? up : 0);
+      e = (uint32_t)x;
+      c = (int32_t)(x >> 32);
+    } while (__builtin_amdgcn_ballot_w64(c != 0) != 0);
+    return out;
+  }
+  __device__ __forceinline__ int32_t resolve(uint32_t (&e)[1], const uint32_t (&lo)[1], int32_t (&c)[1], int32_t) const {
+    return resolve<true>(e[0], lo[0], c[0], high, TOP);
+  }
+  // the low half's balanced digits, what they carry out dropped
+  __device__ __forceinline__ void low_digits(uint32_t &e, v4i a) const {
+    const int64_t s = sum(a);
+    resolve<false>(e, low ? (uint32_t)s : kBias, low ? (int32_t)(s >> 32) : 0, low, TOP_LOW);
+  }
+
+  // the high half's digits of limb sums s, within 0.502 R; from_low joins the
+  // first high limb (lane TOP_LOW's value)
+  __device__ __forceinline__ void digits_mod(uint32_t (&e)[1], int64_t (&s)[1], int32_t from_low) const {
+    for (int it = 0; it < 4; it++) {
+      const int32_t k = __builtin_amdgcn_readlane((int32_t)(s[0] >> 32), TOP);
+      if (k != 0) s[0] -= (int64_t)k * (int64_t)(uint64_t)mw[0];
+      const int32_t c = high ? (int32_t)(s[0] >> 32) : (lane == TOP_LOW ? from_low : 0);
+      const int32_t out = resolve<true>(e[0], high ? (uint32_t)s[0] : kBias, c, high, TOP);
+      if (out == 0) break;
+      from_low = 0;
+      s[0] = (int64_t)(uint64_t)e[0] + (lane == TOP ? (int64_t)out << 32 : 0);
+    }
+  }
+
+  // the low half of (T fragments from tf) * (X in LDS)
+  template <class F>
+  __device__ __forceinline__ void low_product(uint32_t &e, const F &tf, int32_t plus) const {
+    const v4i half = v4i{64, 64, 64, 64};
+    v4i a = mfma(tf(0), cfrag(0), half), b = half;
+    if (KB == 2) b = mfma(tf(KB - 1), cfrag(KB - 1), half);
+    a += b;
+    if (lane == 0) a.x += plus;
+    low_digits(e, a);
+  }
+
+  template <bool XTOP = false, class F>
+  __device__ __forceinline__ void mont(uint32_t (&e)[1], const F &tf) const {
+    const v4i half = v4i{64, 64, 64, 64}, zero = v4i{0, 0, 0, 0};
+    uint32_t q;
+    v4i p;
+    {
+      v4i c[KB + 1], t[KB + 1];
+#pragma unroll
+      for (int kb = 0; kb <= KB; kb++) {
+        c[kb] = cfrag(kb);
+        t[kb] = tf(kb);
+      }
+      p = mfma(t[0], c[0], half);
+      const v4i b = mfma(t[1], c[1], half);
+      if (KB == 2) p = mfma(t[KB], c[KB], p);
+      p += b;
+    }
+    low_digits(q, p);
+    mx_fence();
+    if (XTOP && lane == 0) cb[16 * (15 + S) + 15] = 0;
+    put_c_low(q);
+    mx_fence();
+    low_product(q, [&](int kb) { return mp[kb]; }, 0);
+    mx_fence();
+    put_c_low(q);
+    mx_fence();
+    v4i c[KB + 1];
+#pragma unroll
+    for (int kb = 0; kb <= KB; kb++) c[kb] = cfrag(kb);
+    p = mfma(mt[0], c[0], p);
+    const v4i b = mfma(mt[1], c[1], zero);
+    if (KB == 2) p = mfma(mt[KB], c[KB], p);
+    p += b;
+    int64_t s[1] = {sum(p)};
+    // (lane TOP_LOW: the low half's total is a whole number of R)
+    digits_mod(e, s, (int32_t)((s[0] + (0x80000000ll - (int64_t)kBias)) >> 32));
+  }
+
+  __device__ __forceinline__ bool load_modulus(const Operand &mod, uint32_t mi) {
+    mw[0] = high ? ld_limb(mod, mi, limb(0)) : 0u;
+    const bool not_one = __builtin_amdgcn_ballot_w64(mw[0] != (lane == S ? 1u : 0u)) != 0;
+    const uint32_t m0 = (uint32_t)__builtin_amdgcn_readlane((int)mw[0], S);
+    uint32_t e[1], z;
+    const uint64_t x = (uint64_t)mw[0] + kBias;
+    const int32_t top = resolve<true>(e[0], (uint32_t)x, (int32_t)(x >> 32), high, TOP);
+    put_t(e);
+    if (lane == 0) tb[16 + N] = (uint8_t)top;
+    mx_fence();
+#pragma unroll
+    for (int kb = 0; kb <= KB; kb++) mt[kb] = tfrag(kb);
+    mx_fence();
+    if (lane == 0) tb[16 + N] = 0;
+    // z = -1/m mod 2^32 on the low lanes, then z (2 + m z) doubles the correct bits
+    const uint64_t y = (uint64_t)(lane == 0 ? neg_inverse32(m0) : 0u) + kBias;
+    resolve<false>(z, (uint32_t)y, (int32_t)(y >> 32), low, TOP_LOW);
+    uint8_t *tlow = tb + 16 + 16 * i + 4 * g;
+#pragma unroll 1
+    for (int bits = 32; bits < 8 * N; bits *= 2) {
+      put_c_low(z);
+      if (low) *reinterpret_cast<uint32_t *>(tlow) = z ^ kBias;
+      mx_fence();
+      low_product(e[0], [&](int kb) { return mt[kb]; }, 2);
+      mx_fence();
+      put_c_low(e[0]);
+      mx_fence();
+      low_product(z, [&](int kb) { return tfrag(kb); }, 0);
+      mx_fence();
+    }
+    if (low) *reinterpret_cast<uint32_t *>(tlow) = z ^ kBias;
+    mx_fence();
+#pragma unroll
+    for (int kb = 0; kb < KB; kb++) mp[kb] = tfrag(kb);
+    mx_fence();
+    return not_one && (m0 & 1u) != 0;
+  }
+};
+
 // One wave an instance.  r2 holds 2^(8N + t) mod m, squared `squarings` times
 // into R^2 mod m (t 2^squarings = 8N).
 template <int S, int WAVES>
 __global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args, uint32_t squarings) {
-  using M = Mx<S>;
+  using M = std::conditional_t<(S <= 8), MxHalf<S <= 8 ? S : 8>, Mx<S>>;
   constexpr int T = M::T;
   __shared__ __attribute__((aligned(16))) uint8_t lds[M::C_BYTES + M::T_BYTES];
   const uint32_t local = blockIdx.x;
@@ -521,9 +730,11 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 // that depends on the modulus.  A wave finishes one instance in a quarter to
 // a tenth of a lane group's time, but a full GPU multiplies 64-bit digits of
 // short moduli faster.  Measured on one MI355X, this kernel against the lane
-// layouts, exponents as long as the moduli: 512 bits x 2,048 0.44 against
-// 0.59 ms (4,096: 0.60, 0.59); 544 x 2,048 0.55, 1.12 (4,096: 0.79, 0.63);
-// 1024 x 4,096 1.42, 1.84 (8,192: 2.73, 2.13); 1056 x 4,096 1.85, 1.95
+// layouts, exponents as long as the moduli: 256 bits x 4,096 0.296 against
+// 0.210 ms; 384 x 2,048 0.31, 0.79 (4,096: 0.41, 0.37); 512 x 4,096 0.52, 0.59
+// (8,192: 0.85, 1.04); 544 x 3,072 0.54, 1.12 (4,096: 0.64, 0.63); 768 x 6,144
+// 1.20, 1.61 (8,192: 1.63, 1.62); 1024 x 4,096 1.27, 1.84, x 7,168 1.86, 2.14
+// (8,192: 2.22, 2.13); 1056 x 4,096 1.85, 1.95
 // (6,144: 2.93, 2.68); 1536 x 12,288 7.8, 8.4 (16,384: 10.1, 8.5); 2048 x
 // 1,024 1.96, 6.69, x 12,288 12.1, 14.1 (16,384: 15.8, 14.3); 2080 x 6,144
 // 9.5, 11.9 (8,192: 12.1, 11.9); 3072 x 1,024 4.2, 32.4, x 16,384 40.8, 43.4;
@@ -531,12 +742,11 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 // lines are the same but for 3072 bits, where R^2 mod m and the set-up weigh
 // more: x 16,384 0.82, 0.87, x 65,536 3.03, 2.76.
 bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
-#ifdef XMP_MX_ALWAYS
-  return true;
-#endif
   if (precision <= 256) return false;
-  if (precision <= 640) return count <= 2048;
-  if (precision <= 1024) return count <= 5120;
+  if (precision <= 480) return count <= 2048;
+  if (precision <= 512) return count <= 8192;
+  if (precision <= 640) return count <= 3072;
+  if (precision <= 1024) return count <= 7168;
   if (precision <= 1152) return count <= 4096;
   if (precision <= 2048) return count <= 12288;
   if (precision <= 2176) return count <= 6144;
