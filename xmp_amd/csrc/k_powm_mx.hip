@@ -28,8 +28,8 @@
 // (x y + q m) / R is at most 0.252 R + 0.502 m, and the top limb's high word
 // k, seen before any carry, says whether m is to be subtracted or added once.
 // The low half of x y + q m is zero mod R; what it carries into the high half
-// is the rounded top limb of the low tile (the limbs below it move it by less
-// than 2^-15).  m' = -1/m mod R comes from Newton's iteration on the same
+// is its top limb's total, rounded, of which a few digits are enough
+// (low_carry).  m' = -1/m mod R comes from Newton's iteration on the same
 // products.
 #include <type_traits>
 
@@ -66,6 +66,8 @@ struct Mx {
   static constexpr int KB = S / 4;            // k-blocks of s = 0 .. S-1; k-block KB holds s = S
   static constexpr int NF = (S + 12) / 4 + 1; // C fragments, u0 - 4 kb = -12 .. S
   static constexpr int NQ = 4 * (T - 1) + 4;  // those of a low half product, -12 .. 16 (T-1)
+  static constexpr int DOTS = T == 1 ? 2 : 3; // digits of q m's top low limb that are summed,
+  static constexpr int UNIT = T == 1 ? 16 : 18;   // in units of 2^UNIT: at most 2^31 - 2^22 in all
   static constexpr int TOP = (S - 1) % 16;    // column of the top limb in the last tile
   static constexpr bool PART = S % 16 != 0;   // the last tile's columns past TOP hold nothing
   static constexpr int C_BYTES = 16 * (S + 31);   // blocks -15 .. S+15
@@ -81,6 +83,7 @@ struct Mx {
   v4i mp[KB];                // T fragments of m' and m
   v4i mt[KB + 1];
   uint32_t mw[T];            // this lane's limbs of m
+  int wm[T][DOTS];           // the digits of m that meet this lane's digits in a low half's top digits
 
   __device__ __forceinline__ Mx(uint8_t *lds) {
     lane = threadIdx.x;
@@ -242,6 +245,33 @@ struct Mx {
     return digits(e, a, cin);
   }
 
+  // What the low half of x y + q m carries out, for the biased digits q and x
+  // y's top low limb.  The half's total is a whole number of R, so its top
+  // limb's, rounded, is enough: the limbs below it move it by less than
+  // 2^-15.  Of q m's part of it the top two digits are summed (the third
+  // adds less than 2^30 = 2^22 2^8 with one tile), or the top three.  A few
+  // multiply-adds a lane and a sum over the wave; as one more tile of the
+  // matrix product it took S/4 instructions, as many LDS reads and a limb sum
+  // (2048 bits x 12,288 12.1 ms, now 10.1; 1536 x 12,288 7.8, now 6.6).
+  __device__ __forceinline__ int32_t low_carry(const uint32_t (&q)[T], uint32_t low_top) const {
+    int32_t x = 0;
+#pragma unroll
+    for (int d = 0; d < DOTS; d++) {
+      int32_t t = 0;
+#pragma unroll
+      for (int r = 0; r < T; r++) t = __builtin_amdgcn_sdot4((int)(q[r] ^ kBias), wm[r][d], t, false);
+      x += 24 - 8 * d >= UNIT ? t << ((24 - 8 * d - UNIT) & 31) : t >> ((UNIT - 24 + 8 * d) & 31);
+    }
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);   // row_shr 1, 2, 4, 8
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);   // row_bcast 15, 31
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);
+    const int32_t top = (int32_t)((uint32_t)__builtin_amdgcn_readlane((int)low_top, top_lane(T - 1)) >> UNIT);
+    return (__builtin_amdgcn_readlane(x, 63) + top - (int32_t)(kBias >> UNIT) + (1 << (31 - UNIT))) >> (32 - UNIT);
+  }
+
   // e = x y / R mod m for X in LDS (which this overwrites) and Y's T
   // fragments.  XTOP: X has a digit of its own in block S, cleared once read.
   template <bool XTOP = false, class F>
@@ -283,16 +313,13 @@ struct Mx {
     mx_fence();
     put_c(q);
     mx_fence();
-    v4i cf[NF], lt = v4i{0, 0, 0, 0}, lt2 = v4i{0, 0, 0, 0};
+    carry += low_carry(q, low_top);
+    v4i cf[NF];
 #pragma unroll
-    for (int f = 0; f < NF; f++) cf[f] = cfrag(f);
+    for (int f = 3; f < NF; f++) cf[f] = cfrag(f);
     if (T == 1) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int kb = 0; kb <= KB; kb++) {
-      if (kb < KB) {
-        if (kb % 2 == 1) lt2 = mfma(mt[kb], cf[4 * (T - 1) - kb + 3], lt2);
-        else lt = mfma(mt[kb], cf[4 * (T - 1) - kb + 3], lt);
-      }
 #pragma unroll
       for (int r = 0; r < T; r++)
         if (kb >= 4 * r) {
@@ -300,10 +327,7 @@ struct Mx {
           else hi[r] = mfma(mt[kb], cf[KB + 4 * r - kb + 3], hi[r]);
         }
     }
-    lt += lt2;
     if (T == 1) hi[0] += h2;
-    const int64_t lsum = sum(lt) + (int64_t)(uint64_t)low_top + (0x80000000ll - (int64_t)kBias);
-    carry += __builtin_amdgcn_readlane((int32_t)(lsum >> 32), top_lane(T - 1));
     int64_t s[T];
 #pragma unroll
     for (int r = 0; r < T; r++) s[r] = sum(hi[r]);
@@ -332,6 +356,14 @@ struct Mx {
     mx_fence();
 #pragma unroll
     for (int kb = 0; kb <= KB; kb++) mt[kb] = tfrag(kb);
+#pragma unroll
+    for (int r = 0; r < T; r++) {
+      // digits N-1-d-4l down to N-4-d-4l, the highest first
+      const uint32_t *w = reinterpret_cast<const uint32_t *>(tb + 16 + N - 8 - (live(r) ? 4 * (int)limb(r) : 0));
+#pragma unroll
+      for (int d = 0; d < DOTS; d++)
+        wm[r][d] = live(r) ? (int)__builtin_bswap32(d ? __builtin_amdgcn_alignbyte(w[1], w[0], 4 - d) : w[1]) : 0;
+    }
     mx_fence();
     if (lane == 0) tb[16 + N] = 0;
     // z = -1/m mod 2^32, then z (2 + m z) doubles the correct bits
@@ -729,27 +761,38 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 // Where the matrix cores are faster than the lane layouts: up to a batch size
 // that depends on the modulus.  A wave finishes one instance in a quarter to
 // a tenth of a lane group's time, but a full GPU multiplies 64-bit digits of
-// short moduli faster.  Measured on one MI355X, this kernel against the lane
-// layouts, exponents as long as the moduli: 256 bits x 4,096 0.296 against
-// 0.210 ms; 384 x 2,048 0.31, 0.79 (4,096: 0.41, 0.37); 512 x 4,096 0.52, 0.59
-// (8,192: 0.85, 1.04); 544 x 3,072 0.54, 1.12 (4,096: 0.64, 0.63); 768 x 6,144
-// 1.20, 1.61 (8,192: 1.63, 1.62); 1024 x 4,096 1.27, 1.84, x 7,168 1.86, 2.14
-// (8,192: 2.22, 2.13); 1056 x 4,096 1.85, 1.95
-// (6,144: 2.93, 2.68); 1536 x 12,288 7.8, 8.4 (16,384: 10.1, 8.5); 2048 x
-// 1,024 1.96, 6.69, x 12,288 12.1, 14.1 (16,384: 15.8, 14.3); 2080 x 6,144
-// 9.5, 11.9 (8,192: 12.1, 11.9); 3072 x 1,024 4.2, 32.4, x 16,384 40.8, 43.4;
-// 4096 x 16,384 71, 98; 8192 x 8,192 227, 388.  With 32-bit exponents the
-// lines are the same but for 3072 bits, where R^2 mod m and the set-up weigh
-// more: x 16,384 0.82, 0.87, x 65,536 3.03, 2.76.
+// short moduli faster; and the lane layouts take the same time for any part
+// of the 16,384 or 32,768 instances that fill the GPU, so that past a whole
+// number of those the matrix cores are ahead again.  Measured on one MI355X,
+// this kernel against the lane layouts, in ms:
+//   exponents as long as the moduli: 256 bits x 4,096 0.296, 0.210; 384 x
+//   2,048 0.31, 0.79 (4,096: 0.41, 0.37); 512 x 8,192 0.85, 1.04; 544 x 3,072
+//   0.54, 1.12 (4,096: 0.64, 0.63); 768 x 6,144 1.20, 1.61; 1024 x 7,168 1.86,
+//   2.14 (8,192: 2.22, 2.13); 1056 x 4,096 1.83, 1.91 (6,144: 2.63, 2.58);
+//   1536 x 12,288 6.9, 8.4 (16,384: 9.0, 8.5; 20,480: 10.9, 15.6); 2048 x
+//   1,024 1.9, 6.7, x 16,384 13.4, 14.3 (32,768: 26.0, 24.8; 65,536: 51, 47);
+//   256-bit exponents: 672 x 6,144 0.49, 0.51 (7,168: 0.54, 0.52); 1280 x
+//   6,144 0.69, 0.85 (12,288: 1.32, 1.21); 1568 x 24,576 2.9, 3.1 (28,672:
+//   3.3, 3.1); 1664 x 28,672 3.4, 3.9; 2048 x 28,672 3.5, 3.7, x 57,344 6.7,
+//   7.0; 2176 x 6,144 1.26, 1.70 (16,384: 3.2, 2.7); 2304 x 16,384 3.2, 3.4
+//   (32,768: 6.1, 5.9); 2368 x 65,536 12.1, 14.5; 3072 x 65,536 14.4, 15.4;
+//   32-bit exponents, where R^2 mod m and the set-up weigh more: 2048 x 12,288
+//   0.33, 0.36 (16,384: 0.43, 0.34); 3072 x 24,576 1.15, 1.30 (32,768: 1.53,
+//   1.42); 4096 x 65,536 3.8, 4.3.
 bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
   if (precision <= 256) return false;
   if (precision <= 480) return count <= 2048;
   if (precision <= 512) return count <= 8192;
   if (precision <= 640) return count <= 3072;
+  if (precision <= 704) return count <= 6144;
   if (precision <= 1024) return count <= 7168;
   if (precision <= 1152) return count <= 4096;
-  if (precision <= 2048) return count <= 12288;
-  if (precision <= 2176) return count <= 6144;
+  if (precision <= 1280) return count <= 6144;
+  if (precision <= 2048 && exp_bits <= 64) return count <= 12288;
+  if (precision <= 1600) return count <= 14336 || (count > 16384 && count <= 24576);
+  if (precision <= 2048) return count <= 28672ull * (((uint64_t)count + 32767) / 32768);
+  if (precision <= 2208) return count <= 6144;
+  if (precision <= 2304) return count <= 16384;
   if (precision <= 3072 && exp_bits <= 64) return count <= 24576;
   return true;
 }
