@@ -28,7 +28,7 @@ def _compact(x, size, order, endian):
     return np.ascontiguousarray(w).reshape(x.shape[0], -1)
 
 
-@pytest.mark.parametrize("limbs", [4, 8, 10, 12, 20, 33, 64, 68, 132])
+@pytest.mark.parametrize("limbs", [1, 3, 4, 8, 9, 10, 12, 20, 33, 64, 68, 132])
 @pytest.mark.parametrize("count", [1, 3, 66, 257])
 def test_word_formats(handle, limbs, count):
     L = xmp_amd.lib()
