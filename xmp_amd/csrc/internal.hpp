@@ -50,6 +50,23 @@ struct _xmpExecutionPolicy_t {
   xmpAlgorithm_t algorithm = xmpAlgorithmDefault;
 };
 
+namespace xmp {
+
+// Pinned buffers between a caller's pageable memory and the GPU, of one
+// handle: allocated by its first synchronous transfer, freed with it, idle
+// between calls.
+struct HostStage {
+  static constexpr size_t kSlot = 512u << 10;
+  static constexpr int kSlots = 4;
+  static constexpr size_t kDirect = 256u << 10;   // up to here a kernel reads or writes one slot itself
+  uint8_t *buf = nullptr;
+  hipEvent_t done[kSlots] = {};                    // the slot's last copy
+
+  uint8_t *slot(size_t k) const { return buf + k % kSlots * kSlot; }
+};
+
+}  // namespace xmp
+
 struct _xmpHandle_t {
   hipStream_t stream = nullptr;
   int32_t device = 0;
@@ -63,6 +80,7 @@ struct _xmpHandle_t {
   uint32_t arch = 0;      // gfx major*100+minor*10+stepping (950 on MI355X)
   uint32_t cuCount = 0;   // compute units
   xmpExecutionPolicy_t policy = nullptr;
+  xmp::HostStage stage;
 };
 
 struct _xmpIntegers_t {
@@ -108,6 +126,12 @@ inline bool hip_ok() { return hipPeekAtLastError() == hipSuccess; }
 // true when `p` is device-accessible memory; other pointers are treated as
 // host memory (reference cudaPointerGetAttributes test, src/xmp.cu:522-531)
 bool is_device_pointer(const void *p);
+
+// whether synchronous transfers with `host` go through the handle's slots
+bool staged(xmpHandle_t h, const void *host);
+// Copies results to host memory on the handle's stream.  Unless async it has
+// waited for the stream and `dst` is written.
+hipError_t copy_out(xmpHandle_t h, void *dst, const void *src, size_t bytes, bool async);
 
 // grow-only scratch owned by the handle (reference src/xmp.cu:105-129)
 xmpError_t set_necessary_scratch(xmpHandle_t h, size_t bytes);

@@ -13,6 +13,9 @@
 
 namespace xmp {
 
+// whole words between device and pinned host memory, both 16-byte aligned
+hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream);
+
 // ---- transfer (k_xfer.hip) ----
 // compact words (count x words of `size` bytes, order/endian/nails, optional
 // gather indices) -> interleaved limbs.  Restates xmpTransform

@@ -83,8 +83,8 @@ extern "C" {
 
 // c = sign(a - b) per instance: -1, 0 or +1 (reference logic.cu:26-116).
 // c may be host or device memory; host results land when the stream completes.
-xmpError_t XMPAPI xmpIntegersCmpAsync(xmpHandle_t handle, int32_t *c, const xmpIntegers_t a, const xmpIntegers_t b,
-                                      uint32_t count) {
+static xmpError_t cmp_internal(xmpHandle_t handle, int32_t *c, const xmpIntegers_t a, const xmpIntegers_t b,
+                               uint32_t count, bool async) {
   XMP_TRACE("xmpIntegersCmpAsync");
   XMP_CHECK_NE(c, nullptr);
   if (a->device != handle->device || b->device != handle->device) return xmpErrorInvalidDevice;
@@ -99,15 +99,17 @@ xmpError_t XMPAPI xmpIntegersCmpAsync(xmpHandle_t handle, int32_t *c, const xmpI
   }
   xmpExecutionPolicy_t p = handle->policy;
   if (launch_cmp(dst, make_in(a, p, 0), make_in(b, p, 1), count, handle->stream) != hipSuccess) return xmpErrorCuda;
-  if (host && hipMemcpyAsync(c, dst, sizeof(int32_t) * (size_t)count, hipMemcpyDeviceToHost, handle->stream) !=
-                  hipSuccess)
-    return xmpErrorCuda;
+  if (host && copy_out(handle, c, dst, sizeof(int32_t) * (size_t)count, async) != hipSuccess) return xmpErrorCuda;
   XMP_CHECK_HIP();
   return xmpErrorSuccess;
 }
+xmpError_t XMPAPI xmpIntegersCmpAsync(xmpHandle_t handle, int32_t *c, const xmpIntegers_t a, const xmpIntegers_t b,
+                                      uint32_t count) {
+  return cmp_internal(handle, c, a, b, count, true);
+}
 xmpError_t XMPAPI xmpIntegersCmp(xmpHandle_t handle, int32_t *c, const xmpIntegers_t a, const xmpIntegers_t b,
                                  uint32_t count) {
-  return sync(handle, xmpIntegersCmpAsync(handle, c, a, b, count));
+  return sync(handle, cmp_internal(handle, c, a, b, count, false));
 }
 
 // c = a << shift[i % shift_count] (truncated) or a >> -shift[...] (reference logic.cu:118-208).
@@ -193,7 +195,7 @@ xmpError_t XMPAPI xmpIntegersNot(xmpHandle_t handle, xmpIntegers_t c, const xmpI
 
 // c[i] = number of one bits of instance i (reference logic.cu:541-605).
 // c may be host or device memory.
-xmpError_t XMPAPI xmpIntegersPopcAsync(xmpHandle_t handle, uint32_t *c, const xmpIntegers_t a, uint32_t count) {
+static xmpError_t popc_internal(xmpHandle_t handle, uint32_t *c, const xmpIntegers_t a, uint32_t count, bool async) {
   XMP_TRACE("xmpIntegersPopcAsync");
   XMP_CHECK_NE(c, nullptr);
   if (a->device != handle->device) return xmpErrorInvalidDevice;
@@ -208,14 +210,15 @@ xmpError_t XMPAPI xmpIntegersPopcAsync(xmpHandle_t handle, uint32_t *c, const xm
     dst = (uint32_t *)handle->scratch;
   }
   if (launch_popc(dst, make_in(a, handle->policy, 0), count, handle->stream) != hipSuccess) return xmpErrorCuda;
-  if (host && hipMemcpyAsync(c, dst, sizeof(uint32_t) * (size_t)count, hipMemcpyDeviceToHost, handle->stream) !=
-                  hipSuccess)
-    return xmpErrorCuda;
+  if (host && copy_out(handle, c, dst, sizeof(uint32_t) * (size_t)count, async) != hipSuccess) return xmpErrorCuda;
   XMP_CHECK_HIP();
   return xmpErrorSuccess;
 }
+xmpError_t XMPAPI xmpIntegersPopcAsync(xmpHandle_t handle, uint32_t *c, const xmpIntegers_t a, uint32_t count) {
+  return popc_internal(handle, c, a, count, true);
+}
 xmpError_t XMPAPI xmpIntegersPopc(xmpHandle_t handle, uint32_t *c, const xmpIntegers_t a, uint32_t count) {
-  return sync(handle, xmpIntegersPopcAsync(handle, c, a, count));
+  return sync(handle, popc_internal(handle, c, a, count, false));
 }
 
 }  // extern "C"
