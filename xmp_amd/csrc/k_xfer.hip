@@ -19,9 +19,7 @@ namespace xmp {
 
 namespace {
 
-constexpr int kTileI = 64;  // instances per tile
-constexpr int kTileJ = 32;  // limbs per tile
-constexpr uint32_t kThreads = 256;
+constexpr uint32_t kTileI = 64;  // instances per LDS tile
 
 // byte k (little-endian significance) of a compact integer row held as
 // `words` words of `size` bytes with the given order/endian/nails.
@@ -38,39 +36,70 @@ __device__ __forceinline__ uint32_t import_byte(const uint8_t *row, uint32_t k, 
   return v & (uint32_t)((wmask >> (8 * kb)) & 0xFF);
 }
 
-// A tile's rows are taken in 1 << LJ columns, the fewest that hold what is left
-// of them: short rows (and the last tile of long ones) are not walked as kTileJ
-// words.  The loops keep a length known at compile time, and with it all of a
-// lane's loads in flight.  Imports and exports of 1,115,080 integers of nine
-// limbs 0.022 and 0.019 ms, with whole tiles 0.035 and 0.028; of 2^23 of one
-// limb 0.044, 0.19 and 0.17.
-template <class F>
-__device__ __forceinline__ void for_columns(uint32_t left, F &&tile) {
-  if (left > 16) tile(std::integral_constant<int, 5>());
-  else if (left > 8) tile(std::integral_constant<int, 4>());
-  else if (left > 4) tile(std::integral_constant<int, 3>());
-  else if (left > 1) tile(std::integral_constant<int, 2>());
-  else tile(std::integral_constant<int, 0>());
+// Tiles of kTileI instances by 1 << LJ limbs, the fewest columns that hold a
+// short row (for_tiles), so that it is not walked as 32 words.  One loop length
+// a kernel: known at compile time, all of a lane's loads are in flight, and the
+// code is short, which a small call waits for.  PLAIN: the words run from the
+// least significant and keep their bytes.  Imports and exports of 1,115,080
+// integers of nine limbs 0.020 and 0.018 ms, with 32 columns 0.035 and 0.028; of
+// 2^23 of one limb 0.034, 0.19 and 0.17.
+template <int LJ, bool PLAIN>
+__global__ void __launch_bounds__(256) import_tile_kernel(uint32_t *__restrict__ dst, uint32_t stride, uint32_t nlimbs,
+                                                          const uint32_t *__restrict__ src, uint32_t count, bool rev,
+                                                          bool swap) {
+  __shared__ uint32_t tile[kTileI][(1 << LJ) + 1];
+  const uint32_t i0 = blockIdx.x * kTileI, j0 = blockIdx.y << LJ;
+#pragma unroll
+  for (uint32_t r = threadIdx.x; r < kTileI << LJ; r += 256) {
+    uint32_t ii = r >> LJ, jj = r & ((1u << LJ) - 1);
+    uint32_t i = i0 + ii, j = j0 + jj;
+    const uint32_t at = !PLAIN && rev ? nlimbs - 1 - j : j;
+    const uint32_t v = (i < count && j < nlimbs) ? src[(size_t)i * nlimbs + at] : 0u;
+    tile[ii][jj] = !PLAIN && swap ? __builtin_bswap32(v) : v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = threadIdx.x; r < kTileI << LJ; r += 256) {
+    uint32_t jj = r / kTileI, ii = r % kTileI;
+    uint32_t i = i0 + ii, j = j0 + jj;
+    if (i < count && j < nlimbs) dst[(size_t)j * stride + i] = tile[ii][jj];
+  }
 }
 
-__global__ void import_fast_kernel(uint32_t *__restrict__ dst, uint32_t stride, uint32_t nlimbs,
-                                   const uint32_t *__restrict__ src, uint32_t count, bool rev, bool swap) {
-  __shared__ uint32_t tile[kTileI][kTileJ + 1];
-  uint32_t i0 = blockIdx.x * kTileI, j0 = blockIdx.y * kTileJ;
-  for_columns(nlimbs - j0, [&](auto lj) {
-    for (uint32_t r = threadIdx.x; r < kTileI << lj(); r += kThreads) {
-      uint32_t ii = r >> lj(), jj = r & ((1u << lj()) - 1);
-      uint32_t i = i0 + ii, j = j0 + jj;
-      const uint32_t v = (i < count && j < nlimbs) ? src[(size_t)i * nlimbs + (rev ? nlimbs - 1 - j : j)] : 0u;
-      tile[ii][jj] = swap ? __builtin_bswap32(v) : v;
-    }
-    __syncthreads();
-    for (uint32_t r = threadIdx.x; r < kTileI << lj(); r += kThreads) {
-      uint32_t jj = r / kTileI, ii = r % kTileI;
-      uint32_t i = i0 + ii, j = j0 + jj;
-      if (i < count && j < nlimbs) dst[(size_t)j * stride + i] = tile[ii][jj];
-    }
-  });
+template <int LJ, bool PLAIN>
+__global__ void __launch_bounds__(256) export_tile_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src,
+                                                          uint32_t stride, uint32_t nlimbs, uint32_t count, bool rev,
+                                                          bool swap) {
+  __shared__ uint32_t tile[kTileI][(1 << LJ) + 1];
+  const uint32_t i0 = blockIdx.x * kTileI, j0 = blockIdx.y << LJ;
+#pragma unroll
+  for (uint32_t r = threadIdx.x; r < kTileI << LJ; r += 256) {
+    uint32_t jj = r / kTileI, ii = r % kTileI;
+    uint32_t i = i0 + ii, j = j0 + jj;
+    tile[ii][jj] = (i < count && j < nlimbs) ? src[(size_t)j * stride + i] : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (uint32_t r = threadIdx.x; r < kTileI << LJ; r += 256) {
+    uint32_t ii = r >> LJ, jj = r & ((1u << LJ) - 1);
+    uint32_t i = i0 + ii, j = j0 + jj;
+    const uint32_t v = tile[ii][jj], at = !PLAIN && rev ? nlimbs - 1 - j : j;
+    if (i < count && j < nlimbs) dst[(size_t)i * nlimbs + at] = !PLAIN && swap ? __builtin_bswap32(v) : v;
+  }
+}
+
+// the tile's columns and the grid
+template <class F>
+void for_tiles(uint32_t nlimbs, uint32_t count, F &&launch) {
+  const uint32_t ni = div_round_up(count, kTileI);
+  // (a small call waits for one tile, a large one wants whole lines of rows:
+  // 300 of 33 limbs with the division before them 10.7 us, with 32 columns
+  // 12.2; 655,360 0.048 ms, with 32 columns 0.037 to 0.043)
+  if (nlimbs > 16 && count > 4096) launch(std::integral_constant<int, 5>(), dim3(ni, div_round_up(nlimbs, 32)));
+  else if (nlimbs > 8) launch(std::integral_constant<int, 4>(), dim3(ni, div_round_up(nlimbs, 16)));
+  else if (nlimbs > 4) launch(std::integral_constant<int, 3>(), dim3(ni));
+  else if (nlimbs > 1) launch(std::integral_constant<int, 2>(), dim3(ni));
+  else launch(std::integral_constant<int, 0>(), dim3(ni));
 }
 
 // 4 x 4 blocks: a lane moves limbs 4 jq .. 4 jq + 3 of instances 4 iq .. 4 iq + 3,
@@ -192,26 +221,6 @@ __global__ void import_general_kernel(uint32_t *__restrict__ dst, uint32_t strid
   dst[(size_t)j * stride + i] = v;
 }
 
-__global__ void export_fast_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src, uint32_t stride,
-                                   uint32_t nlimbs, uint32_t count, bool rev, bool swap) {
-  __shared__ uint32_t tile[kTileI][kTileJ + 1];
-  uint32_t i0 = blockIdx.x * kTileI, j0 = blockIdx.y * kTileJ;
-  for_columns(nlimbs - j0, [&](auto lj) {
-    for (uint32_t r = threadIdx.x; r < kTileI << lj(); r += kThreads) {
-      uint32_t jj = r / kTileI, ii = r % kTileI;
-      uint32_t i = i0 + ii, j = j0 + jj;
-      tile[ii][jj] = (i < count && j < nlimbs) ? src[(size_t)j * stride + i] : 0u;
-    }
-    __syncthreads();
-    for (uint32_t r = threadIdx.x; r < kTileI << lj(); r += kThreads) {
-      uint32_t ii = r >> lj(), jj = r & ((1u << lj()) - 1);
-      uint32_t i = i0 + ii, j = j0 + jj;
-      const uint32_t v = tile[ii][jj];
-      if (i < count && j < nlimbs) dst[(size_t)i * nlimbs + (rev ? nlimbs - 1 - j : j)] = swap ? __builtin_bswap32(v) : v;
-    }
-  });
-}
-
 // one thread per output word (size bytes) of the compact output
 __global__ void export_general_kernel(uint8_t *__restrict__ dst, const uint32_t *__restrict__ src, uint32_t stride,
                                       uint32_t nlimbs, uint32_t count, uint32_t words, int32_t order,
@@ -267,9 +276,11 @@ hipError_t launch_import(uint32_t *dst, uint32_t dst_stride, uint32_t nlimbs, co
                          reinterpret_cast<const uint32_t *>(src), count, rev, swap);
     });
   } else if (plain) {
-    dim3 grid(div_round_up(count, kTileI), div_round_up(nlimbs, kTileJ));
-    hipLaunchKernelGGL(import_fast_kernel, grid, dim3(256), 0, stream, dst, dst_stride, nlimbs,
-                       reinterpret_cast<const uint32_t *>(src), count, rev, swap);
+    for_tiles(nlimbs, count, [&](auto lj, dim3 grid) {
+      hipLaunchKernelGGL((rev || swap ? import_tile_kernel<lj(), false> : import_tile_kernel<lj(), true>), grid,
+                         dim3(256), 0, stream, dst, dst_stride, nlimbs, reinterpret_cast<const uint32_t *>(src), count,
+                         rev, swap);
+    });
   } else {
     dim3 grid(div_round_up(count, 256), nlimbs);
     hipLaunchKernelGGL(import_general_kernel, grid, dim3(256), 0, stream, dst, dst_stride, nlimbs, src, count,
@@ -290,9 +301,11 @@ hipError_t launch_export(uint8_t *dst, const uint32_t *src, uint32_t src_stride,
                          src_stride, nlimbs, count, rev, swap);
     });
   } else if (plain) {
-    dim3 grid(div_round_up(count, kTileI), div_round_up(nlimbs, kTileJ));
-    hipLaunchKernelGGL(export_fast_kernel, grid, dim3(256), 0, stream, reinterpret_cast<uint32_t *>(dst), src,
-                       src_stride, nlimbs, count, rev, swap);
+    for_tiles(nlimbs, count, [&](auto lj, dim3 grid) {
+      hipLaunchKernelGGL((rev || swap ? export_tile_kernel<lj(), false> : export_tile_kernel<lj(), true>), grid,
+                         dim3(256), 0, stream, reinterpret_cast<uint32_t *>(dst), src, src_stride, nlimbs, count, rev,
+                         swap);
+    });
   } else {
     dim3 grid(div_round_up(count, 256), words);
     hipLaunchKernelGGL(export_general_kernel, grid, dim3(256), 0, stream, dst, src, src_stride, nlimbs, count,
