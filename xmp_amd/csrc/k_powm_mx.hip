@@ -26,7 +26,9 @@
 //
 // Values stay balanced, |x| <= 0.502 R, for any m < R: q is balanced, so
 // (x y + q m) / R is at most 0.252 R + 0.502 m, and the top limb's high word
-// k, seen before any carry, says whether m is to be subtracted or added once.
+// k, seen before any carry, says whether m is to be subtracted or added once
+// (k m is subtracted whatever k is: no branch on the values but for the rare
+// carries' rounds).
 // The low half of x y + q m is zero mod R; what it carries into the high half
 // is its top limb's total, rounded, of which a few digits are enough
 // (low_carry).  m' = -1/m mod R comes from Newton's iteration on the same
@@ -55,6 +57,12 @@ __device__ __forceinline__ uint32_t neg_inverse32(uint32_t m0) {
 #pragma unroll
   for (int it = 0; it < 4; it++) inv = inv * (2u - m0 * inv);
   return 0u - inv;
+}
+
+// s + k m for a small signed k, with no branch on it
+__device__ __forceinline__ int64_t add_multiple(int64_t s, int32_t k, uint32_t m) {
+  const uint64_t x = (uint64_t)s + (uint64_t)(uint32_t)k * m;
+  return (int64_t)(x - ((uint64_t)(m & (uint32_t)(k >> 31)) << 32));
 }
 
 template <int S>
@@ -200,11 +208,9 @@ struct Mx {
   // or subtracting m
   __device__ __forceinline__ void digits_mod(uint32_t (&e)[T], int64_t (&s)[T], int32_t cin) const {
     for (int it = 0; it < 4; it++) {
-      const int32_t k = __builtin_amdgcn_readlane((int32_t)(s[T - 1] >> 32), top_lane(T - 1));
-      if (k != 0) {
+      const int32_t k = -__builtin_amdgcn_readlane((int32_t)(s[T - 1] >> 32), top_lane(T - 1));
 #pragma unroll
-        for (int r = 0; r < T; r++) s[r] -= (int64_t)k * (int64_t)(uint64_t)mw[r];
-      }
+      for (int r = 0; r < T; r++) s[r] = add_multiple(s[r], k, mw[r]);
       uint32_t lo[T];
       int32_t c[T];
 #pragma unroll
@@ -504,8 +510,7 @@ struct MxHalf {
   // first high limb (lane TOP_LOW's value)
   __device__ __forceinline__ void digits_mod(uint32_t (&e)[1], int64_t (&s)[1], int32_t from_low) const {
     for (int it = 0; it < 4; it++) {
-      const int32_t k = __builtin_amdgcn_readlane((int32_t)(s[0] >> 32), TOP);
-      if (k != 0) s[0] -= (int64_t)k * (int64_t)(uint64_t)mw[0];
+      s[0] = add_multiple(s[0], -__builtin_amdgcn_readlane((int32_t)(s[0] >> 32), TOP), mw[0]);
       const int32_t c = high ? (int32_t)(s[0] >> 32) : (lane == TOP_LOW ? from_low : 0);
       const int32_t out = resolve<true>(e[0], high ? (uint32_t)s[0] : kBias, c, high, TOP);
       if (out == 0) break;
