@@ -607,10 +607,16 @@ struct MxHalf {
   }
 };
 
-// One wave an instance.  r2 holds 2^(8N + t) mod m, squared `squarings` times
-// into R^2 mod m (t 2^squarings = 8N).
+// R^2 mod m is 2^(5/4 8N) mod m, from a division, squared twice.  Each squaring
+// less costs the division as many quotient bits again as it had: with nine to
+// thirteen of them (a division of a few bits) 2048 bits x 12,288 took 0.33 ms
+// with 32-bit exponents and 8192 x 2,048 0.49, with two 0.295 and 0.43, with
+// none 0.297 and 0.436.
+constexpr uint32_t kR2Squarings = 2;
+
+// One wave an instance.  r2 holds 2^(5/4 8N) mod m.
 template <int S, int WAVES>
-__global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args, uint32_t squarings) {
+__global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args) {
   using M = std::conditional_t<(S <= 8), MxHalf<S <= 8 ? S : 8>, Mx<S>>;
   constexpr int T = M::T;
   __shared__ __attribute__((aligned(16))) uint8_t lds[M::C_BYTES + M::T_BYTES];
@@ -641,7 +647,7 @@ __global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args, uint3
     s[r] = (int64_t)kBias + (mx.live(r) && w < args.mod.len ? args.r2[(size_t)w * args.r2_stride + mi] : 0u);
   }
   mx.digits_mod(e, s, 0);
-  for (uint32_t j = 0; j < squarings; j++) {
+  for (uint32_t j = 0; j < kR2Squarings; j++) {
     mx.put_c(e);
     mx.put_t(e);
     mx_fence();
@@ -747,7 +753,7 @@ __global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args, uint3
 
 struct MxEntry {
   uint32_t blocks;
-  void (*kernel)(PowmArgs, uint32_t);
+  void (*kernel)(PowmArgs);
 };
 const MxEntry kMx[] = {
     {4, powm_mx_kernel<4, 4>},   {8, powm_mx_kernel<8, 4>},   {12, powm_mx_kernel<12, 4>}, {16, powm_mx_kernel<16, 4>},
@@ -781,9 +787,9 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 //   3.3, 3.1); 1664 x 28,672 3.4, 3.9; 2048 x 28,672 3.5, 3.7, x 57,344 6.7,
 //   7.0; 2176 x 6,144 1.26, 1.70 (16,384: 3.2, 2.7); 2304 x 16,384 3.2, 3.4
 //   (32,768: 6.1, 5.9); 2368 x 65,536 12.1, 14.5; 3072 x 65,536 14.4, 15.4;
-//   32-bit exponents, where R^2 mod m and the set-up weigh more: 2048 x 12,288
-//   0.33, 0.36 (16,384: 0.43, 0.34); 3072 x 24,576 1.15, 1.30 (32,768: 1.53,
-//   1.42); 4096 x 65,536 3.8, 4.3.
+//   32-bit exponents, where the set-up weighs more: 1312 x 12,288 0.245, 0.208;
+//   1536 x 14,336 0.281, 0.300; 2048 x 16,384 0.363, 0.383, x 24,576 0.52,
+//   0.64; 3072 x 65,536 2.42, 2.52; 4096 x 65,536 3.3, 4.2.
 bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
   if (precision <= 256) return false;
   if (precision <= 480) return count <= 2048;
@@ -792,13 +798,11 @@ bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
   if (precision <= 704) return count <= 6144;
   if (precision <= 1024) return count <= 7168;
   if (precision <= 1152) return count <= 4096;
-  if (precision <= 1280) return count <= 6144;
-  if (precision <= 2048 && exp_bits <= 64) return count <= 12288;
-  if (precision <= 1600) return count <= 14336 || (count > 16384 && count <= 24576);
-  if (precision <= 2048) return count <= 28672ull * (((uint64_t)count + 32767) / 32768);
+  if (precision <= 1312) return count <= 6144;
+  if (precision <= 1600) return count <= 14336 || (count > 16384 && count <= 24576 && exp_bits > 64);
+  if (precision <= 2048) return count <= (exp_bits <= 64 ? 24576ull : 28672ull) * (((uint64_t)count + 32767) / 32768);
   if (precision <= 2208) return count <= 6144;
   if (precision <= 2304) return count <= 16384;
-  if (precision <= 3072 && exp_bits <= 64) return count <= 24576;
   return true;
 }
 
@@ -808,15 +812,15 @@ size_t powm_mx_table_words(uint32_t blocks, uint32_t count, uint32_t window_bits
 
 hipError_t launch_mx_r2(uint32_t blocks, uint32_t *r2, uint32_t r2_stride, const uint32_t *m, uint32_t m_len,
                         uint32_t m_stride, uint32_t count, hipStream_t stream) {
-  const uint32_t rbits = 128u * blocks, j = (uint32_t)__builtin_ctz(rbits);
-  return launch_pow2_mod(r2, m_len, r2_stride, m, m_len, m_stride, count, rbits + (rbits >> j), nullptr, stream);
+  const uint32_t rbits = 128u * blocks;
+  return launch_pow2_mod(r2, m_len, r2_stride, m, m_len, m_stride, count, rbits + (rbits >> kR2Squarings), nullptr,
+                         stream);
 }
 
 hipError_t launch_powm_mx(uint32_t blocks, const PowmArgs &args, hipStream_t stream) {
-  const uint32_t squarings = (uint32_t)__builtin_ctz(128u * blocks);
   for (const MxEntry &e : kMx)
     if (e.blocks == blocks && args.count != 0) {
-      hipLaunchKernelGGL(e.kernel, dim3(args.count), dim3(64), 0, stream, args, squarings);
+      hipLaunchKernelGGL(e.kernel, dim3(args.count), dim3(64), 0, stream, args);
       return hipGetLastError();
     }
   return hipErrorInvalidValue;

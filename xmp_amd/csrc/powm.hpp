@@ -112,7 +112,7 @@ hipError_t launch_wide_r2(uint32_t tier, uint32_t *r2, uint32_t r2_stride, const
 // the 16-byte blocks for a precision, 0 where it does not reach
 uint32_t powm_mx_blocks(uint32_t precision);
 size_t powm_mx_table_words(uint32_t blocks, uint32_t count, uint32_t window_bits);
-// r2 = 2^(128 blocks + t) mod m, which launch_powm_mx squares into R^2 mod m (t the odd part of 128 blocks)
+// r2 = 2^(160 blocks) mod m, which launch_powm_mx squares into R^2 mod m
 hipError_t launch_mx_r2(uint32_t blocks, uint32_t *r2, uint32_t r2_stride, const uint32_t *m, uint32_t m_len,
                         uint32_t m_stride, uint32_t count, hipStream_t stream);
 hipError_t launch_powm_mx(uint32_t blocks, const PowmArgs &args, hipStream_t stream);
