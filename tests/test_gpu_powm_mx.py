@@ -57,6 +57,23 @@ def test_matrix_core_powm_edges(handle, bits):
         x.close()
 
 
+@pytest.mark.parametrize("bits", [5152, 6144, 6176, 7168, 7200, 8192])
+def test_matrix_core_powm_crowded(handle, bits):
+    """More instances than SIMDs: moduli above 5120 bits keep m' in LDS."""
+    n = 1030
+    m, b, e = inputs.powm_class(4700 + bits, n, bits, exp_bits=32)
+    _edge_rows(m, b, e)
+    want = np.zeros_like(m)
+    odd = (m[:, 0] & 1).astype(bool)
+    want[odd] = gmp(O.GO_POWM, int(odd.sum()), bits // 32, b[odd], e[odd], m[odd])
+    M, B, E = handle.from_array(m), handle.from_array(b), handle.from_array(e)
+    out = handle.integers(bits, n)
+    handle.powm(out, B, E, M)
+    assert_rows_equal(out.get(), want, "%d bits" % bits)
+    for x in (M, B, E, out):
+        x.close()
+
+
 @pytest.mark.parametrize("bits,count", [(480, 2048), (512, 2048), (640, 3072), (1024, 4096), (2048, 4096), (4096, 512)])
 def test_matrix_core_powm_long_runs(handle, bits, count):
     """Batches of full-length exponents: millions of limb sums, some of whose

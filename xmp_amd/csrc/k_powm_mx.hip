@@ -65,7 +65,9 @@ __device__ __forceinline__ int64_t add_multiple(int64_t s, int32_t k, uint32_t m
   return (int64_t)(x - ((uint64_t)(m & (uint32_t)(k >> 31)) << 32));
 }
 
-template <int S>
+// MP_LDS keeps m' in LDS, as fragments, instead of S registers: from 48 blocks
+// on a second wave then fits the SIMD.
+template <int S, bool MP_LDS>
 struct Mx {
   static_assert(S % 4 == 0 && S >= 4, "whole k-blocks");
   static constexpr int N = 16 * S;            // bytes of R
@@ -80,6 +82,7 @@ struct Mx {
   static constexpr bool PART = S % 16 != 0;   // the last tile's columns past TOP hold nothing
   static constexpr int C_BYTES = 16 * (S + 31);   // blocks -15 .. S+15
   static constexpr int T_BYTES = 16 * (S + 6);    // bytes -16 .. 16 (S+5) - 1
+  static constexpr int LDS_BYTES = C_BYTES + T_BYTES + (MP_LDS ? 1024 * KB : 0);
 
   uint8_t *cb, *tb;     // LDS: X by reversed blocks, Y plain
   const uint8_t *cread; // this lane's C fragments (offset 16 (u0 - 4 kb + 12))
@@ -88,7 +91,7 @@ struct Mx {
   uint32_t tshift;
   int32_t k8, k16, k24;      // 2^8, 2^16, 2^24 in registers, for v_mad_i64_i32
   v4i bias4;
-  v4i mp[KB];                // T fragments of m' and m
+  v4i mp[MP_LDS ? 1 : KB];   // T fragments of m' and m
   v4i mt[KB + 1];
   uint32_t mw[T];            // this lane's limbs of m
   int wm[T][DOTS];           // the digits of m that meet this lane's digits in a low half's top digits
@@ -144,6 +147,8 @@ struct Mx {
   // constant of the instruction), with more the tiles share a register
   __device__ __forceinline__ v4i bias() const { return T == 1 ? v4i{64, 64, 64, 64} : bias4; }
   __device__ __forceinline__ static v4i bias2() { return v4i{64, 64, 64, 64}; }
+  __device__ __forceinline__ v4i *mp_lds() const { return reinterpret_cast<v4i *>(tb + T_BYTES) + lane; }
+  __device__ __forceinline__ v4i mpfrag(int kb) const { return MP_LDS ? mp_lds()[64 * kb] : mp[kb]; }
   static __device__ __forceinline__ v4i mfma(v4i t, v4i c, v4i acc) {
     return __builtin_amdgcn_mfma_i32_16x16x64_i8(t, c, acc, 0, 0, 0);
   }
@@ -315,7 +320,7 @@ struct Mx {
     if (XTOP && lane == 0) cb[16 * (15 + S) + 15] = 0;
     put_c(q);
     mx_fence();
-    (void)low_product(q, [&](int kb) { return mp[kb]; }, 0);
+    (void)low_product(q, [&](int kb) { return mpfrag(kb); }, 0);
     mx_fence();
     put_c(q);
     mx_fence();
@@ -395,7 +400,10 @@ struct Mx {
     put_t(z);
     mx_fence();
 #pragma unroll
-    for (int kb = 0; kb < KB; kb++) mp[kb] = tfrag(kb);
+    for (int kb = 0; kb < KB; kb++) {
+      if (MP_LDS) mp_lds()[64 * kb] = tfrag(kb);
+      else mp[kb] = tfrag(kb);
+    }
     mx_fence();
     return not_one && (m0 & 1u) != 0;
   }
@@ -415,7 +423,7 @@ template <int S>
 struct MxHalf {
   static_assert(S == 4 || S == 8, "one tile");
   static constexpr int N = 16 * S, LIMBS = 4 * S, T = 1, KB = S / 4;
-  static constexpr int C_BYTES = 16 * 31, T_BYTES = 16 * (S + 6);
+  static constexpr int C_BYTES = 16 * 31, T_BYTES = 16 * (S + 6), LDS_BYTES = C_BYTES + T_BYTES;
   static constexpr int TOP_LOW = 47 + S, TOP = 47 + 2 * S;   // lanes of the halves' top limbs
 
   uint8_t *cb, *tb;
@@ -615,11 +623,11 @@ struct MxHalf {
 constexpr uint32_t kR2Squarings = 2;
 
 // One wave an instance.  r2 holds 2^(5/4 8N) mod m.
-template <int S, int WAVES>
+template <int S, int WAVES, bool MP_LDS = false>
 __global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args) {
-  using M = std::conditional_t<(S <= 8), MxHalf<S <= 8 ? S : 8>, Mx<S>>;
+  using M = std::conditional_t<(S <= 8), MxHalf<S <= 8 ? S : 8>, Mx<S, MP_LDS>>;
   constexpr int T = M::T;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[M::C_BYTES + M::T_BYTES];
+  __shared__ __attribute__((aligned(16))) uint8_t lds[M::LDS_BYTES];
   const uint32_t local = blockIdx.x;
   const uint32_t gi = args.start + local;
   const uint32_t bi = in_index(args.base, gi), ei = in_index(args.exp, gi), mi = in_index(args.mod, gi);
@@ -751,14 +759,24 @@ __global__ void __launch_bounds__(64, WAVES) powm_mx_kernel(PowmArgs args) {
   }
 }
 
+// `crowded`: two waves a SIMD instead of one, for more instances than the GPU
+// has SIMDs.  8192 bits x 8,192 with 256-bit exponents 8.15 -> 6.05 ms, x 2,048
+// 2.14 -> 1.73; up to 1,024 instances the wave alone is faster (1.10 against
+// 1.23; 6144 bits 0.73, 0.78).  Below 48 blocks the registers hold two waves
+// as they are, and a third or fourth gains less than m' in LDS costs (3072 and
+// 4096 bits within 5 % either way).
+constexpr uint32_t kSimds = 1024;
 struct MxEntry {
   uint32_t blocks;
-  void (*kernel)(PowmArgs);
+  void (*kernel)(PowmArgs), (*crowded)(PowmArgs);
 };
 const MxEntry kMx[] = {
-    {4, powm_mx_kernel<4, 4>},   {8, powm_mx_kernel<8, 4>},   {12, powm_mx_kernel<12, 4>}, {16, powm_mx_kernel<16, 4>},
-    {20, powm_mx_kernel<20, 3>}, {24, powm_mx_kernel<24, 3>}, {28, powm_mx_kernel<28, 2>}, {32, powm_mx_kernel<32, 2>},
-    {40, powm_mx_kernel<40, 2>}, {48, powm_mx_kernel<48, 1>}, {56, powm_mx_kernel<56, 1>}, {64, powm_mx_kernel<64, 1>},
+    {4, powm_mx_kernel<4, 4>, powm_mx_kernel<4, 4>},    {8, powm_mx_kernel<8, 4>, powm_mx_kernel<8, 4>},
+    {12, powm_mx_kernel<12, 4>, powm_mx_kernel<12, 4>}, {16, powm_mx_kernel<16, 4>, powm_mx_kernel<16, 4>},
+    {20, powm_mx_kernel<20, 3>, powm_mx_kernel<20, 3>}, {24, powm_mx_kernel<24, 3>, powm_mx_kernel<24, 3>},
+    {28, powm_mx_kernel<28, 2>, powm_mx_kernel<28, 2>}, {32, powm_mx_kernel<32, 2>, powm_mx_kernel<32, 2>},
+    {40, powm_mx_kernel<40, 2>, powm_mx_kernel<40, 2>}, {48, powm_mx_kernel<48, 1>, powm_mx_kernel<48, 2, true>},
+    {56, powm_mx_kernel<56, 1>, powm_mx_kernel<56, 2, true>}, {64, powm_mx_kernel<64, 1>, powm_mx_kernel<64, 2, true>},
 };
 
 }  // namespace
@@ -820,7 +838,7 @@ hipError_t launch_mx_r2(uint32_t blocks, uint32_t *r2, uint32_t r2_stride, const
 hipError_t launch_powm_mx(uint32_t blocks, const PowmArgs &args, hipStream_t stream) {
   for (const MxEntry &e : kMx)
     if (e.blocks == blocks && args.count != 0) {
-      hipLaunchKernelGGL(e.kernel, dim3(args.count), dim3(64), 0, stream, args);
+      hipLaunchKernelGGL(args.count > kSimds ? e.crowded : e.kernel, dim3(args.count), dim3(64), 0, stream, args);
       return hipGetLastError();
     }
   return hipErrorInvalidValue;
