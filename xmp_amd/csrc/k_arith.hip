@@ -3,10 +3,11 @@
 // add/sub (reference src/add_sub.cu:35-256, implementations.h:36-248,
 // digitmp/add.h, digitmp/sub.h): s = (a + b) mod 2^P(s), d = (a - b) mod
 // 2^P(d); inputs are zero-extended to the output length, the carry of an add
-// lands in the next limb, a negative difference wraps.  These are HBM-bound:
-// the fast path gives each lane four consecutive instances so that every limb
+// lands in the next limb, a negative difference wraps.  Large batches are
+// HBM-bound: each lane takes four consecutive instances so that every limb
 // is one 16-byte load per operand (dwordx4) and the carry chains run in
-// registers (v_add_co_u32/v_addc_co_u32).
+// registers (v_add_co_u32/v_addc_co_u32).  Others wait for their loads: there
+// the limbs are split over the waves of a workgroup.
 //
 // mul (reference src/mul.cu:140-303, digitmp/mul.h:24-55): p = a*b mod
 // 2^P(p).  The longer operand is split into radix-2^28 (2^27 above 4096 bits)
@@ -57,6 +58,8 @@ __device__ __forceinline__ u32x4 addsub4(u32x4 a, u32x4 b, uint32_t (&c)[4]) {
   return u32x4{r0, r1, r2, r3};
 }
 
+constexpr uint32_t kSplitWaves = 16;
+
 template <bool SUB, bool FULL>
 __global__ void __launch_bounds__(64) addsub_vec4_kernel(uint32_t *__restrict__ s, uint32_t s_len, uint32_t s_stride,
                                                          const uint32_t *__restrict__ a, uint32_t a_len,
@@ -100,6 +103,70 @@ __global__ void __launch_bounds__(64) addsub_vec4_kernel(uint32_t *__restrict__ 
       s[(size_t)j * s_stride + i] = r;
     }
   }
+}
+
+// The limbs of 64 instances split over a workgroup's waves, K each, so that
+// every load of a pass is in flight at once.  A chunk is summed without what
+// enters it; then it learns that from the chunks below, of which each says
+// whether it carries out and whether it passes a carry on.  LONG: more limbs
+// than one pass takes.
+template <bool SUB, int K, bool LONG>
+__global__ void __launch_bounds__(1024) addsub_split_kernel(uint32_t *__restrict__ s, uint32_t s_len, uint32_t s_stride,
+                                                            const uint32_t *__restrict__ a, uint32_t a_len,
+                                                            uint32_t a_stride, const uint32_t *__restrict__ b,
+                                                            uint32_t b_len, uint32_t b_stride, uint32_t count) {
+  __shared__ uint32_t chunk[LONG ? 2 : 1][kSplitWaves][64];
+  const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const uint32_t i = blockIdx.x * 64 + lane;   // (rows are padded to 64 instances)
+  uint32_t below = 0;                          // what the last pass carried out
+  for (uint32_t base = 0, pass = 0;; base += kSplitWaves * K, pass ^= 1) {
+    const uint32_t j0 = base + w * K;
+    uint32_t av[K], bv[K], c = 0, same = SUB ? 0u : ~0u;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      av[k] = j0 + k < a_len ? a[(size_t)(j0 + k) * a_stride + i] : 0u;
+      bv[k] = j0 + k < b_len ? b[(size_t)(j0 + k) * b_stride + i] : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      addsub_limb<SUB>(av[k], av[k], bv[k], c);
+      same = SUB ? same | av[k] : same & av[k];
+    }
+    chunk[pass][w][lane] = c | (same == (SUB ? 0u : ~0u) ? 2u : 0u);
+    __syncthreads();   // (before a buffer's next writes lies the other's barrier)
+    uint32_t in = below;
+    for (uint32_t v = 0; v < (LONG ? kSplitWaves : w); v++) {
+      const uint32_t x = chunk[pass][v][lane];
+      below = (x | (below & (x >> 1))) & 1u;
+      if (!LONG || v + 1 == w) in = below;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+      addsub_limb<SUB>(av[k], av[k], 0u, in);
+      if (j0 + k < s_len && i < count) s[(size_t)(j0 + k) * s_stride + i] = av[k];
+    }
+    if (!LONG || base + kSplitWaves * K >= s_len) break;
+  }
+}
+
+// The batches that it is for: with four instances a lane the kernel above has
+// one wave for 256 of them, each waiting for its limbs eight at a time (one at
+// a time past a multiple of four instances).  Measured, that against this
+// kernel: 64 limbs x 113 24.6 and 3.5 us, x 4,096 9.5, 3.7, x 65,536 26, 7.7, x
+// 262,144 39, 28; 128 limbs x 262,144 75, 78; 256 limbs x 65,536 109, 33, x
+// 262,144 149, 157; 512 limbs x 65,536 215, 170, x 131,072 243, 336.
+template <bool SUB>
+bool launch_addsub_split(const OutOperand &s, const Operand &a, const Operand &b, uint32_t count, hipStream_t stream) {
+  constexpr uint32_t kPass = 16 * kSplitWaves;
+  if (count == 0 || count > (s.len <= kPass ? 196608u : 65536u)) return false;
+  if (std::min(a.stride, b.stride) < round_up(count, 64)) return false;   // (whole rows of 64 are read)
+  const uint32_t k = s.len <= 8 * kSplitWaves ? 8 : 16, waves = std::min(kSplitWaves, div_round_up(s.len, k));
+  auto kernel = s.len > kPass ? addsub_split_kernel<SUB, 16, true>
+                : k == 16     ? addsub_split_kernel<SUB, 16, false>
+                              : addsub_split_kernel<SUB, 8, false>;
+  hipLaunchKernelGGL(kernel, dim3(div_round_up(count, 64)), dim3(64 * waves), 0, stream, s.data, s.len, s.stride, a.data,
+                     a.len, a.stride, b.data, b.len, b.stride, count);
+  return true;
 }
 
 template <bool SUB>
@@ -611,7 +678,7 @@ __global__ void __launch_bounds__(256) mul_general_kernel(OutOperand p, Operand 
 
 hipError_t launch_add(OutOperand s, Operand a, Operand b, uint32_t count, hipStream_t stream) {
   if (!s.idx && !a.idx && !b.idx && a.count >= count && b.count >= count) {
-    launch_addsub_vec4<false>(s, a, b, count, stream);
+    if (!launch_addsub_split<false>(s, a, b, count, stream)) launch_addsub_vec4<false>(s, a, b, count, stream);
   } else {
     hipLaunchKernelGGL(addsub_general_kernel<false>, dim3(div_round_up(count, 256)), dim3(256), 0, stream, s, a, b,
                        count);
@@ -621,7 +688,7 @@ hipError_t launch_add(OutOperand s, Operand a, Operand b, uint32_t count, hipStr
 
 hipError_t launch_sub(OutOperand d, Operand a, Operand b, uint32_t count, hipStream_t stream) {
   if (!d.idx && !a.idx && !b.idx && a.count >= count && b.count >= count) {
-    launch_addsub_vec4<true>(d, a, b, count, stream);
+    if (!launch_addsub_split<true>(d, a, b, count, stream)) launch_addsub_vec4<true>(d, a, b, count, stream);
   } else {
     hipLaunchKernelGGL(addsub_general_kernel<true>, dim3(div_round_up(count, 256)), dim3(256), 0, stream, d, a, b,
                        count);
