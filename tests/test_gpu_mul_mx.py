@@ -92,3 +92,27 @@ def test_matrix_core_products_gathered_shared_in_place(handle, limbs, n):
     assert_rows_equal(A.get(), gmp(O.GO_MUL, n, limbs, a, b), "in place, truncated")
     for x in (A, B, P, one):
         x.close()
+
+
+def test_beyond_the_matrix_cores(fresh_handle):
+    """One limb past what the kernel holds: all-ones operands through
+    Karatsuba's carry terms, and the schoolbook where the scratch limit leaves
+    Karatsuba no room."""
+    h, n, limbs = fresh_handle, 3, 2049
+    ones = np.full((n, limbs), 0xFFFFFFFF, np.uint32)
+    a, b = _pair(6500, n, limbs, limbs)
+    A, B, S, P = h.from_array(ones), h.from_array(b), h.from_array(a), h.integers(64 * limbs, n)
+    for limit in (0, 4096):
+        h.set_scratch_limit(limit)
+        h.mul(P, A, A)
+        assert_rows_equal(_get(h, P), gmp(O.GO_MUL, n, 2 * limbs, ones, ones), "all ones, limit %d" % limit)
+        h.set_scratch_limit(limit)
+        h.mul(P, S, B)
+        assert_rows_equal(_get(h, P), gmp(O.GO_MUL, n, 2 * limbs, a, b), "limit %d" % limit)
+    for x in (A, B, S, P):
+        x.close()
+
+
+def _get(h, x):
+    h.set_scratch_limit(0)   # the export's staging is scratch too
+    return x.get()
