@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 # widest sizes of the compiled block counts, and one limb above the next smaller
 SIZES = [512, 1024, 1536, 2048, 2560, 3072, 3584, 4096, 5120, 6144, 7168, 8192]
-SIZES += [288] + [b + 32 for b in SIZES[:-1]]
+SIZES += [160, 256, 288] + [b + 32 for b in SIZES[:-1]]
 
 
 def _edge_rows(m, b, e):

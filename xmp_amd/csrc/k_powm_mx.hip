@@ -794,8 +794,9 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 // of the 16,384 or 32,768 instances that fill the GPU, so that past a whole
 // number of those the matrix cores are ahead again.  Measured on one MI355X,
 // this kernel against the lane layouts, in ms:
-//   exponents as long as the moduli: 256 bits x 4,096 0.296, 0.210; 384 x
-//   2,048 0.31, 0.79 (4,096: 0.41, 0.37); 512 x 8,192 0.85, 1.04; 544 x 3,072
+//   exponents as long as the moduli: 160 bits x 512 0.127, 0.133; 256 x 256
+//   0.179, 0.199, x 1,024 0.191, 0.199 (2,048: 0.207, 0.199); 288 x 3,072 0.256,
+//   0.285; 384 x 3,072 0.32, 0.78 (4,096: 0.38, 0.35); 512 x 8,192 0.85, 1.04; 544 x 3,072
 //   0.54, 1.12 (4,096: 0.64, 0.63); 768 x 6,144 1.20, 1.61; 1024 x 7,168 1.86,
 //   2.14 (8,192: 2.22, 2.13); 1056 x 4,096 1.83, 1.91 (6,144: 2.63, 2.58);
 //   1536 x 12,288 6.9, 8.4 (16,384: 9.0, 8.5; 20,480: 10.9, 15.6); 2048 x
@@ -809,8 +810,9 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 //   1536 x 14,336 0.281, 0.300; 2048 x 16,384 0.363, 0.383, x 24,576 0.52,
 //   0.64; 3072 x 65,536 2.42, 2.52; 4096 x 65,536 3.3, 4.2.
 bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
-  if (precision <= 256) return false;
-  if (precision <= 480) return count <= 2048;
+  if (precision <= 128) return false;
+  if (precision <= 256) return count <= 1024;
+  if (precision <= 480) return count <= 3072;
   if (precision <= 512) return count <= 8192;
   if (precision <= 640) return count <= 3072;
   if (precision <= 704) return count <= 6144;
