@@ -172,6 +172,8 @@ def make_keys(nkeys, bits, seed):
     r = 0
     for k in range(nkeys):
         while True:
+            if r + 4 > len(raw):   # (the halves are coprime four times in five)
+                raw = np.concatenate([raw, inputs.uniform(seed + len(raw), 8, h32)])
             p = to_int(raw[r]) | 1 | (1 << (bits // 2 - 1))
             q = to_int(raw[r + 1]) | 1 | (1 << (bits // 2 - 1))
             r += 2
