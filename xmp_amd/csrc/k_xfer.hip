@@ -117,6 +117,17 @@ __device__ __forceinline__ u32x4 to_words(u32x4 v, bool rev, bool swap) {
   return rev ? u32x4{v.w, v.z, v.y, v.x} : v;
 }
 
+template <bool NT>
+__device__ __forceinline__ u32x4 ld_quad(const uint32_t *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
+  else return *reinterpret_cast<const u32x4 *>(p);
+}
+template <bool NT>
+__device__ __forceinline__ void st_quad(uint32_t *p, u32x4 v) {
+  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<u32x4 *>(p));
+  else *reinterpret_cast<u32x4 *>(p) = v;
+}
+
 template <int LJ>
 __device__ __forceinline__ bool quad_at(uint32_t nq, uint32_t count, uint32_t *iq, uint32_t *jq) {
   // a workgroup's four waves: two by two tiles of 8 x 8, else four along the instances
@@ -128,7 +139,7 @@ __device__ __forceinline__ bool quad_at(uint32_t nq, uint32_t count, uint32_t *i
   return *jq < nq && 4 * *iq < count;
 }
 
-template <int LJ>
+template <int LJ, bool NT, bool LINES>
 __global__ void __launch_bounds__(256) import_quads_kernel(uint32_t *__restrict__ dst, uint32_t stride, uint32_t nlimbs,
                                                            const uint32_t *__restrict__ src, uint32_t count, bool rev,
                                                            bool swap) {
@@ -140,21 +151,19 @@ __global__ void __launch_bounds__(256) import_quads_kernel(uint32_t *__restrict_
   u32x4 v[4];
 #pragma unroll
   for (uint32_t e = 0; e < 4; e++)   // (the last row again in the place of those past the end)
-    v[e] = to_words(__builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(row + (size_t)min(e, n - 1) * nlimbs)),
-                    rev, swap);
+    v[e] = to_words(ld_quad<LINES>(row + (size_t)min(e, n - 1) * nlimbs), rev, swap);
   uint32_t *out = dst + (size_t)(4 * jq) * stride + i;
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     if (n == 4) {
-      __builtin_nontemporal_store(u32x4{v[0][k], v[1][k], v[2][k], v[3][k]},
-                                  reinterpret_cast<u32x4 *>(out + (size_t)k * stride));
+      st_quad<NT>(out + (size_t)k * stride, u32x4{v[0][k], v[1][k], v[2][k], v[3][k]});
     } else {
       for (uint32_t e = 0; e < n; e++) out[(size_t)k * stride + e] = e == 0 ? v[0][k] : e == 1 ? v[1][k] : v[2][k];
     }
   }
 }
 
-template <int LJ>
+template <int LJ, bool LINES>
 __global__ void __launch_bounds__(256) export_quads_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src,
                                                            uint32_t stride, uint32_t nlimbs, uint32_t count, bool rev,
                                                            bool swap) {
@@ -166,13 +175,12 @@ __global__ void __launch_bounds__(256) export_quads_kernel(uint32_t *__restrict_
   u32x4 r[4];
 #pragma unroll
   for (int k = 0; k < 4; k++)
-    r[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(in + (size_t)k * stride));
+    r[k] = ld_quad<true>(in + (size_t)k * stride);
   uint32_t *row = dst + (size_t)i * nlimbs + 4 * (rev ? nq - 1 - jq : jq);
 #pragma unroll
   for (int e = 0; e < 4; e++)
     if (i + (uint32_t)e < count)
-      __builtin_nontemporal_store(to_words(u32x4{r[0][e], r[1][e], r[2][e], r[3][e]}, rev, swap),
-                                  reinterpret_cast<u32x4 *>(row + (size_t)e * nlimbs));
+      st_quad<LINES>(row + (size_t)e * nlimbs, to_words(u32x4{r[0][e], r[1][e], r[2][e], r[3][e]}, rev, swap));
 }
 
 // whether a format is 32-bit words in either order with their bytes in either
@@ -195,6 +203,16 @@ void for_quads(uint32_t nlimbs, uint32_t count, F &&launch) {
   else if (nq > 1) launch(std::integral_constant<int, 1>(), dim3(div_round_up(ni, 128)));
   else launch(std::integral_constant<int, 0>(), dim3(div_round_up(ni, 256)));
 }
+
+// Which sides bypass the caches.  An export's limbs are read once, and its rows
+// are written past the caches where they are whole lines (a partial line must wait in
+// the L2 for its other part): an operation and its export, with rows by this rule
+// and by its opposite, 64 limbs x 300,000 products 133 and 148 us, 128-limb
+// quotients and 64-limb remainders x 65,536 62 and 66, 164 limbs x 82,196 96 and
+// 110, 8 limbs x 10^6 sums 34 and 43.  An import's limbs are about to be used, so
+// it stays in the caches that hold it (64 limbs x 300,000 24 and 31 us, 4 x
+// 4,000,000 20 and 29), and passes them by beyond (128 x 2^20 191, 208).
+constexpr size_t kCached = 192u << 20;   // compact bytes; as many again on the other side
 
 // whole words to or from pinned host memory, over the bus: 4 MiB of writes 86 us, 51 GB/s
 __global__ void __launch_bounds__(256) copy_kernel(uint32_t *__restrict__ dst, const uint32_t *__restrict__ src,
@@ -271,8 +289,12 @@ hipError_t launch_import(uint32_t *dst, uint32_t dst_stride, uint32_t nlimbs, co
   const bool plain = in_idx == nullptr && (uintptr_t)src % 4 == 0 &&
                      as_words(words, order, endian, nails, size, nlimbs, &rev, &swap);
   if (plain && nlimbs % 4 == 0 && (uintptr_t)src % 16 == 0) {
+    const bool cached = (size_t)4 * nlimbs * count <= kCached;
     for_quads(nlimbs, count, [&](auto lj, dim3 grid) {
-      hipLaunchKernelGGL(import_quads_kernel<lj()>, grid, dim3(256), 0, stream, dst, dst_stride, nlimbs,
+      auto kernel = cached             ? import_quads_kernel<lj(), false, false>
+                    : nlimbs % 32 == 0 ? import_quads_kernel<lj(), true, true>
+                                       : import_quads_kernel<lj(), true, false>;
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, dst, dst_stride, nlimbs,
                          reinterpret_cast<const uint32_t *>(src), count, rev, swap);
     });
   } else if (plain) {
@@ -297,8 +319,9 @@ hipError_t launch_export(uint8_t *dst, const uint32_t *src, uint32_t src_stride,
                      as_words(words, order, endian, nails, size, nlimbs, &rev, &swap);
   if (plain && nlimbs % 4 == 0 && (uintptr_t)dst % 16 == 0) {
     for_quads(nlimbs, count, [&](auto lj, dim3 grid) {
-      hipLaunchKernelGGL(export_quads_kernel<lj()>, grid, dim3(256), 0, stream, reinterpret_cast<uint32_t *>(dst), src,
-                         src_stride, nlimbs, count, rev, swap);
+      hipLaunchKernelGGL((nlimbs % 32 == 0 ? export_quads_kernel<lj(), true> : export_quads_kernel<lj(), false>), grid,
+                         dim3(256), 0, stream, reinterpret_cast<uint32_t *>(dst), src, src_stride, nlimbs, count, rev,
+                         swap);
     });
   } else if (plain) {
     for_tiles(nlimbs, count, [&](auto lj, dim3 grid) {
