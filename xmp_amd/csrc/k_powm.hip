@@ -699,7 +699,7 @@ struct R2Entry {
 // kMaxRegDivisorLimbs limbs)
 const R2Entry kR2Variants[] = {
     XMP_R2(8, 29, 27), XMP_R2(8, 38, 27), XMP_R2(16, 19, 27), XMP_R2(32, 20, 26), XMP_R2(64, 20, 26),
-    XMP_R2(8, 37, 28),
+    XMP_R2(8, 37, 28), XMP_R2(4, 37, 28),   // (4x37: 4128 bits, 129 limbs)
 };
 #undef XMP_R2
 
