@@ -11,7 +11,9 @@
  *    precision classes (the reference issues one xmpIntegersPowm per class,
  *    src/powm.cu:250-307).
  *  - Tuner: measured choice of lane layout and window per precision
- *    (replaces src/tune/tune.cu and the compiled tables of src/powm.cu:117-236).
+ *    (replaces src/tune/tune.cu and the compiled tables of src/powm.cu:117-236);
+ *    the matrix-core kernel, which the plain call and mixed batches take by a
+ *    rule of the library, is not among its layouts.
  *  - Serving: a continuous-batching request loop over resident moduli.
  */
 #pragma once
@@ -133,7 +135,13 @@ xmpError_t XMPAPI xmpServerRunPoisson(xmpServer_t server, double rate_per_s, uin
  * (capacity `json_bytes`).  Returns the number of measurements in *measured. */
 xmpError_t XMPAPI xmpTunerRun(xmpHandle_t handle, uint32_t precision, uint32_t exp_precision, uint32_t count,
                               char *json, size_t json_bytes, uint32_t *measured);
-/* Load a tuning table (JSON text as written by xmpTunerRun or the tune tool). */
+/* Load a tuning table: JSON text, {"entries": [objects as xmpTunerRun writes
+ * them]}.  Its entries decide the lane layout of every call of the precisions
+ * that they list.  xmpTunerRun measures lane layouts only; with
+ * "matrix_cores": 1 beside "entries", as the tune tool writes and the shipped
+ * table has, xmpIntegersPowm and mixed batches first ask the library's own rule
+ * for the matrix cores, and the table decides the rest: the calls that the rule
+ * leaves, Montgomery contexts and servers. */
 xmpError_t XMPAPI xmpTunerLoad(const char *json);
 
 /* ---------------- allocation-free exponentiation ---------------- */

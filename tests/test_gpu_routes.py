@@ -1,0 +1,129 @@
+"""GPU: which plan a call takes, told by the device memory it allocates.
+
+A handle with its own memory functions records every allocation.  A powm call's
+scratch is R^2 mod m and the window table, whose size tells the lane layouts
+and the matrix-core kernel apart."""
+import ctypes
+import json
+import os
+
+import numpy as np
+import pytest
+
+import xmp_amd
+from helpers import O, assert_rows_equal, gmp, inputs
+from xmp_amd import ext, hip
+
+pytestmark = pytest.mark.gpu
+
+_ALLOC = ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_size_t)
+_FREE = ctypes.CFUNCTYPE(None, ctypes.c_void_p)
+
+
+class Recording(xmp_amd.Handle):
+    """A handle whose device allocations are listed in `sizes`."""
+
+    def __init__(self):
+        libc = ctypes.CDLL(None)
+        libc.malloc.restype, libc.malloc.argtypes = ctypes.c_void_p, [ctypes.c_size_t]
+        libc.free.argtypes = [ctypes.c_void_p]
+        self.sizes = []
+
+        def da(n):
+            self.sizes.append(n)
+            return hip.malloc(max(n, 1))
+
+        self._fns = (_ALLOC(lambda n: libc.malloc(max(n, 1))), _FREE(libc.free), _ALLOC(da),
+                     _FREE(lambda p: hip.free(p) if p else None))
+        self.h = ctypes.c_void_p()
+        rc = xmp_amd.lib().xmpHandleCreateWithMemoryFunctions(
+            ctypes.byref(self.h), *[ctypes.cast(f, ctypes.c_void_p) for f in self._fns])
+        assert rc == 0
+        self._policy = None
+
+
+@pytest.fixture
+def recording():
+    h = Recording()
+    yield h
+    h.close()
+
+
+SHIPPED = os.path.join(os.path.dirname(xmp_amd.LIB_PATH), "tune_gfx950.json")
+
+
+@pytest.fixture
+def tables():
+    yield lambda table: ext.tuner_load(json.dumps(table))
+    with open(SHIPPED) as f:
+        ext.tuner_load(f.read())
+
+
+def _entry(bits, exp_bits, count, layout, window):
+    lanes, digits, radix = layout
+    return {"precision": bits, "exp_bits": exp_bits, "count": count, "lanes": lanes, "digits": digits, "radix": radix,
+            "window": window, "ms": 1.0, "powm_per_s": 1.0}
+
+
+def _r2_bytes(bits, n):
+    return 4 * (bits // 32) * (-(-n // 64) * 64)
+
+
+def _lane_bytes(layout, n, window):
+    return 4 * ((-(-n // 64) * 64) << window) * layout[0] * layout[1]
+
+
+def _mx_bytes(bits, n, window):
+    return 4 * (n << window) * 4 * (bits // 128)   # (sizes of a whole number of compiled blocks)
+
+
+def _powm(h, bits, exp_bits, n):
+    """One call, checked; the device memory that it allocated."""
+    m, b, e = inputs.powm_class(8100 + bits, n, bits, exp_bits=exp_bits)
+    M, B, E, out = h.from_array(m), h.from_array(b), h.from_array(e), h.integers(bits, n)
+    h.sizes.clear()
+    h.powm(out, B, E, M)
+    sizes = list(h.sizes)
+    assert_rows_equal(out.get(), gmp(O.GO_POWM, n, bits // 32, b, e, m), "%d x %d bits" % (n, bits))
+    for x in (M, B, E, out):
+        x.close()
+    return sizes
+
+
+@pytest.mark.parametrize("bits,layout", [(1024, (16, 3, 28)), (3072, (4, 28, 28)), (4096, (4, 37, 28))])
+def test_a_loaded_table_decides(recording, tables, bits, layout):
+    """A program's own table decides the plain call of a precision that it
+    lists; others, and the shipped table's, go to the matrix cores first."""
+    n, exp_bits, window = 100, 96, 3
+    tables({"device": "gfx950", "entries": [_entry(bits, exp_bits, n, layout, window)]})
+    assert _powm(recording, bits, exp_bits, n) == [_r2_bytes(bits, n) + _lane_bytes(layout, n, window)]
+    assert _powm(recording, 2048, exp_bits, 3 * n) == [_r2_bytes(2048, 3 * n) + _mx_bytes(2048, 3 * n, window)]
+    with open(SHIPPED) as f:
+        ext.tuner_load(f.read())
+    n = 700   # (the scratch of the calls before is too short)
+    assert _powm(recording, bits, exp_bits, n) == [_r2_bytes(bits, n) + _mx_bytes(bits, n, window)]
+
+
+def test_a_loaded_table_decides_for_batches(recording, tables):
+    """The classes of a mixed batch that a program's table lists run in the
+    persistent queue, the others on the matrix cores."""
+    sizes, counts, exp_bits, window = (1024, 4096), (70, 30), 96, 3
+    tables({"device": "gfx950", "entries": [_entry(4096, exp_bits, 30, (4, 38, 27), window)]})
+    arrays, wants = [], []
+    for bits, c in zip(sizes, counts):
+        m, b, e = inputs.powm_class(8300 + bits, c, bits, exp_bits=exp_bits)
+        wants.append(gmp(O.GO_POWM, c, bits // 32, b, e, m))
+        arrays.append([recording.integers(bits, c)] + [recording.from_array(x) for x in (b, e, m)])
+    recording.sizes.clear()
+    batch = ext.Batch(recording, *[[a[k] for a in arrays] for k in range(4)], list(counts))
+    assert _mx_bytes(1024, 70, window) in recording.sizes
+    assert _lane_bytes((4, 38, 27), 30, window) in recording.sizes
+    assert _mx_bytes(4096, 30, window) not in recording.sizes
+    for _ in range(2):
+        batch.launch_async()
+        for a, want, bits in zip(arrays, wants, sizes):
+            assert_rows_equal(a[0].get(), want, "batched %d-bit class" % bits)
+    batch.close()
+    for a in arrays:
+        for x in a:
+            x.close()

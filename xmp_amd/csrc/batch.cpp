@@ -173,8 +173,8 @@ xmpError_t XMPAPI xmpBatchCreate(xmpHandle_t handle, xmpBatch_t *batch, uint32_t
     PowmChoice ch;
     e = choose_powm(handle, out[c]->precision, exp[c]->precision, counts[c], xmpAlgorithmDefault, &ch, true);
     if (e != xmpErrorSuccess) break;
-    const uint32_t mx = powm_mx_pays(out[c]->precision, exp[c]->precision,
-                                     (uint32_t)std::min<uint64_t>(instances, 0xFFFFFFFFu))
+    const uint32_t mx = !ch.decided && powm_mx_pays(out[c]->precision, exp[c]->precision,
+                                                    (uint32_t)std::min<uint64_t>(instances, 0xFFFFFFFFu))
                             ? powm_mx_blocks(out[c]->precision)
                             : 0u;
     if (mx) ch.window_bits = best_window_bits(exp[c]->precision);

@@ -24,6 +24,10 @@ struct TunedEntry {
 
 std::mutex g_mu;
 std::vector<TunedEntry> g_table;
+// The table says "matrix_cores": 1 (the shipped one does, which lists lane
+// layouts alone): powm_mx_pays is asked before it.  Without that a table's
+// entries decide every call of the precisions that they list.
+bool g_matrix_cores = false;
 bool g_loaded = false;
 
 bool find_number(const std::string &obj, const char *key, double *out) {
@@ -36,7 +40,9 @@ bool find_number(const std::string &obj, const char *key, double *out) {
   return true;
 }
 
-void parse_table(const std::string &text, std::vector<TunedEntry> *dst) {
+void parse_table(const std::string &text, std::vector<TunedEntry> *dst, bool *matrix_cores) {
+  double mx = 0;
+  *matrix_cores = find_number(text, "matrix_cores", &mx) && mx != 0;
   size_t p = text.find("\"entries\"");
   if (p == std::string::npos) return;
   while (true) {
@@ -79,7 +85,7 @@ void ensure_loaded() {
   size_t n;
   while ((n = std::fread(buf, 1, sizeof buf, f)) > 0) text.append(buf, n);
   std::fclose(f);
-  parse_table(text, &g_table);
+  parse_table(text, &g_table, &g_matrix_cores);
 }
 
 }  // namespace
@@ -89,7 +95,7 @@ int tuner_load_text(const char *text) {
   std::lock_guard<std::mutex> lk(g_mu);
   g_loaded = true;
   std::vector<TunedEntry> t;
-  parse_table(text ? std::string(text) : std::string(), &t);
+  parse_table(text ? std::string(text) : std::string(), &t, &g_matrix_cores);
   g_table.swap(t);
   return (int)g_table.size();
 }
@@ -178,6 +184,7 @@ xmpError_t choose_powm(xmpHandle_t h, uint32_t precision, uint32_t exp_bits, uin
     if (pick) {
       out->variant = powm_find_variant(pick->lanes, pick->digits, pick->radix);
       out->window_bits = eb == exp_bits ? pick->window : best_window_bits(exp_bits);
+      out->decided = !g_matrix_cores;
       return xmpErrorSuccess;
     }
   }
@@ -200,6 +207,7 @@ xmpError_t choose_powm(xmpHandle_t h, uint32_t precision, uint32_t exp_bits, uin
   if (best) {
     out->variant = powm_find_variant(best->lanes, best->digits, best->radix);
     out->window_bits = best->exp_bits == exp_bits ? best->window : best_window_bits(exp_bits);
+    out->decided = !g_matrix_cores;
     return xmpErrorSuccess;
   }
   const uint32_t w = best_window_bits(exp_bits);
@@ -217,6 +225,7 @@ xmpError_t choose_powm(xmpHandle_t h, uint32_t precision, uint32_t exp_bits, uin
   if (bi < 0) return xmpErrorUnsupported;
   out->variant = bi;
   out->window_bits = w;
+  out->decided = false;
   return xmpErrorSuccess;
 }
 

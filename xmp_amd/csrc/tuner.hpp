@@ -17,6 +17,8 @@ namespace xmp {
 struct PowmChoice {
   int variant;
   uint32_t window_bits;
+  // from a table that decides by itself: no kernel outside the table is asked
+  bool decided = false;
 };
 
 // window width minimising table build + one multiply per window for an

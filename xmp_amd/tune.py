@@ -8,7 +8,9 @@ layout (lanes x digits x radix) and the window widths around the modelled best
 on random per-instance moduli; the table is written as JSON next to the
 library (xmp_amd/tune_gfx950.json), where the runtime loads it by default
 ($XMP_TUNE_FILE overrides).  The choice for a call is the fastest layout at
-the smallest measured batch size that holds its batch.
+the smallest measured batch size that holds its batch.  Plain calls and mixed
+batches go to the matrix cores first where the library's own rule says so: the
+table asks for that with "matrix_cores": 1, and one without it decides alone.
 
 Usage (on the GPU):  python -m xmp_amd.tune [--out PATH] [--quick]
 """
@@ -67,6 +69,7 @@ def main():
     entries = sorted(best.values(), key=lambda r: (r["precision"], r["count"], -r["powm_per_s"]))
     table = {"device": "gfx950",
              "note": "measured by xmp_amd/tune.py (xmpTunerRun) on one MI355X; best window per layout and batch size",
+             "matrix_cores": 1,   # lane layouts alone are measured: the matrix cores keep the calls that are theirs
              "entries": entries}
     with open(args.out, "w") as f:
         json.dump(table, f, indent=1)
