@@ -47,10 +47,11 @@ typedef enum {
   xmpScratchSizeLimit
 } xmpExecutionPolicyParam_t;
 
-/* reference xmp.h:62-67.  On this library: Default lets the tuner choose;
- * RegMP forces one lane per instance; DistributedMP forces a multi-lane
- * layout; DigitMP is accepted and treated as Default (there is no
- * digit-serial path; see xmp_ext.h). */
+/* reference xmp.h:62-67.  On this library, for powm: Default takes the matrix
+ * cores where the library's rule finds them faster and a lane layout of the
+ * tuner's table elsewhere (xmpTunerLoad in xmp_ext.h); RegMP forces one lane
+ * per instance; DistributedMP forces a multi-lane layout; DigitMP is accepted
+ * and treated as Default (there is no digit-serial path). */
 typedef enum {
   xmpAlgorithmDefault,
   xmpAlgorithmRegMP,

@@ -127,3 +127,13 @@ def test_a_loaded_table_decides_for_batches(recording, tables):
     for a in arrays:
         for x in a:
             x.close()
+
+
+@pytest.mark.parametrize("bits,n", [(1024, 300), (3072, 50)])
+def test_digitmp_takes_the_default_plan(recording, bits, n):
+    """The digit-serial policy is accepted and treated as the default one."""
+    plans = []
+    for alg, k in ((xmp_amd.ALG_DEFAULT, n), (xmp_amd.ALG_DIGITMP, 2 * n)):   # (scratch only grows)
+        recording.set_algorithm(alg)
+        plans.append(_powm(recording, bits, 96, k))
+        assert plans[-1] == [_r2_bytes(bits, k) + _mx_bytes(bits, k, 3)]

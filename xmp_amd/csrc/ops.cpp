@@ -259,7 +259,8 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   // moduli wider than every lane layout take the workgroup layout (under the
   // default and digit-serial policies, as the reference's DigitMP fallback)
   uint32_t wide = 0;
-  if (e == xmpErrorUnsupported && (p->algorithm == xmpAlgorithmDefault || p->algorithm == xmpAlgorithmDigitMP)) {
+  const bool any = p->algorithm == xmpAlgorithmDefault || p->algorithm == xmpAlgorithmDigitMP;
+  if (e == xmpErrorUnsupported && any) {
     wide = powm_wide_digits_per_thread(out->precision);
     if (wide) {
       c.variant = -1;
@@ -291,8 +292,7 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   const size_t fixed = (r2_words + div_words + r2blk_words + obuf_words) * sizeof(uint32_t);
   uint32_t wbits = c.window_bits;
   uint32_t chunk = count;
-  if (!wide && !c.decided && p->algorithm == xmpAlgorithmDefault &&
-      powm_mx_pays(out->precision, exp->precision, count)) {
+  if (!wide && !c.decided && any && powm_mx_pays(out->precision, exp->precision, count)) {
     mx = powm_mx_blocks(out->precision);
     const uint32_t mx_bits = best_window_bits(exp->precision);
     if (mx && fixed + table_words(count, mx_bits) * sizeof(uint32_t) <= limit)
