@@ -137,3 +137,57 @@ def test_digitmp_takes_the_default_plan(recording, bits, n):
         recording.set_algorithm(alg)
         plans.append(_powm(recording, bits, 96, k))
         assert plans[-1] == [_r2_bytes(bits, k) + _mx_bytes(bits, k, 3)]
+
+
+@pytest.mark.parametrize("bits", [5120, 6144, 8192])
+def test_long_moduli_take_no_division_workspace(recording, bits):
+    """R^2 mod m of the matrix-core kernel is a division in LDS."""
+    assert _powm(recording, bits, 96, 40) == [_r2_bytes(bits, 40) + _mx_bytes(bits, 40, 3)]
+
+
+@pytest.mark.parametrize("la,lb,uses", [
+    (300, 150, False),     # signed digits
+    (2080, 1040, False),
+    (2200, 1100, False),   # a wave's LDS: longer divisors, and dividends too long for the rows
+    (9000, 300, False),
+    (8001, 8000, True),    # neither holds it
+])
+def test_division_allocates_what_its_kernel_uses(recording, la, lb, uses):
+    """A limit still refuses by the sizes alone."""
+    h, n = recording, 40
+    a, b = inputs.uniform(8500 + la, n, la), inputs.uniform(8501 + lb, n, lb)
+    b[:, -1] |= np.uint32(0x80000000)
+    A, B, Q, R = h.from_array(a), h.from_array(b), h.integers(32 * la, n), h.integers(32 * lb, n)
+    words = (2 * lb + 1) * 256
+    h.sizes.clear()
+    h.divmod(Q, R, A, B)
+    assert h.sizes == ([4 * words] if uses else [])
+    wq, wr = gmp(O.GO_DIV, n, la, a, b, out2_limbs=lb)
+    assert_rows_equal(Q.get(), wq, "q")
+    assert_rows_equal(R.get(), wr, "r")
+    h.set_scratch_limit(4 * words - 1)
+    with pytest.raises(xmp_amd.XmpError) as err:
+        h.divmod(Q, R, A, B)
+    assert err.value.code == xmp_amd.INCREASE_SCRATCH_LIMIT
+    h.set_scratch_limit(0)
+    for x in (A, B, Q, R):
+        x.close()
+
+
+def test_short_transfers_take_no_scratch(recording):
+    """Imports and exports through the handle's pinned slots; a limit below
+    their size still refuses them."""
+    h, n, limbs = recording, 50, 20
+    a = inputs.uniform(8600, n, limbs)
+    x = h.integers(32 * limbs, n)
+    h.sizes.clear()
+    x.load(a)
+    assert np.array_equal(x.get(), a)
+    assert h.sizes == []
+    h.set_scratch_limit(4 * n * limbs - 1)
+    for call in (lambda: x.load(a), x.get):
+        with pytest.raises(xmp_amd.XmpError) as err:
+            call()
+        assert err.value.code == xmp_amd.INCREASE_SCRATCH_LIMIT
+    h.set_scratch_limit(0)
+    x.close()

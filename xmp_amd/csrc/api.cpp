@@ -28,10 +28,15 @@ static void device_free(void *p) {
   if (p) (void)hipFree(p);
 }
 
-xmpError_t set_necessary_scratch(xmpHandle_t h, size_t bytes) {
+xmpError_t check_scratch_limit(xmpHandle_t h, size_t bytes) {
   size_t max_size = h->policy ? h->policy->scratch_size_limit : 0;
   if (max_size == 0) max_size = h->memorySize / 4 * 3;   // reference xmp.cu:110-115
-  if (bytes > max_size) return xmpErrorIncreaseScratchLimit;
+  return bytes > max_size ? xmpErrorIncreaseScratchLimit : xmpErrorSuccess;
+}
+
+xmpError_t set_necessary_scratch(xmpHandle_t h, size_t bytes) {
+  const xmpError_t e = check_scratch_limit(h, bytes);
+  if (e != xmpErrorSuccess) return e;
   if (h->scratchSize < bytes) {
     if (h->scratch) h->df(h->scratch);
     h->scratch = h->da(bytes);
@@ -398,14 +403,18 @@ static xmpError_t import_internal(xmpHandle_t handle, xmpIntegers_t out, uint32_
   size_t bytes = rows * words * size;
   const uint8_t *src = (const uint8_t *)in;
   if (!is_device_pointer(in)) {
-    xmpError_t e = set_necessary_scratch(handle, bytes);
+    // (the limit is held against the sizes alone, whichever way the words take)
+    xmpError_t e = check_scratch_limit(handle, bytes);
     if (e != xmpErrorSuccess) return e;
-    src = (const uint8_t *)handle->scratch;
     if (!async && !idx && bytes <= HostStage::kDirect && staged(handle, in)) {
       std::memcpy(handle->stage.slot(0), in, bytes);
       src = handle->stage.slot(0);
-    } else if (hipMemcpyAsync(handle->scratch, in, bytes, hipMemcpyHostToDevice, handle->stream) != hipSuccess) {
-      return xmpErrorCuda;
+    } else {
+      e = set_necessary_scratch(handle, bytes);
+      if (e != xmpErrorSuccess) return e;
+      src = (const uint8_t *)handle->scratch;
+      if (hipMemcpyAsync(handle->scratch, in, bytes, hipMemcpyHostToDevice, handle->stream) != hipSuccess)
+        return xmpErrorCuda;
     }
   }
   if (launch_import(out->limbs, out->stride, out->nlimbs, src, count, words, order, endian, nails, (uint32_t)size,
@@ -452,16 +461,22 @@ static xmpError_t export_internal(xmpHandle_t handle, void *out, uint32_t *words
   size_t bytes = rows * in->nlimbs * 4;
   bool host = !is_device_pointer(out);
   uint8_t *dst = (uint8_t *)out;
+  bool direct = false;
   if (host) {
-    xmpError_t e = set_necessary_scratch(handle, bytes);
+    xmpError_t e = check_scratch_limit(handle, bytes);   // (as for an import)
     if (e != xmpErrorSuccess) return e;
-    dst = (uint8_t *)handle->scratch;
+    direct = !async && !idx && bytes <= HostStage::kDirect && staged(handle, out);
+    if (direct) {
+      dst = handle->stage.slot(0);
+    } else {
+      e = set_necessary_scratch(handle, bytes);
+      if (e != xmpErrorSuccess) return e;
+      dst = (uint8_t *)handle->scratch;
+    }
     // scattered export leaves unselected rows of the caller's buffer untouched
     if (idx && hipMemcpyAsync(dst, out, bytes, hipMemcpyHostToDevice, handle->stream) != hipSuccess)
       return xmpErrorCuda;
   }
-  const bool direct = host && !async && !idx && bytes <= HostStage::kDirect && staged(handle, out);
-  if (direct) dst = handle->stage.slot(0);
   if (launch_export(dst, in->limbs, in->stride, in->nlimbs, count, w, order, endian, nails, (uint32_t)size, idx,
                     idx_count, handle->stream) != hipSuccess)
     return xmpErrorCuda;

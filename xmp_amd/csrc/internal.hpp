@@ -133,6 +133,8 @@ bool staged(xmpHandle_t h, const void *host);
 // waited for the stream and `dst` is written.
 hipError_t copy_out(xmpHandle_t h, void *dst, const void *src, size_t bytes, bool async);
 
+// whether the policy's scratch limit allows so much
+xmpError_t check_scratch_limit(xmpHandle_t h, size_t bytes);
 // grow-only scratch owned by the handle (reference src/xmp.cu:105-129)
 xmpError_t set_necessary_scratch(xmpHandle_t h, size_t bytes);
 // grow-only temporary output for in-place ops (reference src/xmp.cu:131-148)

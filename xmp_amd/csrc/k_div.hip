@@ -861,6 +861,11 @@ size_t divmod_scratch_words(uint32_t b_len, uint32_t count) {
   return (size_t)(2 * b_len + 1) * round_up(count, 256);
 }
 
+bool divmod_uses_scratch(uint32_t a_len, uint32_t b_len, uint32_t count) {
+  return b_len > kMaxRegDivisorLimbs && wave_div_words(a_len, b_len) > kWaveDivMaxWords &&
+         !divmod_lazy_takes(a_len, b_len, count);
+}
+
 template <int H>
 hipError_t launch_divmod_pair(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream) {
   hipLaunchKernelGGL(divmod_pair_kernel<H>, dim3(div_round_up(2 * count, 256)), dim3(256), 0, stream, q, r, a, b,

@@ -461,6 +461,10 @@ const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count) {
 
 }  // namespace
 
+bool divmod_lazy_takes(uint32_t a_len, uint32_t b_len, uint32_t count) {
+  return lazy_entry(a_len, b_len, count) != nullptr;
+}
+
 bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
                         hipError_t *st) {
   const LazyEntry *e = lazy_entry(a.len, b.len, count);

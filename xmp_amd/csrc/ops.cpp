@@ -176,8 +176,12 @@ static xmpError_t divmod_async(xmpHandle_t h, xmpIntegers_t q, xmpIntegers_t m, 
   const int sa = divmod ? 2 : 1, sb = divmod ? 3 : 2, sq = 0, sr = divmod ? 1 : 0;
   bool qin = q && (q == a || q == b), min_ = m && (m == a || m == b);
   size_t qbytes = qin ? out_bytes(q) : 0, mbytes = min_ ? out_bytes(m) : 0;
+  // a limit is held against the sizes alone, whichever kernel takes the call
   size_t ws = divmod_scratch_words(b->nlimbs, count) * sizeof(uint32_t);
-  xmpError_t e = set_necessary_scratch(h, qbytes + mbytes + ws);
+  xmpError_t e = check_scratch_limit(h, qbytes + mbytes + ws);
+  if (e != xmpErrorSuccess) return e;
+  if (!divmod_uses_scratch(a->nlimbs, b->nlimbs, count)) ws = 0;
+  e = set_necessary_scratch(h, qbytes + mbytes + ws);
   if (e != xmpErrorSuccess) return e;
   uint8_t *scr = (uint8_t *)h->scratch;
   uint32_t *qbuf = q ? (qin ? (uint32_t *)scr : q->limbs) : nullptr;
@@ -284,22 +288,24 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   const uint32_t nmod = p->indices[3] ? mod->count : std::min(count, mod->count);
   const uint32_t mstride = round_up(nmod, kStrideAlign);
   const size_t r2_words = (size_t)mod->nlimbs * mstride;
-  const size_t div_words = mod->nlimbs > kMaxRegDivisorLimbs ? divmod_scratch_words(mod->nlimbs, nmod) : 0;
+  size_t div_words = mod->nlimbs > kMaxRegDivisorLimbs ? divmod_scratch_words(mod->nlimbs, nmod) : 0;
   // the memory tier's R^2 squarings need a block per modulus of their own
   const size_t r2blk_words = wide ? powm_wide_r2_scratch_words(wide, nmod) : 0;
   const size_t obuf_words = ws ? round_up((uint32_t)(obytes / sizeof(uint32_t)), 64) : 0;
   const size_t limit = ws ? ws->bytes : (p->scratch_size_limit ? p->scratch_size_limit : handle->memorySize / 4 * 3);
-  const size_t fixed = (r2_words + div_words + r2blk_words + obuf_words) * sizeof(uint32_t);
   uint32_t wbits = c.window_bits;
   uint32_t chunk = count;
   if (!wide && !c.decided && any && powm_mx_pays(out->precision, exp->precision, count)) {
     mx = powm_mx_blocks(out->precision);
     const uint32_t mx_bits = best_window_bits(exp->precision);
-    if (mx && fixed + table_words(count, mx_bits) * sizeof(uint32_t) <= limit)
+    if (mx && (r2_words + obuf_words + table_words(count, mx_bits)) * sizeof(uint32_t) <= limit) {
       wbits = mx_bits;
-    else
+      div_words = 0;   // its R^2 is a division in LDS
+    } else {
       mx = 0;
+    }
   }
+  const size_t fixed = (r2_words + div_words + r2blk_words + obuf_words) * sizeof(uint32_t);
   while (fixed + table_words(chunk, wbits) * sizeof(uint32_t) > limit) {
     // (a workgroup-layout instance can need megabytes: its chunks may shrink further)
     if (!ws && chunk > (wide ? kStrideAlign : 65536u)) {

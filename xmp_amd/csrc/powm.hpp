@@ -12,12 +12,17 @@ namespace xmp {
 
 constexpr uint32_t kMaxRegDivisorLimbs = 128;
 
-// division workspace (words) for divisors beyond the register kernels
+// division workspace (words) for divisors beyond the register kernels, and
+// whether the kernel that a division takes uses it (all but the longest keep
+// their operands in LDS)
 size_t divmod_scratch_words(uint32_t b_len, uint32_t count);
+bool divmod_uses_scratch(uint32_t a_len, uint32_t b_len, uint32_t count);
 hipError_t launch_divmod_ws(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, uint32_t *scratch,
                             hipStream_t stream);
-// the same two by signed radix-2^28 digits (k_div_lazy.hip), for the sizes and
-// batches where that is faster; false, and nothing launched, for the others
+// launch_divmod_ws and launch_pow2_mod by signed digits of 26 to 28 bits
+// (k_div_lazy.hip), for the sizes and batches where that is faster; false, and
+// nothing launched, for the others
+bool divmod_lazy_takes(uint32_t a_len, uint32_t b_len, uint32_t count);
 bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
                         hipError_t *st);
 bool launch_pow2_mod_lazy(uint32_t *out, uint32_t out_len, uint32_t out_stride, const uint32_t *m, uint32_t m_len,
