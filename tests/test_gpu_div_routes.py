@@ -1,0 +1,82 @@
+"""GPU: divisions on both sides of the rules that choose between the signed-digit
+kernels and the 32-bit ones (register, lane-pair and wave kernels), against
+GMP's fdiv_qr: quotients of a few limbs, and dividends shorter than the divisor.
+
+Dividends and divisors repeat with coprime periods, so that a large batch has
+1,517 different divisions, each at several places of it; among the rows division
+by zero and by 1, unnormalised divisors, all-ones operands and quotients whose
+digits are all ones."""
+import numpy as np
+import pytest
+
+from helpers import O, gmp, inputs
+
+pytestmark = pytest.mark.gpu
+
+NA, NB = 37, 41
+
+
+def _operands(seed, la, lb):
+    a, b = inputs.uniform(seed, NA, la), inputs.uniform(seed + 1, NB, lb)
+    ones = np.uint32(0xFFFFFFFF)
+    b[:, -1] |= np.uint32(1)                # (a longer divisor than that is the rule)
+    b[0] = 0
+    b[1], b[1, 0] = 0, 1
+    b[2] = ones
+    b[3], b[3, -1] = 0, 0x80000000
+    b[4, -1] = 0                            # a leading zero limb
+    b[5, lb // 2:] = 0
+    b[5, 0] |= np.uint32(1)
+    b[6], b[6, -1] = 0x80000000, 0x7FFFFFFF
+    a[0] = 0
+    a[1] = ones
+    a[2], a[2, 0] = 0, 5
+    a[3], a[3, -1] = 0, 0x80000000
+    if la >= lb:                            # q d - 1 and q d: the remainder at its ends
+        d = O.to_int(b[7])
+        q = (1 << 32 * (la - lb)) - 1 if la > lb else 1
+        a[4], a[5] = O.from_int(q * d - 1, la), O.from_int(q * d, la)
+        a[6, -1] = min(int(b[8, -1]), int(a[6, -1]))
+    return a, b
+
+
+def _assert_periodic(got, want, what):
+    n, p = got.shape[0], want.shape[0]
+    for k in range(0, n, p):
+        part = got[k:k + p]
+        bad = np.nonzero((part != want[:part.shape[0]]).any(axis=1))[0]
+        assert bad.size == 0, "%s: rows %s from %d on differ" % (what, bad[:5], k)
+
+
+@pytest.mark.parametrize("lb,more,n", [
+    # quotients up to the rule's lengths and one limb past them
+    (9, 0, 300), (15, 2, 16384), (15, 3, 300), (16, 4, 1000), (16, 5, 16384), (16, 6, 64),
+    (16, -5, 300), (20, 1, 20000), (17, 4, 32768), (25, 4, 20000), (29, 5, 32768),
+    (30, 2, 4097), (31, 3, 16384), (32, 7, 30000), (32, 8, 30000), (25, 2, 32769), (32, 4, 98304), (32, 5, 65536),
+    (32, 10, 131073), (32, 11, 262144), (60, 6, 20000), (64, 0, 16385), (64, 7, 24576), (56, 8, 65537), (64, 9, 98304),
+    (72, 3, 65536), (96, 5, 49152), (96, 6, 65536), (96, 4, 131072), (96, 12, 262144),
+    (129, 4, 600), (129, 5, 16), (129, -40, 64), (130, 9, 600), (195, 10, 64), (160, 5, 2000), (160, 4, 4000),
+    (196, 6, 512), (256, 7, 16), (256, 1, 1500), (384, 1, 600), (896, 1, 4096), (1040, 5, 3000), (1040, -9, 3000),
+])
+def test_division_routes(handle, lb, more, n):
+    la = lb + more
+    a, b = _operands(9000 + lb + more, la, lb)
+    rows = np.arange(min(n, NA * NB))
+    x, y = a[rows % NA], b[rows % NB]
+    zero = ~y.any(axis=1)
+    wq, wr = gmp(O.GO_DIV, rows.size, la, x, np.where(zero[:, None], np.uint32(1), y), out2_limbs=lb)
+    wq[zero] = 0
+    wr[zero] = np.pad(x, ((0, 0), (0, max(0, -more))))[zero][:, :lb]
+    A, B, Q, R = handle.from_array(a), handle.from_array(b), handle.integers(32 * la, n), handle.integers(32 * lb, n)
+    what = "%d / %d limbs x %d" % (la, lb, n)
+    handle.divmod(Q, R, A, B, n)
+    _assert_periodic(Q.get(), wq, what + " q")
+    _assert_periodic(R.get(), wr, what + " r")
+    R.load(np.zeros((1, lb), np.uint32))
+    handle.mod(R, A, B, n)
+    _assert_periodic(R.get(), wr, what + " mod")
+    Q.load(np.zeros((1, la), np.uint32))
+    handle.div(Q, A, B, n)
+    _assert_periodic(Q.get(), wq, what + " div")
+    for z in (A, B, Q, R):
+        z.close()

@@ -459,6 +459,43 @@ const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count) {
   return nullptr;
 }
 
+// Divisions that the 32-bit kernels (registers up to 128 limbs, a wave each up
+// to 1,040) do as fast or faster though the digits above hold them.
+//
+// Short quotients: a signed-digit division first finds the divisor's length and
+// stages the dividend, and carries both results at its end, which takes as long
+// as a few of the 32-bit kernels' limbs.  Up to so many limbs of quotient
+// (dividend's limbs less divisor's) without and with the quotient stored; the
+// ranges are where those kernels' registers are just filled, or where a batch
+// just opens another round of this one's waves.  Measured, signed digits and
+// 32-bit kernels, us: 512/512 bits x 1,000 6.0 and 4.5, 1024/1024 x 8,192 7.1
+// and 6.4, x 65,536 10.9 and 9.2, 3072/3072 x 65,536 22.1 and 18.9, 6144/6144 x
+// 16 12.5 and 5.2, x 1,000 13.3 and 8.3.
+struct ShortRule {
+  uint32_t from, to;           // divisor's limbs
+  uint32_t count_from, count_to;
+  int32_t quotient, stored;    // limbs
+};
+const ShortRule kShort[] = {
+    {9, 15, 1, 16384, 0, 2},         {16, 16, 1, 16384, 4, 5},
+    {30, 32, 4097, 16384, 1, 2},     {17, 24, 16385, 32768, 1, 3},   {25, 29, 16385, 32768, 2, 4},
+    {30, 32, 16385, 32768, 4, 7},    {25, 32, 32769, 98304, 2, 4},   {32, 32, 131073, 280000, 4, 10},
+    {60, 64, 16385, 24576, -1, 6},   {56, 64, 65537, 98304, 4, 8},
+    {72, 87, 57344, 65536, 3, 3},    {88, 96, 49152, 65536, 3, 5},   {96, 96, 131072, 135168, 4, 4},
+    {96, 96, 262144, kAny, 7, 12},   {129, 129, 1, 600, 3, 4},       {130, 195, 1, 600, 8, 9},
+    {130, 195, 601, 2000, 4, 5},     {130, 195, 2001, 4000, 2, 4},   {196, 256, 1, 512, 4, 6},
+    {196, 256, 513, 1500, 1, 1},     {257, 384, 1, 600, 0, 1},       {896, 1016, 4096, 24576, 1, 1},
+    {1017, 1040, 3000, 24576, 5, 4},
+};
+bool register_division_pays(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient) {
+  const int32_t more = a_len > b_len ? (int32_t)(a_len - b_len) : 0;
+  for (const ShortRule &r : kShort)
+    if (b_len >= r.from && b_len <= r.to && count >= r.count_from && count <= r.count_to &&
+        more <= (quotient ? r.stored : r.quotient))
+      return true;
+  return false;
+}
+
 }  // namespace
 
 bool divmod_lazy_takes(uint32_t a_len, uint32_t b_len, uint32_t count) {
@@ -468,7 +505,7 @@ bool divmod_lazy_takes(uint32_t a_len, uint32_t b_len, uint32_t count) {
 bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
                         hipError_t *st) {
   const LazyEntry *e = lazy_entry(a.len, b.len, count);
-  if (!e) return false;
+  if (!e || register_division_pays(a.len, b.len, count, q.data != nullptr)) return false;
   const uint32_t per = 64 / e->lanes;
   hipLaunchKernelGGL(e->div, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a.len, e->lanes * e->digits, e->radix),
                      stream, q, r, a, b, count);
