@@ -1,6 +1,7 @@
 """GPU: divisions on both sides of the rules that choose between the signed-digit
 kernels and the 32-bit ones (register, lane-pair and wave kernels), against
-GMP's fdiv_qr: quotients of a few limbs, and dividends shorter than the divisor.
+GMP's fdiv_qr: quotients of a few limbs, dividends shorter than the divisor, and
+dividends several times the divisor in full batches.
 
 Dividends and divisors repeat with coprime periods, so that a large batch has
 1,517 different divisions, each at several places of it; among the rows division
@@ -57,6 +58,10 @@ def _assert_periodic(got, want, what):
     (72, 3, 65536), (96, 5, 49152), (96, 6, 65536), (96, 4, 131072), (96, 12, 262144),
     (129, 4, 600), (129, 5, 16), (129, -40, 64), (130, 9, 600), (195, 10, 64), (160, 5, 2000), (160, 4, 4000),
     (196, 6, 512), (256, 7, 16), (256, 1, 1500), (384, 1, 600), (896, 1, 4096), (1040, 5, 3000), (1040, -9, 3000),
+    # rows that take more lanes than the batch's rule gives
+    (20, 120, 65536), (24, 150, 65536), (32, 128, 65536), (32, 200, 65536), (64, 390, 65536),
+    # ... and that go to the register kernels
+    (24, 150, 131072), (32, 96, 131072), (40, 240, 131072), (52, 340, 131072), (64, 260, 131072),
 ])
 def test_division_routes(handle, lb, more, n):
     la = lb + more

@@ -440,22 +440,46 @@ const LazyRule kRules[] = {
     {520, 2048, 64, 10, 26}, {520, kAny, 16, 40, 26},
     {1040, kAny, 64, 20, 26},
 };
-constexpr size_t kLazyLds = 64 * 1024;
+constexpr size_t kLazyLds = 64 * 1024, kCuLds = 160 * 1024;
+constexpr uint32_t kCuInstances = 256 * 64;   // instances of one lane that are a wave a CU
 
-const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count) {
-  if (b_len <= 8) return nullptr;
-  uint32_t limbs = 0;   // the smallest that holds the divisor
-  for (const LazyRule &r : kRules)
-    if (b_len <= r.limbs && !limbs) limbs = r.limbs;
-  if (limbs == 0 || (limbs == 16 && count > 16384)) return nullptr;
-  // the batch's rule; a dividend too long for its rows in LDS takes the first
-  // of the divisor's rules whose lanes are more and rows fewer
-  for (int any = 0; any < 2; any++)
-    for (const LazyRule &r : kRules)
-      if (r.limbs == limbs && (any || count <= r.count) &&
-          4 * (size_t)(64 / r.lanes) * lazy_row(a_len, r.lanes * r.digits, r.radix) <= kLazyLds)
-        for (const LazyEntry &e : kLazy)
-          if (e.lanes == r.lanes && e.digits == r.digits && e.radix == r.radix) return &e;
+size_t lazy_lds(const LazyRule &r, uint32_t a_len) {
+  return 4 * (size_t)(64 / r.lanes) * lazy_row(a_len, r.lanes * r.digits, r.radix);
+}
+
+// The rule for a division, or null for the 32-bit kernels.  Long dividends'
+// rows in LDS leave a CU few waves: where those are fewer than the batch has
+// for it (four are enough), a rule of more lanes, whose rows are fewer, is as
+// fast or faster for the quotient's sake, and with no quotient stored where
+// rows leave two.  Measured, with the quotient, against the batch's own rule:
+// 5120/1024 bits x 65,536 76 and 105 us, 4480/640 72 and 86.  A dividend too long
+// for its rows takes the first of the divisor's rules that holds it.
+const LazyRule *lazy_rule(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient) {
+  const LazyRule *first = nullptr, *own = nullptr, *end = kRules;
+  for (const LazyRule &r : kRules) {
+    if (b_len > r.limbs || (first && r.limbs != first->limbs)) continue;
+    if (!first) first = &r;
+    if (!own && count <= r.count) own = &r;
+    end = &r + 1;
+  }
+  if (b_len <= 8 || !own) return nullptr;
+  const size_t residents = kCuLds / lazy_lds(*own, a_len);
+  if (count > 32768 && b_len <= 64 && (quotient || (b_len > 24 && residents <= 2))) {
+    auto crowded = [&](const LazyRule &r) {
+      const uint64_t waves = ((uint64_t)count * r.lanes + kCuInstances - 1) / kCuInstances;
+      return kCuLds / lazy_lds(r, a_len) < std::min<uint64_t>(4, waves);
+    };
+    while (own != first && crowded(*own)) own--;
+  }
+  if (lazy_lds(*own, a_len) > kLazyLds)
+    for (own = first; own != end && lazy_lds(*own, a_len) > kLazyLds;) own++;
+  return own != end ? own : nullptr;
+}
+
+const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient) {
+  if (const LazyRule *r = lazy_rule(a_len, b_len, count, quotient))
+    for (const LazyEntry &e : kLazy)
+      if (e.lanes == r->lanes && e.digits == r->digits && e.radix == r->radix) return &e;
   return nullptr;
 }
 
@@ -487,24 +511,33 @@ const ShortRule kShort[] = {
     {196, 256, 513, 1500, 1, 1},     {257, 384, 1, 600, 0, 1},       {896, 1016, 4096, 24576, 1, 1},
     {1017, 1040, 3000, 24576, 5, 4},
 };
+// Long quotients of full batches: rows that leave a CU so few waves that the
+// 32-bit kernels, which keep nothing in LDS, are ahead.  Measured, us: 5120/1024
+// bits x 262,144 208 and 158 (with the quotient stored 313 and 182), 10752/1536
+// x 131,072 349 and 258, 3072/1024 x 262,144 with the quotient 122 and 95.
 bool register_division_pays(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient) {
   const int32_t more = a_len > b_len ? (int32_t)(a_len - b_len) : 0;
   for (const ShortRule &r : kShort)
     if (b_len >= r.from && b_len <= r.to && count >= r.count_from && count <= r.count_to &&
         more <= (quotient ? r.stored : r.quotient))
       return true;
-  return false;
+  if (count < 131072 || b_len <= 16 || b_len > 64) return false;
+  const LazyRule *r = kRules;
+  while (b_len > r->limbs || count > r->count) r++;   // the batch's own rule
+  const size_t residents = kCuLds / lazy_lds(*r, a_len);
+  const bool loose = b_len <= 24 || (b_len > 48 && b_len <= 56);   // registers of the 32-bit kernels half filled
+  return residents <= (!quotient ? (loose ? 2u : 3u) : loose ? 3u : b_len <= 32 ? 5u : 4u);
 }
 
 }  // namespace
 
 bool divmod_lazy_takes(uint32_t a_len, uint32_t b_len, uint32_t count) {
-  return lazy_entry(a_len, b_len, count) != nullptr;
+  return lazy_entry(a_len, b_len, count, true) != nullptr;
 }
 
 bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
                         hipError_t *st) {
-  const LazyEntry *e = lazy_entry(a.len, b.len, count);
+  const LazyEntry *e = lazy_entry(a.len, b.len, count, q.data != nullptr);
   if (!e || register_division_pays(a.len, b.len, count, q.data != nullptr)) return false;
   const uint32_t per = 64 / e->lanes;
   hipLaunchKernelGGL(e->div, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a.len, e->lanes * e->digits, e->radix),
@@ -516,7 +549,7 @@ bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32
 bool launch_pow2_mod_lazy(uint32_t *out, uint32_t out_len, uint32_t out_stride, const uint32_t *m, uint32_t m_len,
                           uint32_t m_stride, uint32_t count, uint32_t exponent, hipStream_t stream, hipError_t *st) {
   const uint32_t a_len = (exponent >> 5) + 1;
-  const LazyEntry *e = lazy_entry(a_len, m_len, count);
+  const LazyEntry *e = lazy_entry(a_len, m_len, count, false);
   if (!e) return false;
   const uint32_t per = 64 / e->lanes;
   hipLaunchKernelGGL(e->pow2, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a_len, e->lanes * e->digits, e->radix),
