@@ -275,6 +275,11 @@ __global__ void set_kernel(uint32_t *__restrict__ out, uint32_t out_stride, uint
 
 }  // namespace
 
+bool transfer_in_words(uint32_t words, int32_t order, int32_t endian, uint32_t nails, uint32_t size, uint32_t nlimbs) {
+  bool rev, swap;
+  return as_words(words, order, endian, nails, size, nlimbs, &rev, &swap);
+}
+
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream) {
   const uint32_t words = (uint32_t)(bytes / 4);
   hipLaunchKernelGGL(copy_kernel, dim3(div_round_up(words, 1024)), dim3(256), 0, stream,
