@@ -193,20 +193,24 @@ def test_short_transfers_take_no_scratch(recording):
     x.close()
 
 
+@pytest.mark.parametrize("n,scratch_in,scratch_out", [(100, False, False), (103, False, True), (513, True, True)])
 @pytest.mark.parametrize("fmt", [(-1, 2, 1), (1, 2, -1), (-1, 8, 1), (1, 8, -1)])   # (order, size, endian)
-def test_formats_of_no_whole_words_stay_on_the_device(recording, fmt):
+def test_formats_of_no_whole_words(recording, fmt, n, scratch_in, scratch_out):
     """Formats that the kernels handle a short word or a byte at a time are
-    transposed in scratch, not across the bus."""
-    h, n, limbs, (order, size, endian) = recording, 60, 20, fmt
+    transposed in device scratch, not across the bus, above 40 KiB in and 8 KiB
+    out (24 as 64-bit words)."""
+    scratch_out = scratch_out and (fmt[1] != 8 or n > 300)
+    h, limbs, (order, size, endian) = recording, 20, fmt
     a = inputs.uniform(8700, n, limbs)
     words = a.astype("<u4").view("<u%d" % size).reshape(n, -1)
     host = np.ascontiguousarray(words[:, ::-order].astype((">" if endian == 1 else "<") + "u%d" % size))
     L, x = xmp_amd.lib(), h.integers(32 * limbs, n)
     h.sizes.clear()
     assert L.xmpIntegersImport(h.h, x.x, words.shape[1], order, size, endian, 0, host.ctypes.data, n) == 0
-    assert h.sizes == [4 * n * limbs]
+    assert h.sizes == ([4 * n * limbs] if scratch_in else [])
     assert np.array_equal(x.get(), a)
     back, got = np.zeros_like(host), ctypes.c_uint32()
     assert L.xmpIntegersExport(h.h, back.ctypes.data, ctypes.byref(got), order, size, endian, 0, x.x, n) == 0
+    assert h.sizes == ([4 * n * limbs] if scratch_in or scratch_out else [])
     assert got.value == words.shape[1] and back.tobytes() == host.tobytes()
     x.close()

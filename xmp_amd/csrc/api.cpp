@@ -75,9 +75,12 @@ bool is_device_pointer(const void *p) {
 // 25-37 us for 2-256 KiB, 270 for 4 MiB and 1190 for 16; through pinned slots,
 // which a kernel writes and a memcpy empties beside the next chunk's, 16-28,
 // 155 and 590 (one core's memcpy).  A transposing kernel has its compact side in
-// a slot only for whole-word formats: as 16-bit words in mixed order 8192 bits x
-// 100 took 68 us out and 33 in that way, 22 (copied to the slots from scratch)
-// and 24.  Chunks are half slots up to 1 MiB, so that
+// a slot (one slot at most) where that is faster than in device scratch: whole
+// words, and other formats, which cross the bus a short word or a byte at a
+// time, up to 40 KiB in (any call's size up to 16 limbs) and 8 KiB out (24 as
+// 64-bit words).  16-bit words in mixed order, out: 1088 bits x 50 17.1 us, from
+// scratch 18.2; x 100 20.8, 18.5; 8192 x 100 68, 22; in: 1088 x 300 18.1, 23.1;
+// 256 x 3,000 18.8, 24.3; 8192 x 100 33, 24.  Chunks are half slots up to 1 MiB, so that
 // there are enough of them to overlap.  From pageable memory its path is as
 // fast as a slot (4 MiB 155 against 170), but for the copy that a short import
 // does not need.
@@ -409,8 +412,9 @@ static xmpError_t import_internal(xmpHandle_t handle, xmpIntegers_t out, uint32_
     // (the limit is held against the sizes alone, whichever way the words take)
     xmpError_t e = check_scratch_limit(handle, bytes);
     if (e != xmpErrorSuccess) return e;
-    if (!async && !idx && bytes <= HostStage::kDirect &&
-        transfer_in_words(words, order, endian, nails, (uint32_t)size, out->nlimbs) && staged(handle, in)) {
+    const bool whole = transfer_in_words(words, order, endian, nails, (uint32_t)size, out->nlimbs);
+    const size_t most = whole || out->nlimbs <= 16 ? HostStage::kDirect : HostStage::kOtherIn;
+    if (!async && !idx && bytes <= most && staged(handle, in)) {
       std::memcpy(handle->stage.slot(0), in, bytes);
       src = handle->stage.slot(0);
     } else {
@@ -469,8 +473,9 @@ static xmpError_t export_internal(xmpHandle_t handle, void *out, uint32_t *words
   if (host) {
     xmpError_t e = check_scratch_limit(handle, bytes);   // (as for an import)
     if (e != xmpErrorSuccess) return e;
-    direct = !async && !idx && bytes <= HostStage::kDirect &&
-             transfer_in_words(w, order, endian, nails, (uint32_t)size, in->nlimbs) && staged(handle, out);
+    const bool whole = transfer_in_words(w, order, endian, nails, (uint32_t)size, in->nlimbs);
+    const size_t most = whole ? HostStage::kDirect : size == 8 ? 3 * HostStage::kOtherOut : HostStage::kOtherOut;
+    direct = !async && !idx && bytes <= most && staged(handle, out);
     if (direct) {
       dst = handle->stage.slot(0);
     } else {

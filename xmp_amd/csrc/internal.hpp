@@ -58,7 +58,8 @@ namespace xmp {
 struct HostStage {
   static constexpr size_t kSlot = 512u << 10;
   static constexpr int kSlots = 4;
-  static constexpr size_t kDirect = 256u << 10;   // up to here a kernel reads or writes one slot itself
+  static constexpr size_t kDirect = 256u << 10;   // up to here a kernel reads or writes one slot itself,
+  static constexpr size_t kOtherIn = 40u << 10, kOtherOut = 8u << 10;   // ... of a format of no whole words
   uint8_t *buf = nullptr;
   hipEvent_t done[kSlots] = {};                    // the slot's last copy
 

@@ -13,9 +13,8 @@
 
 namespace xmp {
 
-// Whether a format moves as whole 32-bit words (k_xfer.hip): only then may a
-// kernel have its compact side in host memory, which the others would cross
-// the bus to a byte or a short word at a time.
+// whether a format moves as whole 32-bit words (k_xfer.hip); a kernel takes the
+// others a byte or a short word at a time
 bool transfer_in_words(uint32_t words, int32_t order, int32_t endian, uint32_t nails, uint32_t size, uint32_t nlimbs);
 // whole words between device and pinned host memory, both 16-byte aligned
 hipError_t launch_copy(void *dst, const void *src, size_t bytes, hipStream_t stream);
