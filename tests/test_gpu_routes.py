@@ -214,3 +214,17 @@ def test_formats_of_no_whole_words(recording, fmt, n, scratch_in, scratch_out):
     assert h.sizes == ([4 * n * limbs] if scratch_in or scratch_out else [])
     assert got.value == words.shape[1] and back.tobytes() == host.tobytes()
     x.close()
+
+
+@pytest.mark.parametrize("limbs,n,uses", [(9, 56, False), (9, 60, True), (33, 124, True), (33, 125, False), (7, 300, False),
+                                          (36, 100, False), (65, 32, False), (65, 33, True)])
+def test_short_imports_of_odd_lengths(recording, limbs, n, uses):
+    """Tiles of 2 to 16 KiB, but for a few rows, are read from device scratch,
+    not across the bus."""
+    a = inputs.uniform(8800 + limbs, n, limbs)
+    x = recording.integers(32 * limbs, n)
+    recording.sizes.clear()
+    x.load(a)
+    assert recording.sizes == ([4 * n * limbs] if uses else [])
+    assert np.array_equal(x.get(), a)
+    x.close()

@@ -414,7 +414,13 @@ static xmpError_t import_internal(xmpHandle_t handle, xmpIntegers_t out, uint32_
     if (e != xmpErrorSuccess) return e;
     const bool whole = transfer_in_words(words, order, endian, nails, (uint32_t)size, out->nlimbs);
     const size_t most = whole || out->nlimbs <= 16 ? HostStage::kDirect : HostStage::kOtherIn;
-    if (!async && !idx && bytes <= most && staged(handle, in)) {
+    // (more than eight limbs, no multiple of four, move through LDS tiles, and
+    // more than half a tile's reads over the bus take longer than the runtime's
+    // copy of up to 16 KiB: 33 limbs x 100 18.9 us, 17.4; x 200 19.3, 23.4; x 10
+    // 14.5, 16.9)
+    const bool tiles = whole && out->nlimbs % 4 != 0 && out->nlimbs > 8 && count > 32 && bytes > (2u << 10) &&
+                       bytes <= (16u << 10);
+    if (!async && !idx && bytes <= most && !tiles && staged(handle, in)) {
       std::memcpy(handle->stage.slot(0), in, bytes);
       src = handle->stage.slot(0);
     } else {
