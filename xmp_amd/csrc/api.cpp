@@ -80,10 +80,10 @@ bool is_device_pointer(const void *p) {
 // time, up to 40 KiB in (any call's size up to 16 limbs) and 8 KiB out (24 as
 // 64-bit words).  16-bit words in mixed order, out: 1088 bits x 50 17.1 us, from
 // scratch 18.2; x 100 20.8, 18.5; 8192 x 100 68, 22; in: 1088 x 300 18.1, 23.1;
-// 256 x 3,000 18.8, 24.3; 8192 x 100 33, 24.  Chunks are half slots up to 1 MiB, so that
-// there are enough of them to overlap.  From pageable memory its path is as
-// fast as a slot (4 MiB 155 against 170), but for the copy that a short import
-// does not need.
+// 256 x 3,000 18.8, 24.3; 8192 x 100 33, 24.  Chunks are half slots up to 1 MiB,
+// so that there are enough of them to overlap.  From pageable memory its path is
+// as fast as a slot (4 MiB 155 against 170), but for the copy that a short
+// import does not need.
 static bool pageable(const void *p) {
   hipPointerAttribute_t attr;
   if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
@@ -102,19 +102,24 @@ static void free_stage(HostStage &st) {
   st.buf = nullptr;
 }
 
-// A stream that is being captured keeps the runtime's path, and so does
-// everything if no memory can be pinned.
+// A stream that is being captured, or that cannot be asked, keeps the runtime's
+// path, and so does everything once no memory could be pinned.
 bool staged(xmpHandle_t h, const void *host) {
-  hipStreamCaptureStatus capture;
-  if (!pageable(host) || hipStreamIsCapturing(h->stream, &capture) != hipSuccess ||
-      capture != hipStreamCaptureStatusNone)
-    return false;
   HostStage &st = h->stage;
+  if (st.none || !pageable(host)) return false;
+  hipStreamCaptureStatus capture;
+  if (hipStreamIsCapturing(h->stream, &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (capture != hipStreamCaptureStatusNone) return false;
   if (st.buf) return true;
-  bool ok = hipHostMalloc((void **)&st.buf, HostStage::kSlot * HostStage::kSlots,
-                          hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess;
+  const hipError_t e = hipHostMalloc((void **)&st.buf, HostStage::kSlot * HostStage::kSlots,
+                                     hipHostMallocMapped | hipHostMallocCoherent);
+  st.none = e == hipErrorOutOfMemory;   // (another thread's capture refuses it too, for a while)
+  bool ok = e == hipSuccess;
   if (!ok) st.buf = nullptr;
-  for (hipEvent_t &e : st.done) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+  for (hipEvent_t &ev : st.done) ok = ok && hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess;
   if (!ok) {
     free_stage(st);
     (void)hipGetLastError();

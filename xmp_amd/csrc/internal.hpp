@@ -61,6 +61,7 @@ struct HostStage {
   static constexpr size_t kDirect = 256u << 10;   // up to here a kernel reads or writes one slot itself,
   static constexpr size_t kOtherIn = 40u << 10, kOtherOut = 8u << 10;   // ... of a format of no whole words
   uint8_t *buf = nullptr;
+  bool none = false;                               // no memory could be pinned: not asked for again
   hipEvent_t done[kSlots] = {};                    // the slot's last copy
 
   uint8_t *slot(size_t k) const { return buf + k % kSlots * kSlot; }
