@@ -228,3 +228,23 @@ def test_short_imports_of_odd_lengths(recording, limbs, n, uses):
     assert recording.sizes == ([4 * n * limbs] if uses else [])
     assert np.array_equal(x.get(), a)
     x.close()
+
+
+def test_more_products_than_a_grid_of_waves_holds(fresh_handle):
+    """2^26 and some squares of 129 limbs, truncated and of repeated operands: a
+    wave each would be 2^32 threads."""
+    h, limbs, n = fresh_handle, 129, (1 << 26) + 100
+    a = inputs.uniform(8900, 3, limbs)
+    want = gmp(O.GO_MUL, 3, limbs, a, a)
+    A, P = h.from_array(a), h.integers(32 * limbs, n)
+    h.mul(P, A, A, n)
+    rows = np.array([0, 1, 2, 63, 64, 65535, n // 2, n - 65, n - 64, n - 2, n - 1], np.uint32)
+    out = h.integers(32 * limbs, rows.size)
+    h.set_indices(1, rows)
+    try:
+        assert xmp_amd.lib().xmpIntegersSet(h.h, out.x, P.x, rows.size) == 0
+    finally:
+        h.clear_indices()
+    assert_rows_equal(out.get(), want[rows % 3], "repeated squares")
+    for x in (A, P, out):
+        x.close()

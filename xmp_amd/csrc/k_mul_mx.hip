@@ -357,6 +357,8 @@ bool mul_mx_holds(uint32_t a_len, uint32_t b_len) {
 bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t count) {
   if (!mul_mx_holds(a_len, b_len)) return false;
   if (a_len > 512) return true;
+  // (a grid has fewer than 2^32 threads; the lane kernels take 8 or 16 a product)
+  if ((uint64_t)count * (a_len + b_len > 512 ? 128 : 64) >> 32) return false;
   if (2 * b_len < a_len || a_len <= 16) return false;
   if (a_len <= 32) return count <= 2048;
   if (a_len <= 64) return count <= 4096;

@@ -810,7 +810,7 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 //   1536 x 14,336 0.281, 0.300; 2048 x 16,384 0.363, 0.383, x 24,576 0.52,
 //   0.64; 3072 x 65,536 2.42, 2.52; 4096 x 65,536 3.3, 4.2.
 bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
-  if (precision <= 128) return false;
+  if (precision <= 128 || count >> 26) return false;   // (a wave an instance: a grid has fewer than 2^32 threads)
   if (precision <= 256) return count <= 1024;
   if (precision <= 480) return count <= 3072;
   if (precision <= 512) return count <= 8192;
