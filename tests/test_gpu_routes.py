@@ -248,3 +248,29 @@ def test_more_products_than_a_grid_of_waves_holds(fresh_handle):
     assert_rows_equal(out.get(), want[rows % 3], "repeated squares")
     for x in (A, P, out):
         x.close()
+
+
+def _sample(h, x, rows):
+    """Some instances of a batch too long to export."""
+    out = h.integers(x.precision, rows.size)
+    h.set_indices(1, rows)
+    try:
+        assert xmp_amd.lib().xmpIntegersSet(h.h, out.x, x.x, rows.size) == 0
+    finally:
+        h.clear_indices()
+    got = out.get()
+    out.close()
+    return got
+
+
+def test_more_long_products_than_a_grid_of_workgroups_holds(fresh_handle):
+    """2^25 and some products of 513 limbs by one, truncated and of repeated
+    operands: two waves each would be 2^32 threads."""
+    h, limbs, n = fresh_handle, 513, (1 << 25) + 100
+    a, b = inputs.uniform(8950, 3, limbs), inputs.uniform(8951, 1, 1)
+    A, B, P = h.from_array(a), h.from_array(b), h.integers(32 * limbs, n)
+    h.mul(P, A, B, n)
+    rows = np.array([0, 1, 2, 63, 64, 65535, n // 2, n - 101, n - 65, n - 64, n - 2, n - 1], np.uint32)
+    assert_rows_equal(_sample(h, P, rows), gmp(O.GO_MUL, 3, limbs, a, np.repeat(b, 3, axis=0))[rows % 3], "products")
+    for x in (A, B, P):
+        x.close()

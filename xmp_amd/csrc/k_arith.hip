@@ -916,29 +916,31 @@ __global__ void __launch_bounds__(64) kar_carry_kernel(OutOperand p, uint32_t co
 
 // workspace limbs per instance column for a product of a_len x b_len limbs
 // (a_len >= b_len): this level's terms, then the largest child's
-size_t kar_limbs(uint32_t a_len, uint32_t b_len) {
-  if (a_len < kKaratsubaMinLimbs || mul_mx_holds(a_len, b_len)) return 0;
+size_t kar_limbs(uint32_t a_len, uint32_t b_len, uint32_t count) {
+  if (a_len < kKaratsubaMinLimbs || mul_mx_holds(a_len, b_len, count)) return 0;
   const uint32_t h = (a_len + 1) / 2;
   const size_t rows = (a_len + b_len + kKarChunk - 1) / kKarChunk;   // chunk carries
   if (b_len <= h) {
     const size_t own = rows + (size_t)(h + b_len) + (a_len - h + b_len);
-    return own + std::max(kar_limbs(h, b_len), kar_limbs(std::max(a_len - h, b_len), std::min(a_len - h, b_len)));
+    return own + std::max(kar_limbs(h, b_len, count),
+                          kar_limbs(std::max(a_len - h, b_len), std::min(a_len - h, b_len), count));
   }
   const size_t own = rows + 2 * (size_t)(h + 1) + 2 * (size_t)h + 2 * (size_t)h + (a_len - h) + (b_len - h);
-  return own + std::max(kar_limbs(h, h), kar_limbs(a_len - h, b_len - h));
+  return own + std::max(kar_limbs(h, h, count), kar_limbs(a_len - h, b_len - h, count));
 }
 
 }  // namespace
 
 size_t mul_karatsuba_words(uint32_t a_len, uint32_t b_len, uint32_t count) {
-  return kar_limbs(std::max(a_len, b_len), std::min(a_len, b_len)) * round_up(count, kStrideAlign);
+  return kar_limbs(std::max(a_len, b_len), std::min(a_len, b_len), count) * round_up(count, kStrideAlign);
 }
 
 hipError_t launch_mul_ws(OutOperand p, Operand a, Operand b, uint32_t count, bool square, uint32_t *ws,
                          hipStream_t stream) {
   if (count == 0) return hipSuccess;
   if (a.len < b.len) std::swap(a, b);
-  if (a.len < kKaratsubaMinLimbs || mul_mx_holds(a.len, b.len)) return square ? launch_sqr(p, a, count, stream) : launch_mul(p, a, b, count, stream);
+  if (a.len < kKaratsubaMinLimbs || mul_mx_holds(a.len, b.len, count))
+    return square ? launch_sqr(p, a, count, stream) : launch_mul(p, a, b, count, stream);
   const uint32_t st = round_up(count, kStrideAlign);
   const uint32_t h = (a.len + 1) / 2;
   auto take = [&](uint32_t limbs) {

@@ -338,10 +338,11 @@ hipError_t launch(const OutOperand &p, const Operand &a, const Operand &b, uint3
 
 }  // namespace
 
-// a_len >= b_len: what a workgroup's threads and LDS hold (65,536 by 65,536 bits)
-bool mul_mx_holds(uint32_t a_len, uint32_t b_len) {
+// a_len >= b_len: what a workgroup's threads and LDS hold (65,536 by 65,536
+// bits), and no more products than a grid, which has fewer than 2^32 threads
+bool mul_mx_holds(uint32_t a_len, uint32_t b_len, uint32_t count) {
   const MulImage<4> im(a_len, b_len, a_len + b_len);
-  return im.tiles <= 64 && im.bytes <= kMaxLds;
+  return im.tiles <= 64 && im.bytes <= kMaxLds && (count + 1ull) * 64 * div_round_up(im.tiles, 8) >> 32 == 0;
 }
 
 // Where the matrix cores are faster than the lane kernels.  A product's wave
@@ -355,10 +356,8 @@ bool mul_mx_holds(uint32_t a_len, uint32_t b_len) {
 // A multiplier shorter than half leaves the lane kernels little to do: 8192 x
 // 1024 bits x 16,384 40, 29.
 bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t count) {
-  if (!mul_mx_holds(a_len, b_len)) return false;
+  if (!mul_mx_holds(a_len, b_len, count)) return false;
   if (a_len > 512) return true;
-  // (a grid has fewer than 2^32 threads; the lane kernels take 8 or 16 a product)
-  if ((uint64_t)count * (a_len + b_len > 512 ? 128 : 64) >> 32) return false;
   if (2 * b_len < a_len || a_len <= 16) return false;
   if (a_len <= 32) return count <= 2048;
   if (a_len <= 64) return count <= 4096;

@@ -47,7 +47,7 @@ hipError_t launch_mul(OutOperand p, Operand a, Operand b, uint32_t count, hipStr
 hipError_t launch_sqr(OutOperand p, Operand a, uint32_t count, hipStream_t stream);
 // Products on the matrix cores (k_mul_mx.hip); for a_len >= b_len, whether it
 // holds them, and whether a batch takes it
-bool mul_mx_holds(uint32_t a_len, uint32_t b_len);
+bool mul_mx_holds(uint32_t a_len, uint32_t b_len, uint32_t count);
 bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t count);
 hipError_t launch_mul_mx(OutOperand p, Operand a, Operand b, uint32_t count, bool square, hipStream_t stream);
 // Products whose longer operand has kKaratsubaMinLimbs limbs or more and that
