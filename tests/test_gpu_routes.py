@@ -274,3 +274,17 @@ def test_more_long_products_than_a_grid_of_workgroups_holds(fresh_handle):
     assert_rows_equal(_sample(h, P, rows), gmp(O.GO_MUL, 3, limbs, a, np.repeat(b, 3, axis=0))[rows % 3], "products")
     for x in (A, B, P):
         x.close()
+
+
+def test_more_divisions_than_a_grid_of_lane_groups_holds(fresh_handle):
+    """2^30 and some divisions by 67 limbs, of repeated operands: four lanes
+    each would be 2^32 threads."""
+    h, n = fresh_handle, (1 << 30) + 100
+    a, b = inputs.uniform(8960, 5, 1), np.zeros((1, 67), np.uint32)
+    b[0, 0] = 12345
+    A, B, Q = h.from_array(a), h.from_array(b), h.integers(32, n)
+    h.div(Q, A, B, n)
+    rows = np.array([0, 1, 2, 63, 64, 65535, n // 2, n - 101, n - 65, n - 64, n - 2, n - 1], np.uint32)
+    assert np.array_equal(_sample(h, Q, rows)[:, 0], (a[:, 0] // 12345)[rows % 5])
+    for x in (A, B, Q):
+        x.close()

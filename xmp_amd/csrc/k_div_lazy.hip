@@ -473,7 +473,8 @@ const LazyRule *lazy_rule(uint32_t a_len, uint32_t b_len, uint32_t count, bool q
   }
   if (lazy_lds(*own, a_len) > kLazyLds)
     for (own = first; own != end && lazy_lds(*own, a_len) > kLazyLds;) own++;
-  return own != end ? own : nullptr;
+  if (own == end || (count + 63ull) * own->lanes >> 32) return nullptr;   // (a grid has fewer than 2^32 threads)
+  return own;
 }
 
 const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient) {
