@@ -288,3 +288,16 @@ def test_more_divisions_than_a_grid_of_lane_groups_holds(fresh_handle):
     assert np.array_equal(_sample(h, Q, rows)[:, 0], (a[:, 0] // 12345)[rows % 5])
     for x in (A, B, Q):
         x.close()
+
+
+@pytest.mark.parametrize("bits", [1024, 2048, 6144])
+def test_a_limit_below_the_lanes_plan_refuses(recording, bits):
+    """One instance's table is short on the matrix cores; the limits that are
+    refused are those of a lane layout's, of 64 instances."""
+    h = recording
+    h.set_scratch_limit(_r2_bytes(bits, 1) + _mx_bytes(bits, 1, 3))
+    with pytest.raises(xmp_amd.XmpError) as err:
+        _powm(h, bits, 96, 1)
+    assert err.value.code == xmp_amd.INCREASE_SCRATCH_LIMIT
+    h.set_scratch_limit(0)
+    assert _powm(h, bits, 96, 1) == [_r2_bytes(bits, 1) + _mx_bytes(bits, 1, 3)]

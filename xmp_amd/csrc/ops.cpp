@@ -295,17 +295,7 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
   const size_t limit = ws ? ws->bytes : (p->scratch_size_limit ? p->scratch_size_limit : handle->memorySize / 4 * 3);
   uint32_t wbits = c.window_bits;
   uint32_t chunk = count;
-  if (!wide && !c.decided && any && powm_mx_pays(out->precision, exp->precision, count)) {
-    mx = powm_mx_blocks(out->precision);
-    const uint32_t mx_bits = best_window_bits(exp->precision);
-    if (mx && (r2_words + obuf_words + table_words(count, mx_bits)) * sizeof(uint32_t) <= limit) {
-      wbits = mx_bits;
-      div_words = 0;   // its R^2 is a division in LDS
-    } else {
-      mx = 0;
-    }
-  }
-  const size_t fixed = (r2_words + div_words + r2blk_words + obuf_words) * sizeof(uint32_t);
+  size_t fixed = (r2_words + div_words + r2blk_words + obuf_words) * sizeof(uint32_t);
   while (fixed + table_words(chunk, wbits) * sizeof(uint32_t) > limit) {
     // (a workgroup-layout instance can need megabytes: its chunks may shrink further)
     if (!ws && chunk > (wide ? kStrideAlign : 65536u)) {
@@ -318,6 +308,20 @@ xmpError_t powm_run(xmpHandle_t handle, xmpIntegers_t out, xmpIntegers_t a, xmpI
       wbits--;
     } else {
       return xmpErrorIncreaseScratchLimit;
+    }
+  }
+  // (a limit is held against the lanes' plan, whichever kernel takes the call)
+  if (!wide && !c.decided && any && powm_mx_pays(out->precision, exp->precision, count)) {
+    mx = powm_mx_blocks(out->precision);
+    const uint32_t mx_bits = best_window_bits(exp->precision);
+    const size_t mx_fixed = fixed - div_words * sizeof(uint32_t);   // (its R^2 is a division in LDS)
+    if (mx && mx_fixed + table_words(count, mx_bits) * sizeof(uint32_t) <= limit) {
+      wbits = mx_bits;
+      chunk = count;
+      div_words = 0;
+      fixed = mx_fixed;
+    } else {
+      mx = 0;
     }
   }
   const size_t need = fixed + table_words(chunk, wbits) * sizeof(uint32_t);
