@@ -879,10 +879,12 @@ hipError_t launch_divmod_ws(OutOperand q, OutOperand r, Operand a, Operand b, ui
   hipError_t st;
   if (launch_divmod_lazy(q, r, a, b, count, stream, &st)) return st;
   const uint32_t nb = b.len;
-  // What is left: divisors up to 512 bits or above 33,280, and dividends too
-  // long for the signed-digit kernels' rows in LDS.  Below 131,072 divisions one lane each
-  // gives fewer than two waves per SIMD (1,024 SIMDs x 2 x 64 lanes): two
-  // lanes per division instead
+  // What is left: divisors up to 256 bits, up to 512 in large batches and above
+  // 33,280, dividends too long for the signed-digit kernels' rows in LDS, and
+  // the short and long quotients that these kernels do faster
+  // (register_division_pays).  Below 131,072 divisions one lane each gives
+  // fewer than two waves per SIMD (1,024 SIMDs x 2 x 64 lanes): two lanes per
+  // division instead
   if (count < 131072 && nb > 16 && nb <= 128) {
     if (nb <= 32) return launch_divmod_pair<16>(q, r, a, b, count, stream);
     if (nb <= 64) return launch_divmod_pair<32>(q, r, a, b, count, stream);
@@ -915,12 +917,9 @@ hipError_t launch_pow2_mod(uint32_t *out, uint32_t out_len, uint32_t out_stride,
   if (count == 0) return hipSuccess;
   hipError_t st;
   if (launch_pow2_mod_lazy(out, out_len, out_stride, m, m_len, m_stride, count, e, stream, &st)) return st;
+  // (all of 17 to 1,040 limbs are taken above: a power's rows fit)
   if (m_len <= 8) return launch_pow2_reg<8>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
   if (m_len <= 16) return launch_pow2_reg<16>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
-  if (m_len <= 32) return launch_pow2_reg<32>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
-  if (m_len <= 64) return launch_pow2_reg<64>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
-  if (m_len <= 96) return launch_pow2_reg<96>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
-  if (m_len <= 128) return launch_pow2_reg<128>(out, out_len, out_stride, m, m_len, m_stride, count, e, stream);
   const uint32_t words = wave_div_words((e >> 5) + 1, m_len);
   if (words <= kWaveDivMaxWords) {
     hipLaunchKernelGGL(pow2_mod_wave_kernel, dim3(count), dim3(64), words * sizeof(uint32_t), stream, out, out_len,
