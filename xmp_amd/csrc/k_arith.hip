@@ -154,7 +154,8 @@ __global__ void __launch_bounds__(1024) addsub_split_kernel(uint32_t *__restrict
 // a time past a multiple of four instances).  Measured, that against this
 // kernel: 64 limbs x 113 24.6 and 3.5 us, x 4,096 9.5, 3.7, x 65,536 26, 7.7, x
 // 262,144 39, 28; 128 limbs x 262,144 75, 78; 256 limbs x 65,536 109, 33, x
-// 262,144 149, 157; 512 limbs x 65,536 215, 170, x 131,072 243, 336.
+// 262,144 149, 157; 512 limbs x 65,536 215, 170, x 131,072 243, 336.  (The line
+// at 196,608 is that of 128 and more limbs, for all.)
 template <bool SUB>
 bool launch_addsub_split(const OutOperand &s, const Operand &a, const Operand &b, uint32_t count, hipStream_t stream) {
   constexpr uint32_t kPass = 16 * kSplitWaves;

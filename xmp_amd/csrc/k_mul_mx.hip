@@ -354,7 +354,9 @@ bool mul_mx_holds(uint32_t a_len, uint32_t b_len, uint32_t count) {
 // (x 16,384 38, 34); 6144 x 32,768 106, 135; 8192 x 32,768 130, 189; 16384 x
 // 4,096 46, 126; 32768 x 4,096 113, 467; 65536 x 64 32, 834, x 1,024 104, 970.
 // A multiplier shorter than half leaves the lane kernels little to do: 8192 x
-// 1024 bits x 16,384 40, 29.
+// 1024 bits x 16,384 40, 29.  Above 16384 bits they split first, and this is
+// faster by any multiplier: 552 x 1 limbs x 8,220 40, 58; 614 x 7 x 14,013 57,
+// 98; 1816 x 1 x 9,238 154, 236; 3461 x 5 x 4,847 154, 363.
 bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t count) {
   if (!mul_mx_holds(a_len, b_len, count)) return false;
   if (a_len > 512) return true;

@@ -807,8 +807,8 @@ uint32_t powm_mx_blocks(uint32_t precision) {
 //   7.0; 2176 x 6,144 1.26, 1.70 (16,384: 3.2, 2.7); 2304 x 16,384 3.2, 3.4
 //   (32,768: 6.1, 5.9); 2368 x 65,536 12.1, 14.5; 3072 x 65,536 14.4, 15.4;
 //   32-bit exponents, where the set-up weighs more: 1312 x 12,288 0.245, 0.208;
-//   1536 x 14,336 0.281, 0.300; 2048 x 16,384 0.363, 0.383, x 24,576 0.52,
-//   0.64; 3072 x 65,536 2.42, 2.52; 4096 x 65,536 3.3, 4.2.
+//   1536 x 14,336 0.254, 0.269; 2048 x 16,384 0.331, 0.338, x 24,576 0.50,
+//   0.59; 3072 x 65,536 2.42, 2.52; 4096 x 65,536 3.3, 4.2.
 bool powm_mx_pays(uint32_t precision, uint32_t exp_bits, uint32_t count) {
   if (precision <= 128 || count >> 26) return false;   // (a wave an instance: a grid has fewer than 2^32 threads)
   if (precision <= 256) return count <= 1024;
