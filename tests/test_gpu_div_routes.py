@@ -85,3 +85,33 @@ def test_division_routes(handle, lb, more, n):
     _assert_periodic(Q.get(), wq, what + " div")
     for z in (A, B, Q, R):
         z.close()
+
+
+@pytest.mark.parametrize("lb,la,n", [
+    (9, 8, 300), (17, 16, 70), (24, 1, 4097), (32, 30, 40000), (35, 34, 33), (49, 47, 7826), (64, 32, 30000), (98, 97, 9000),
+    (129, 64, 700), (195, 194, 9), (256, 1, 600), (401, 399, 70), (520, 519, 2100), (831, 829, 65),
+])
+def test_dividends_of_fewer_limbs(handle, lb, la, n):
+    """Divisors that are all longer than the dividends, and batches with one that
+    is not at its start, within or at its end: a shorter one, 1 and 0."""
+    a, b = inputs.uniform(9300 + lb, n, la), inputs.uniform(9301 + lb, n, lb)
+    b[:, -1] |= np.uint32(1)
+    b[2 % n, la:], b[2 % n, la] = 0, 1                  # one bit more than the dividends have
+    A, Q, R = handle.from_array(a), handle.integers(32 * la, n), handle.integers(32 * lb, n)
+    for at in (None, 0, n // 2, n - 1):
+        for d in ([None] if at is None else [O.to_int(a[at]) >> 1, O.to_int(a[at]), 1, 0]):
+            c = b.copy()
+            if d is not None:
+                c[at] = O.from_int(d, lb)
+            B = handle.from_array(c)
+            handle.divmod(Q, R, A, B)
+            wq, wr = np.zeros_like(a), np.pad(a, ((0, 0), (0, lb - la)))
+            if d:
+                x = O.to_int(a[at])
+                wq[at], wr[at] = O.from_int(x // d, la), O.from_int(x % d, lb)
+            what = "%d / %d limbs x %d, %s at %s" % (la, lb, n, d if d is None or d < 2 else "a short one", at)
+            _assert_periodic(Q.get(), wq, what + " q")
+            _assert_periodic(R.get(), wr, what + " r")
+            B.close()
+    for x in (A, Q, R):
+        x.close()

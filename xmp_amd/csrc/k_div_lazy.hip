@@ -211,6 +211,22 @@ __device__ __forceinline__ void divide_lazy(const Dividend &A, const ArrayDivide
     if (k < L || __builtin_amdgcn_ballot_w64(bits == 0) == 0) break;
   }
   const bool zero = bits == 0;
+  // dividends of fewer limbs: q = 0 and r = a where the divisor is the longer
+  if (A.len < B.len && __builtin_amdgcn_ballot_w64(!zero && bits <= (int32_t)(32 * A.len)) == 0) {
+    if (active && o.q)
+      for (uint32_t k = (uint32_t)l; k < o.q_len; k += L) o.q[(size_t)k * o.q_stride] = 0u;
+    if (o.r)
+      for (uint32_t k0 = 8 * (uint32_t)l; k0 < o.r_len; k0 += 8 * L) {
+        uint32_t x[8];
+        A.template load<8>(x, (int32_t)k0);
+        if (active) {
+#pragma unroll
+          for (uint32_t k = 0; k < 8; k++)
+            if (k0 + k < o.r_len) o.r[(size_t)(k0 + k) * o.r_stride] = x[k];
+        }
+      }
+    return;
+  }
   const int32_t sh = D * ND - bits;
   int32_t v[K];
   {
