@@ -100,6 +100,7 @@ static xmpError_t cmp_internal(xmpHandle_t handle, int32_t *c, const xmpIntegers
   xmpExecutionPolicy_t p = handle->policy;
   if (launch_cmp(dst, make_in(a, p, 0), make_in(b, p, 1), count, handle->stream) != hipSuccess) return xmpErrorCuda;
   if (host && copy_out(handle, c, dst, sizeof(int32_t) * (size_t)count, async) != hipSuccess) return xmpErrorCuda;
+  if (!host && !async) (void)hipStreamSynchronize(handle->stream);   // (copy_out has waited)
   XMP_CHECK_HIP();
   return xmpErrorSuccess;
 }
@@ -109,7 +110,7 @@ xmpError_t XMPAPI xmpIntegersCmpAsync(xmpHandle_t handle, int32_t *c, const xmpI
 }
 xmpError_t XMPAPI xmpIntegersCmp(xmpHandle_t handle, int32_t *c, const xmpIntegers_t a, const xmpIntegers_t b,
                                  uint32_t count) {
-  return sync(handle, cmp_internal(handle, c, a, b, count, false));
+  return cmp_internal(handle, c, a, b, count, false);
 }
 
 // c = a << shift[i % shift_count] (truncated) or a >> -shift[...] (reference logic.cu:118-208).
@@ -211,6 +212,7 @@ static xmpError_t popc_internal(xmpHandle_t handle, uint32_t *c, const xmpIntege
   }
   if (launch_popc(dst, make_in(a, handle->policy, 0), count, handle->stream) != hipSuccess) return xmpErrorCuda;
   if (host && copy_out(handle, c, dst, sizeof(uint32_t) * (size_t)count, async) != hipSuccess) return xmpErrorCuda;
+  if (!host && !async) (void)hipStreamSynchronize(handle->stream);
   XMP_CHECK_HIP();
   return xmpErrorSuccess;
 }
@@ -218,7 +220,7 @@ xmpError_t XMPAPI xmpIntegersPopcAsync(xmpHandle_t handle, uint32_t *c, const xm
   return popc_internal(handle, c, a, count, true);
 }
 xmpError_t XMPAPI xmpIntegersPopc(xmpHandle_t handle, uint32_t *c, const xmpIntegers_t a, uint32_t count) {
-  return sync(handle, popc_internal(handle, c, a, count, false));
+  return popc_internal(handle, c, a, count, false);
 }
 
 }  // extern "C"
