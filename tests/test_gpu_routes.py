@@ -216,6 +216,21 @@ def test_formats_of_no_whole_words(recording, fmt, n, scratch_in, scratch_out):
     x.close()
 
 
+@pytest.mark.parametrize("limbs,n,uses", [(1, 65536, False), (2, 28672, False), (2, 28700, True), (8, 1792, False),
+                                          (8, 1800, True), (11, 950, True), (12, 850, False), (16, 700, True)])
+def test_imports_of_short_integers_of_no_whole_words(recording, limbs, n, uses):
+    """The slot keeps 448 KiB by the limbs, 40 from 12 limbs on, and more than
+    that is transposed in scratch."""
+    a = inputs.uniform(8750 + limbs, n, limbs)
+    host = np.ascontiguousarray(a.astype("<u4").view("<u2").astype(">u2"))   # 16-bit big-endian words, low one first
+    x = recording.integers(32 * limbs, n)
+    recording.sizes.clear()
+    assert xmp_amd.lib().xmpIntegersImport(recording.h, x.x, 2 * limbs, -1, 2, 1, 0, host.ctypes.data, n) == 0
+    assert recording.sizes == ([4 * n * limbs] if uses else [])
+    assert np.array_equal(x.get(), a)
+    x.close()
+
+
 @pytest.mark.parametrize("limbs,n,uses", [(9, 56, False), (9, 60, True), (33, 124, True), (33, 125, False), (7, 300, False),
                                           (36, 100, False), (65, 32, False), (65, 33, True)])
 def test_short_imports_of_odd_lengths(recording, limbs, n, uses):

@@ -77,10 +77,11 @@ bool is_device_pointer(const void *p) {
 // 155 and 590 (one core's memcpy).  A transposing kernel has its compact side in
 // a slot (one slot at most) where that is faster than in device scratch: whole
 // words, and other formats, which cross the bus a short word or a byte at a
-// time, up to 40 KiB in (any call's size up to 16 limbs) and 8 KiB out (24 as
-// 64-bit words).  16-bit words in mixed order, out: 1088 bits x 50 17.1 us, from
-// scratch 18.2; x 100 20.8, 18.5; 8192 x 100 68, 22; in: 1088 x 300 18.1, 23.1;
-// 256 x 3,000 18.8, 24.3; 8192 x 100 33, 24.  Chunks are half slots up to 1 MiB,
+// time, up to 40 KiB in (more below 12 limbs, whose neighbours share lines) and
+// 8 KiB out (24 as 64-bit words).  16-bit words in mixed order, out: 1088 bits x
+// 50 17.1 us, from scratch 18.2; x 100 20.8, 18.5; 8192 x 100 68, 22; in: 1088 x
+// 300 18.1, 23.1; 64 x 30,000 25, 28; 256 x 1,700 23.7, 23.7; x 6,400 46, 27; 512
+// x 700 22, 23; x 3,840 60, 28; 8192 x 100 33, 24.  Chunks are half slots up to 1 MiB,
 // so that there are enough of them to overlap.  From pageable memory its path is
 // as fast as a slot (4 MiB 155 against 170), but for the copy that a short
 // import does not need.
@@ -418,7 +419,7 @@ static xmpError_t import_internal(xmpHandle_t handle, xmpIntegers_t out, uint32_
     xmpError_t e = check_scratch_limit(handle, bytes);
     if (e != xmpErrorSuccess) return e;
     const bool whole = transfer_in_words(words, order, endian, nails, (uint32_t)size, out->nlimbs);
-    const size_t most = whole || out->nlimbs <= 16 ? HostStage::kDirect : HostStage::kOtherIn;
+    const size_t most = whole ? HostStage::kDirect : HostStage::other_in(out->nlimbs);
     // (more than eight limbs, no multiple of four, move through LDS tiles, and
     // more than half a tile's reads over the bus take longer than the runtime's
     // copy of up to 16 KiB: 33 limbs x 100 18.9 us, 17.4; x 200 19.3, 23.4; x 10

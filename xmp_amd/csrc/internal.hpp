@@ -59,7 +59,10 @@ struct HostStage {
   static constexpr size_t kSlot = 512u << 10;
   static constexpr int kSlots = 4;
   static constexpr size_t kDirect = 256u << 10;   // up to here a kernel reads or writes one slot itself,
-  static constexpr size_t kOtherIn = 40u << 10, kOtherOut = 8u << 10;   // ... of a format of no whole words
+  static constexpr size_t kOtherOut = 8u << 10;    // ... of a format of no whole words, and in
+  static size_t other_in(uint32_t limbs) {
+    return limbs < 2 ? kDirect : limbs < 12 ? (448u << 10) / limbs : 40u << 10;
+  }
   uint8_t *buf = nullptr;
   bool none = false;                               // no memory could be pinned: not asked for again
   hipEvent_t done[kSlots] = {};                    // the slot's last copy
