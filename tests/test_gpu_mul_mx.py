@@ -116,3 +116,24 @@ def test_beyond_the_matrix_cores(fresh_handle):
 def _get(h, x):
     h.set_scratch_limit(0)   # the export's staging is scratch too
     return x.get()
+
+
+@pytest.mark.parametrize("limbs", [17, 20, 25, 28, 32])
+@pytest.mark.parametrize("n", [1, 1000, 2049])
+def test_truncated_products_on_both_kernels(handle, limbs, n):
+    """Products and squares whose last limb asked for is at the lines between
+    the lane kernels and the matrix cores."""
+    a, b = inputs.uniform(5600 + limbs, n, limbs), inputs.uniform(5700 + limbs, n, limbs)
+    a[0], b[0] = 0xFFFFFFFF, 0xFFFFFFFF
+    A, B = handle.from_array(a), handle.from_array(b)
+    for lp in sorted({limbs, 25, 26, 36, 37, 2 * limbs, 2 * limbs + 3}):
+        if lp < limbs:
+            continue
+        P = handle.integers(32 * lp, n)
+        handle.mul(P, A, B)
+        assert_rows_equal(P.get(), gmp(O.GO_MUL, n, lp, a, b), "%d x %d -> %d limbs" % (limbs, limbs, lp))
+        handle.mul(P, A, A)
+        assert_rows_equal(P.get(), gmp(O.GO_MUL, n, lp, a, a), "%d limbs squared -> %d" % (limbs, lp))
+        P.close()
+    for x in (A, B):
+        x.close()

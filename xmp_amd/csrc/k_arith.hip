@@ -737,7 +737,7 @@ bool launch_rows(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t
 }  // namespace
 
 hipError_t launch_mul(OutOperand p, Operand a, Operand b, uint32_t count, hipStream_t stream) {
-  if (mul_mx_pays(a.len, b.len, count)) return launch_mul_mx(p, a, b, count, false, stream);
+  if (mul_mx_pays(a.len, b.len, p.len, false, count)) return launch_mul_mx(p, a, b, count, false, stream);
   // one lane per product with both operands in registers (product scanning)
   // for 513-1024-bit by 513-1024-bit and 1537-2048-bit by 513-2048-bit
   if (a.len > 16 && a.len <= 32 && b.len > 16) return launch_mul_cols<37, 37, false>(p, a, b, count, stream);
@@ -752,7 +752,7 @@ hipError_t launch_mul(OutOperand p, Operand a, Operand b, uint32_t count, hipStr
 }
 
 hipError_t launch_sqr(OutOperand p, Operand a, uint32_t count, hipStream_t stream) {
-  if (mul_mx_pays(a.len, a.len, count)) return launch_mul_mx(p, a, a, count, true, stream);
+  if (mul_mx_pays(a.len, a.len, p.len, true, count)) return launch_mul_mx(p, a, a, count, true, stream);
   // symmetric product scanning: each product of two different digits once
   if (a.len > 16 && a.len <= 32) return launch_mul_cols<37, 37, true>(p, a, a, count, stream);
   if (a.len > 48 && a.len <= 64) return launch_mul_cols<74, 74, true>(p, a, a, count, stream);

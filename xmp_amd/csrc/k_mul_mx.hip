@@ -357,11 +357,18 @@ bool mul_mx_holds(uint32_t a_len, uint32_t b_len, uint32_t count) {
 // 1024 bits x 16,384 40, 29.  Above 16384 bits they split first, and this is
 // faster by any multiplier: 552 x 1 limbs x 8,220 40, 58; 614 x 7 x 14,013 57,
 // 98; 1816 x 1 x 9,238 154, 236; 3461 x 5 x 4,847 154, 363.
-bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t count) {
+//   The lane kernels stop at the product's last limb that is asked for, which
+// this one gains little by: 640-bit products x 1,000 of 640 bits 5.2, 4.5, of 800
+// 5.2, 5.1, of 960 5.2, 5.7; 896-bit squares x 1,000 of 896 4.9, 4.0, of 1120 4.9,
+// 4.6, of 1344 5.0, 5.1; 544-bit squares whole 4.7, 4.5.
+bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t p_len, bool square, uint32_t count) {
   if (!mul_mx_holds(a_len, b_len, count)) return false;
   if (a_len > 512) return true;
   if (2 * b_len < a_len || a_len <= 16) return false;
-  if (a_len <= 32) return count <= 2048;
+  if (a_len <= 32) {
+    if (b_len > 16 && std::min(a_len + b_len, p_len) <= (square ? 36 : 25)) return false;
+    return count <= 2048;
+  }
   if (a_len <= 64) return count <= 4096;
   return a_len > 128 || count <= 8192;
 }

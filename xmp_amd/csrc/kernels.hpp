@@ -48,7 +48,7 @@ hipError_t launch_sqr(OutOperand p, Operand a, uint32_t count, hipStream_t strea
 // Products on the matrix cores (k_mul_mx.hip); for a_len >= b_len, whether it
 // holds them, and whether a batch takes it
 bool mul_mx_holds(uint32_t a_len, uint32_t b_len, uint32_t count);
-bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t count);
+bool mul_mx_pays(uint32_t a_len, uint32_t b_len, uint32_t p_len, bool square, uint32_t count);
 hipError_t launch_mul_mx(OutOperand p, Operand a, Operand b, uint32_t count, bool square, hipStream_t stream);
 // Products whose longer operand has kKaratsubaMinLimbs limbs or more and that
 // the matrix cores do not hold split by Karatsuba into products that they do;
