@@ -115,3 +115,64 @@ def test_dividends_of_fewer_limbs(handle, lb, la, n):
             B.close()
     for x in (A, Q, R):
         x.close()
+
+
+@pytest.mark.parametrize("lb,la,n", [
+    (17, 271, 24576), (24, 272, 33000), (20, 192, 33001), (24, 143, 50001), (17, 144, 66000), (25, 150, 66001),
+    (32, 256, 24576), (33, 288, 30000), (48, 320, 40000), (49, 168, 50001), (64, 192, 66001), (65, 384, 24576),
+    (96, 192, 50001), (96, 288, 66001), (97, 448, 24576), (128, 447, 24576),
+    (24, 72, 131072), (32, 47, 131072), (48, 72, 150000), (64, 96, 131072), (96, 143, 131072), (128, 192, 131072),
+])
+def test_gathered_long_dividends(handle, lb, la, n):
+    """Both sides of the rule for dividends that an index array gathers, and the
+    same sizes without one."""
+    a, b = _operands(9400 + lb + la, la, lb)
+    rows = np.arange(NA * NB)
+    x, y = a[rows % NA], b[rows // NA]
+    zero = ~y.any(axis=1)
+    wq, wr = gmp(O.GO_DIV, rows.size, la, x, np.where(zero[:, None], np.uint32(1), y), out2_limbs=lb)
+    wq[zero], wr[zero] = 0, x[zero][:, :lb]
+    rng = np.random.default_rng(la)
+    ia, ib = rng.integers(0, NA, n).astype(np.uint32), rng.integers(0, NB, n).astype(np.uint32)
+    A, B, Q, R = handle.from_array(a), handle.from_array(b), handle.integers(32 * la, n), handle.integers(32 * lb, n)
+    what = "%d / %d limbs x %d" % (la, lb, n)
+    handle.set_indices(2, ia)
+    handle.set_indices(3, ib)
+    try:
+        handle.divmod(Q, R, A, B, n)
+    finally:
+        handle.clear_indices()
+    pair = ia.astype(np.int64) + NA * ib
+    assert np.array_equal(Q.get(), wq[pair]), what + " gathered q"
+    assert np.array_equal(R.get(), wr[pair]), what + " gathered r"
+    handle.divmod(Q, R, A, B, n)
+    pair = np.arange(n) % NA + NA * (np.arange(n) % NB)
+    assert np.array_equal(Q.get(), wq[pair]), what + " q"
+    assert np.array_equal(R.get(), wr[pair]), what + " r"
+    for z in (A, B, Q, R):
+        z.close()
+
+
+@pytest.mark.parametrize("lb,la,n,stored", [
+    (24, 320, 50001, True), (17, 240, 66001, False), (28, 600, 24576, True), (32, 384, 131071, False), (40, 480, 66000, True),
+    (48, 576, 66001, True), (56, 448, 50001, False), (64, 384, 66001, True), (80, 768, 33001, True), (96, 576, 50001, False),
+])
+def test_long_dividends_of_middling_batches(handle, lb, la, n, stored):
+    """The first dividends that go to the lane pairs, and one limb less."""
+    for la in (la - 1, la):
+        a, b = _operands(9500 + lb + la, la, lb)
+        rows = np.arange(NA * NB)
+        x, y = a[rows % NA], b[rows % NB]
+        zero = ~y.any(axis=1)
+        wq, wr = gmp(O.GO_DIV, rows.size, la, x, np.where(zero[:, None], np.uint32(1), y), out2_limbs=lb)
+        wq[zero], wr[zero] = 0, x[zero][:, :lb]
+        A, B, Q, R = handle.from_array(a), handle.from_array(b), handle.integers(32 * la, n), handle.integers(32 * lb, n)
+        what = "%d / %d limbs x %d" % (la, lb, n)
+        if stored:
+            handle.divmod(Q, R, A, B, n)
+            _assert_periodic(Q.get(), wq, what + " q")
+        else:
+            handle.mod(R, A, B, n)
+        _assert_periodic(R.get(), wr, what + " r")
+        for z in (A, B, Q, R):
+            z.close()

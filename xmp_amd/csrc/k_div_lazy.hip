@@ -528,15 +528,53 @@ const ShortRule kShort[] = {
     {196, 256, 513, 1500, 1, 1},     {257, 384, 1, 600, 0, 1},       {896, 1016, 4096, 24576, 1, 1},
     {1017, 1040, 3000, 24576, 5, 4},
 };
+// Long dividends of batches that fill the lane pairs once or a few times: from
+// so many limbs of dividend on, without and with the quotient stored, and for
+// dividends that an index array gathers.  The 32-bit kernels read a limb of
+// every instance at a time, which the caches then hold for the rows'
+// neighbours; here a wave reads whole dividends, and a gather fetches most
+// lines once for each instance.  Measured, us: 576/24 limbs x 58,000 379 and
+// 307, 480/40 x 65,536 with the quotient 419 and 346; gathered in random order
+// 384/24 x 65,536 503 and 249, 144/24 153 and 119, 288/96 454 and 351, 96/48 x
+// 131,072 310 and 164.
+struct LongRule {
+  uint32_t from, to;           // divisor's limbs
+  uint32_t count_from, count_to;
+  uint32_t dividend, stored, gathered;
+};
+const LongRule kLong[] = {
+    {17, 24, 24576, 33000, kAny, 576, 272},    {17, 24, 33001, 50000, kAny, kAny, 192},
+    {17, 24, 50001, 66000, 240, 320, 144},     {17, 24, 66001, 131071, 240, 288, 144},
+    {25, 32, 24576, 33000, 768, 600, 256},     {25, 32, 33001, 50000, 672, 672, 192},
+    {25, 32, 50001, 66000, 448, 336, 150},     {25, 32, 66001, 131071, 384, 256, 150},
+    {33, 48, 24576, 33000, 1152, 960, 288},    {33, 48, 33001, 50000, 960, 960, 320},
+    {33, 48, 50001, 66000, 576, 480, 192},     {33, 48, 66001, 131071, kAny, 576, 240},
+    {49, 64, 24576, 33000, 1176, 896, 294},    {49, 64, 33001, 50000, 1176, 896, 336},
+    {49, 64, 50001, 66000, 448, 384, 168},     {49, 64, 66001, 131071, 448, 384, 192},
+    {65, 96, 24576, 33000, 1280, 1152, 384},   {65, 96, 33001, 50000, kAny, 768, 480},
+    {65, 96, 50001, 66000, 576, 576, 192},     {65, 96, 66001, 131071, kAny, kAny, 288},
+    {97, 128, 24576, 33000, kAny, kAny, 448},  {97, 128, 50001, 66000, kAny, kAny, 768},
+    // (above, one lane a division; those whose registers are just filled again)
+    {17, 31, 131072, kAny, kAny, kAny, 72},    {32, 32, 131072, kAny, kAny, kAny, 48},
+    {33, 47, 131072, 300000, kAny, kAny, 49},  {48, 48, 131072, kAny, kAny, kAny, 72},
+    {49, 63, 131072, 300000, kAny, kAny, 73},  {64, 64, 131072, kAny, kAny, kAny, 96},
+    {65, 79, 131072, 140000, kAny, kAny, 97},  {80, 95, 131072, 300000, kAny, kAny, 120},
+    {96, 96, 131072, kAny, kAny, kAny, 144},   {97, 127, 131072, 140000, kAny, kAny, 145},
+    {128, 128, 131072, kAny, kAny, kAny, 192},
+};
 // Long quotients of full batches: rows that leave a CU so few waves that the
 // 32-bit kernels, which keep nothing in LDS, are ahead.  Measured, us: 5120/1024
 // bits x 262,144 208 and 158 (with the quotient stored 313 and 182), 10752/1536
 // x 131,072 349 and 258, 3072/1024 x 262,144 with the quotient 122 and 95.
-bool register_division_pays(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient) {
+bool register_division_pays(uint32_t a_len, uint32_t b_len, uint32_t count, bool quotient, bool gathered) {
   const int32_t more = a_len > b_len ? (int32_t)(a_len - b_len) : 0;
   for (const ShortRule &r : kShort)
     if (b_len >= r.from && b_len <= r.to && count >= r.count_from && count <= r.count_to &&
         more <= (quotient ? r.stored : r.quotient))
+      return true;
+  for (const LongRule &r : kLong)
+    if (b_len >= r.from && b_len <= r.to && count >= r.count_from && count <= r.count_to &&
+        a_len >= std::min(quotient ? r.stored : r.dividend, gathered ? r.gathered : kAny))
       return true;
   if (count < 131072 || b_len <= 16 || b_len > 64) return false;
   const LazyRule *r = kRules;
@@ -555,7 +593,8 @@ bool divmod_lazy_takes(uint32_t a_len, uint32_t b_len, uint32_t count) {
 bool launch_divmod_lazy(OutOperand q, OutOperand r, Operand a, Operand b, uint32_t count, hipStream_t stream,
                         hipError_t *st) {
   const LazyEntry *e = lazy_entry(a.len, b.len, count, q.data != nullptr);
-  if (!e || register_division_pays(a.len, b.len, count, q.data != nullptr)) return false;
+  if (!e || register_division_pays(a.len, b.len, count, q.data != nullptr, a.idx != nullptr))
+    return false;
   const uint32_t per = 64 / e->lanes;
   hipLaunchKernelGGL(e->div, dim3(div_round_up(count, per)), dim3(64), 4 * per * lazy_row(a.len, e->lanes * e->digits, e->radix),
                      stream, q, r, a, b, count);
