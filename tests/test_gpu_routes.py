@@ -129,6 +129,34 @@ def test_a_loaded_table_decides_for_batches(recording, tables):
             x.close()
 
 
+def test_a_long_chain_beside_many_short_ones(recording):
+    """A class of which one tile takes longer than the queue's whole load goes to
+    the matrix cores however many instances the other classes have; with as
+    many long ones it does not."""
+    for shapes, matrix in ((((1536, 32, 8000), (1024, 1024, 200)), True), (((1024, 1024, 60000), (1024, 1024, 200)), False)):
+        arrays, wants = [], []
+        for bits, exp_bits, c in shapes:
+            m, b, e = inputs.powm_class(8350 + bits + c, c, bits, exp_bits=exp_bits)
+            if c > 200:
+                m, b, e = (np.tile(x[:100], (c // 100, 1)) for x in (m, b, e))
+            wants.append(gmp(O.GO_POWM, 100, bits // 32, b[:100], e[:100], m[:100]))
+            arrays.append([recording.integers(bits, c)] + [recording.from_array(x) for x in (b, e, m)])
+        recording.sizes.clear()
+        batch = ext.Batch(recording, *[[a[k] for a in arrays] for k in range(4)], [c for _, _, c in shapes])
+        assert any(_mx_bytes(1024, 200, w) in recording.sizes for w in range(2, 8)) == matrix
+        for _ in range(2):
+            batch.launch_async()
+            for a, want in zip(arrays, wants):
+                got = a[0].get()
+                assert_rows_equal(got[:100], want, "first instances")
+                if got.shape[0] > 200:
+                    assert_rows_equal(got[-100:], want, "last instances")
+        batch.close()
+        for a in arrays:
+            for x in a:
+                x.close()
+
+
 @pytest.mark.parametrize("bits,n", [(1024, 300), (3072, 50)])
 def test_digitmp_takes_the_default_plan(recording, bits, n):
     """The digit-serial policy is accepted and treated as the default one."""
