@@ -58,6 +58,7 @@ def _assert_periodic(got, want, what):
     (72, 3, 65536), (96, 5, 49152), (96, 6, 65536), (96, 4, 131072), (96, 12, 262144),
     (129, 4, 600), (129, 5, 16), (129, -40, 64), (130, 9, 600), (195, 10, 64), (160, 5, 2000), (160, 4, 4000),
     (196, 6, 512), (256, 7, 16), (256, 1, 1500), (384, 1, 600), (896, 1, 4096), (1040, 5, 3000), (1040, -9, 3000),
+    (750, 9, 8192), (760, 5, 8192), (900, 7, 9000), (961, 3, 24577), (1016, 4, 8192), (1040, 9, 12000), (1017, 6, 11999),
     # rows that take more lanes than the batch's rule gives
     (20, 120, 65536), (24, 150, 65536), (32, 128, 65536), (32, 200, 65536), (64, 390, 65536),
     # ... and that go to the register kernels

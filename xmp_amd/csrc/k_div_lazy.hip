@@ -511,7 +511,7 @@ const LazyEntry *lazy_entry(uint32_t a_len, uint32_t b_len, uint32_t count, bool
 // just opens another round of this one's waves.  Measured, signed digits and
 // 32-bit kernels, us: 512/512 bits x 1,000 6.0 and 4.5, 1024/1024 x 8,192 7.1
 // and 6.4, x 65,536 10.9 and 9.2, 3072/3072 x 65,536 22.1 and 18.9, 6144/6144 x
-// 16 12.5 and 5.2, x 1,000 13.3 and 8.3.
+// 16 12.5 and 5.2, x 1,000 13.3 and 8.3; 980/980 limbs x 30,000 1096 and 895.
 struct ShortRule {
   uint32_t from, to;           // divisor's limbs
   uint32_t count_from, count_to;
@@ -525,8 +525,9 @@ const ShortRule kShort[] = {
     {72, 87, 57344, 65536, 3, 3},    {88, 96, 49152, 65536, 3, 5},   {96, 96, 131072, 135168, 4, 4},
     {96, 96, 262144, kAny, 7, 12},   {129, 129, 1, 600, 3, 4},       {130, 195, 1, 600, 8, 9},
     {130, 195, 601, 2000, 4, 5},     {130, 195, 2001, 4000, 2, 4},   {196, 256, 1, 512, 4, 6},
-    {196, 256, 513, 1500, 1, 1},     {257, 384, 1, 600, 0, 1},       {896, 1016, 4096, 24576, 1, 1},
-    {1017, 1040, 3000, 24576, 5, 4},
+    {196, 256, 513, 1500, 1, 1},     {257, 384, 1, 600, 0, 1},       {750, 849, 8192, kAny, 4, 9},
+    {850, 960, 8192, kAny, 6, 9},    {896, 1016, 4096, 8191, 1, 1},   {961, 1016, 8192, kAny, 2, 3},
+    {1017, 1040, 3000, 11999, 5, 5}, {1017, 1040, 12000, kAny, 6, 9},
 };
 // Long dividends of batches that fill the lane pairs once or a few times: from
 // so many limbs of dividend on, without and with the quotient stored, and for
